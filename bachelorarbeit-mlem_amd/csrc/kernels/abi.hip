@@ -353,7 +353,7 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
     if (tiled_lds_bytes(t->plan, w->view.span, BC) + 4096 > (size_t)lds_max)
         return set_err(MLEM_ERR_UNSUPPORTED, "tiling (width %u, rows %u, %u right-hand sides) needs too much LDS", W,
                        R, BC);
-    HIPCHK(part->alloc(std::max<size_t>(4, tiled_part_bytes(t->plan, w->view.nwg, BC))));
+    if (part) HIPCHK(part->alloc(std::max<size_t>(4, tiled_part_bytes(t->plan, w->view.nwg, BC))));
     *tiled = t;
     *work = w;
     return MLEM_OK;
@@ -407,11 +407,12 @@ hipError_t enqueue_iteration(mlem_recon *r, IterEvents *ev) {
     fa.out = r->ratio.as<float>();
     fa.g = r->g.as<int32_t>();
     if (r->tfp) {
-        if ((e = launch_tiled_partials(r->tfp->plan, r->tfp->view, r->wfp->view, r->f.as<float>(),
+        if ((e = launch_tiled_partials(r->tfp->plan, r->tfp->view, r->wfp->view, one_pass(r->f.as<float>()),
                                        r->part_fp.as<float>(), 1, 0, s)) != hipSuccess)
             return e;
         if ((e = mark(1)) != hipSuccess) return e;
-        e = launch_tiled_reduce(r->tfp->plan, r->tfp->view, r->wfp->view, r->part_fp.as<float>(), 1, EPI_RATIO, fa, s);
+        e = launch_tiled_reduce(r->tfp->plan, r->tfp->view, r->wfp->view, r->part_fp.as<float>(), 1, EPI_RATIO,
+                                one_pass(fa), s);
     } else {
         if (r->opts.spmv == 0)
             e = launch_merge_spmv(r->pfp->plan, r->pfp->buf.p, r->scratch_fp.p, m->rowptr.as<uint64_t>(),
@@ -429,12 +430,12 @@ hipError_t enqueue_iteration(mlem_recon *r, IterEvents *ev) {
     ba.f = r->f.as<float>();
     if (r->opts.using_trans == 0) {
         if (r->tbp) {
-            if ((e = launch_tiled_partials(r->tbp->plan, r->tbp->view, r->wbp->view, r->ratio.as<float>(),
+            if ((e = launch_tiled_partials(r->tbp->plan, r->tbp->view, r->wbp->view, one_pass(r->ratio.as<float>()),
                                            r->part_bp.as<float>(), 1, 0, s)) != hipSuccess)
                 return e;
             if ((e = mark(3)) != hipSuccess) return e;
             e = launch_tiled_reduce(r->tbp->plan, r->tbp->view, r->wbp->view, r->part_bp.as<float>(), 1, EPI_UPDATE,
-                                    ba, s);
+                                    one_pass(ba), s);
         } else {
             if (r->bp_merge)
                 e = launch_merge_spmv(r->pbp->plan, r->pbp->buf.p, r->scratch_bp.p, m->rowptrT.as<uint64_t>(),
@@ -1311,10 +1312,10 @@ int mlem_recon_loglik(mlem_recon *r, double *ll) {
         HIPCHK(y.alloc(sizeof(float) * std::max<size_t>(1, m->rows)));
         EpiArgs ea{};
         ea.out = y.as<float>();
-        HIPCHK(launch_tiled_partials(r->tfp->plan, r->tfp->view, r->wfp->view, r->f.as<float>(), r->part_fp.as<float>(),
+        HIPCHK(launch_tiled_partials(r->tfp->plan, r->tfp->view, r->wfp->view, one_pass(r->f.as<float>()), r->part_fp.as<float>(),
                                      1, 0, r->stream));
-        HIPCHK(launch_tiled_reduce(r->tfp->plan, r->tfp->view, r->wfp->view, r->part_fp.as<float>(), 1, EPI_PLAIN, ea,
-                                   r->stream));
+        HIPCHK(launch_tiled_reduce(r->tfp->plan, r->tfp->view, r->wfp->view, r->part_fp.as<float>(), 1, EPI_PLAIN,
+                                   one_pass(ea), r->stream));
         HIPCHK(launch_loglik_y(y.as<float>(), r->g.as<int32_t>(), m->rows, r->llpart.as<double>(), r->stream));
         HIPCHK(hipStreamSynchronize(r->stream));
     } else {

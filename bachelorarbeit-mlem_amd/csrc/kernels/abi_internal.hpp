@@ -183,8 +183,10 @@ struct mlem_batch {
     size_t rows_x = 0, cols_x = 0;  // padded vector lengths
     hipStream_t stream = nullptr;
     std::vector<std::unique_ptr<BatchPass>> pass;  // [passes], null until a slot of the pass is set
-    // sensitivity, [slots] active flags, a rows/cols-long staging vector, partial sums of FP and BP
-    mlem::abi::DevBuf sens, active, stage, part_fp, part_bp;
+    // sensitivity, [slots] active flags, a rows/cols-long staging vector, the
+    // partial sums of FP or BP (never both at once) for `group` passes
+    mlem::abi::DevBuf sens, active, stage, part;
+    uint32_t group = 1;  // passes per launch
     const Tiled *tfp = nullptr, *tbp = nullptr;
     const TileWorkDev *wfp = nullptr, *wbp = nullptr;
     const uint32_t *row_order = nullptr;  // tiles in the matrix's row order: where each count of g goes
@@ -197,7 +199,7 @@ struct mlem_batch {
     // Device bytes of one pass, and of everything else the batch holds.
     uint64_t pass_bytes() const { return (uint64_t)BC * 4u * (2u * rows_x + cols_x); }
     uint64_t fixed_bytes() const {
-        return sens.bytes + active.bytes + stage.bytes + part_fp.bytes + part_bp.bytes;
+        return sens.bytes + active.bytes + stage.bytes + part.bytes;
     }
     uint64_t device_bytes() const {
         uint64_t b = fixed_bytes();
@@ -242,7 +244,8 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
               uint32_t *flags);
 // Work list of t for about `target` workgroups, built on first use.
 int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev **out);
-// Tiles, work list and partial-sum buffer of one side for BC right-hand sides.
+// Tiles, work list and partial-sum buffer (part null: none) of one side for
+// BC right-hand sides.
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
                 const Tiled **tiled, const TileWorkDev **work, DevBuf *part);
 // The blocked or the plain merge path for one side of a reconstruction.
@@ -271,6 +274,12 @@ int batch_deactivate_async(mlem_batch *b, uint32_t slot);
 // stream, the flags swapped.  A slot's arithmetic does not depend on its
 // place, so the images are bitwise those it would have had in `from`.
 int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to);
+// The partial-sum buffer for up to `passes` passes per launch (at most
+// kMaxPasses), fewer where the memory for them is not free; `limit` (0:
+// none) bounds its bytes, one pass always allowed.
+int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t limit);
+// What one pass of FP and one of BP would take in buffers of their own.
+uint64_t batch_part_pair_bytes(const mlem_batch *b);
 // Frees pass p when none of its slots is active (returns the bytes freed).
 uint64_t batch_release_pass(mlem_batch *b, uint32_t p);
 // Progress of long builds on stderr when MLEM_VERBOSE is set.

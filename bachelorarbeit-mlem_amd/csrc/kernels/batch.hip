@@ -7,29 +7,33 @@ using namespace mlem::abi;
 
 namespace {
 
-// One iteration of the passes marked in `passes` on the batch's stream.
+// One iteration of the passes marked in `passes` on the batch's stream, up to
+// b->group passes per launch.
 int enqueue_batch_iteration(mlem_batch *b, const std::vector<uint8_t> &passes) {
     hipStream_t s = b->stream;
     const uint32_t BC = b->BC;
-    for (uint32_t p = 0; p < b->passes; ++p) {
-        if (!passes[p] || !b->pass[p]) continue;
-        float *f = b->pass[p]->f.as<float>();
-        float *ratio = b->pass[p]->ratio.as<float>();
-        EpiArgs fa{};
-        fa.out = ratio;
-        fa.g = b->pass[p]->g.as<int32_t>();
-        HIPCHK(launch_tiled_partials(b->tfp->plan, b->tfp->view, b->wfp->view, f, b->part_fp.as<float>(), BC, b->nt,
-                                     s));
-        HIPCHK(launch_tiled_reduce(b->tfp->plan, b->tfp->view, b->wfp->view, b->part_fp.as<float>(), BC, EPI_RATIO, fa,
-                                   s));
-        EpiArgs ba{};
-        ba.norm = b->sens.as<float>();
-        ba.f = f;
-        ba.active = b->active.as<uint32_t>() + (size_t)p * BC;
-        HIPCHK(launch_tiled_partials(b->tbp->plan, b->tbp->view, b->wbp->view, ratio, b->part_bp.as<float>(), BC,
-                                     b->nt, s));
-        HIPCHK(launch_tiled_reduce(b->tbp->plan, b->tbp->view, b->wbp->view, b->part_bp.as<float>(), BC, EPI_UPDATE,
-                                   ba, s));
+    for (uint32_t p = 0; p < b->passes;) {
+        PassX fx{}, bx{};
+        PassEpi fe{}, be{};
+        for (; p < b->passes && fx.n < b->group; ++p) {
+            if (!passes[p] || !b->pass[p]) continue;
+            float *f = b->pass[p]->f.as<float>(), *ratio = b->pass[p]->ratio.as<float>();
+            const uint32_t k = fx.n++;
+            fx.x[k] = f;
+            fe.ea[k].out = ratio;
+            fe.ea[k].g = b->pass[p]->g.as<int32_t>();
+            bx.x[k] = ratio;
+            be.ea[k].norm = b->sens.as<float>();
+            be.ea[k].f = f;
+            be.ea[k].active = b->active.as<uint32_t>() + (size_t)p * BC;
+        }
+        fe.n = bx.n = be.n = fx.n;
+        if (!fx.n) break;
+        float *part = b->part.as<float>();
+        HIPCHK(launch_tiled_partials(b->tfp->plan, b->tfp->view, b->wfp->view, fx, part, BC, b->nt, s));
+        HIPCHK(launch_tiled_reduce(b->tfp->plan, b->tfp->view, b->wfp->view, part, BC, EPI_RATIO, fe, s));
+        HIPCHK(launch_tiled_partials(b->tbp->plan, b->tbp->view, b->wbp->view, bx, part, BC, b->nt, s));
+        HIPCHK(launch_tiled_reduce(b->tbp->plan, b->tbp->view, b->wbp->view, part, BC, EPI_UPDATE, be, s));
     }
     return MLEM_OK;
 }
@@ -114,12 +118,37 @@ int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to) {
     return MLEM_OK;
 }
 
+uint64_t batch_part_pair_bytes(const mlem_batch *b) {
+    return tiled_part_bytes(b->tfp->plan, b->wfp->view.nwg, b->BC) +
+           tiled_part_bytes(b->tbp->plan, b->wbp->view.nwg, b->BC);
+}
+
+int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t limit) {
+    const uint64_t one = std::max<uint64_t>(4, std::max(tiled_part_bytes(b->tfp->plan, b->wfp->view.nwg, b->BC),
+                                                        tiled_part_bytes(b->tbp->plan, b->wbp->view.nwg, b->BC)));
+    // One right-hand side per pass: the blocked kernel takes one pass per launch.
+    uint32_t n = b->BC == 1 ? 1u : std::max(1u, std::min(passes, kMaxPasses));
+    while (n > 1 && limit && n * one > limit) --n;
+    for (;; n = (n + 1) / 2) {
+        const hipError_t e = b->part.alloc(n * one);
+        b->group = n;
+        if (e == hipSuccess) return MLEM_OK;
+        b->part.bytes = 0;
+        if (n == 1 || e != hipErrorOutOfMemory) HIPCHK(e);
+        (void)hipGetLastError();
+    }
+}
+
 uint64_t batch_release_pass(mlem_batch *b, uint32_t p) {
     if (!b || p >= b->passes || !b->pass[p]) return 0;
     for (uint32_t q = 0; q < b->BC; ++q)
         if (b->active_host[(size_t)p * b->BC + q]) return 0;
     if (hipSetDevice(b->m->device) != hipSuccess || hipStreamSynchronize(b->stream) != hipSuccess) return 0;
     const uint64_t bytes = b->pass[p]->g.bytes + b->pass[p]->ratio.bytes + b->pass[p]->f.bytes;
+    if (b->gexec) {  // a captured iteration may hold the pass's addresses
+        (void)hipGraphExecDestroy(b->gexec);
+        b->gexec = nullptr;
+    }
     b->pass[p].reset();
     return bytes;
 }
@@ -197,8 +226,9 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
         ea.out = y;
         for (int rep = 0; rep < 4; ++rep) {
             if (rep == 1 && hipEventRecord(e0, s) != hipSuccess) return hipErrorUnknown;
-            hipError_t e = launch_tiled_partials(t->plan, t->view, w->view, x, part.as<float>(), BC, nt, s);
-            if (e == hipSuccess) e = launch_tiled_reduce(t->plan, t->view, w->view, part.as<float>(), BC, EPI_PLAIN, ea, s);
+            hipError_t e = launch_tiled_partials(t->plan, t->view, w->view, one_pass(x), part.as<float>(), BC, nt, s);
+            if (e == hipSuccess)
+                e = launch_tiled_reduce(t->plan, t->view, w->view, part.as<float>(), BC, EPI_PLAIN, one_pass(ea), s);
             if (e != hipSuccess) return e;
         }
         hipError_t e = hipEventRecord(e1, s);
@@ -317,8 +347,9 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     int cus = 256, dev = 0;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     const uint32_t groups = o.tile_groups ? o.tile_groups : (BC == 1 ? 24u : 8u) * (uint32_t)std::max(1, cus);
-    if (int st = setup_tiled(m, 0, W, R, o.values, BC, groups, &b->tfp, &b->wfp, &b->part_fp)) return st;
-    if (int st = setup_tiled(m, 1, W, R, o.values, BC, groups, &b->tbp, &b->wbp, &b->part_bp)) return st;
+    if (int st = setup_tiled(m, 0, W, R, o.values, BC, groups, &b->tfp, &b->wfp, nullptr)) return st;
+    if (int st = setup_tiled(m, 1, W, R, o.values, BC, groups, &b->tbp, &b->wbp, nullptr)) return st;
+    if (int st = batch_alloc_part(b.get(), b->passes, 0)) return st;
     if (b->tfp->ordered != b->tbp->ordered)  // a row order set from another thread between the two builds
         return set_err(MLEM_ERR_INVALID_ARGUMENT, "mlem_batch_create: the row order changed while the tiles were built");
     if (b->tfp->ordered) b->row_order = m->row_order.as<uint32_t>();

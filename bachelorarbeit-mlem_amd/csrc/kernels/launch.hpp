@@ -209,18 +209,40 @@ const uint32_t *tile_count_sizes(const TilePlan &p, void *scratch);
 // tile_off.
 TileWorkList tile_work_list(const TilePlan &p, const uint32_t *tile_nz, const uint64_t *tile_off,
                             uint32_t target_wgs);
-// Y = A X for BC right-hand sides in two launches: the partial row sums of
-// every run into part (tiled_part_bytes(p, wk.nwg, BC)), then their
-// reduction with the row scales and the epilogue.  Vectors are [n][BC]
-// (right-hand side fastest); X must be readable (and finite) up to
+// Y = A X for n passes of BC right-hand sides each (n = 1 for BC = 1) in two
+// launches: the partial row sums of every run into part
+// (n * tiled_part_bytes(p, wk.nwg, BC), pass after pass), then their
+// reduction with the row scales and the epilogue.  Vectors are [rows][BC]
+// per pass (right-hand side fastest); X must be readable (and finite) up to
 // nseg * W rows: callers pad their vectors to whole segments (kTileXPad).
 // nt: work-items per workgroup of the kernel for several right-hand sides
 // (128, 256 or 512; 0 = 512), each taking 512 / nt groups of a window.
-hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *x,
+constexpr uint32_t kMaxPasses = 8;  // passes of a batch per launch
+struct PassX {
+    const float *x[kMaxPasses];
+    uint32_t n;
+};
+struct PassEpi {
+    EpiArgs ea[kMaxPasses];
+    uint32_t n;
+};
+inline PassX one_pass(const float *x) {
+    PassX v{};
+    v.x[0] = x;
+    v.n = 1;
+    return v;
+}
+inline PassEpi one_pass(const EpiArgs &ea) {
+    PassEpi v{};
+    v.ea[0] = ea;
+    v.n = 1;
+    return v;
+}
+hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x,
                                  float *part, uint32_t BC, uint32_t nt, hipStream_t s);
 bool valid_stream_threads(uint32_t nt);
 hipError_t launch_tiled_reduce(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *part,
-                               uint32_t BC, Epi epi, const EpiArgs &ea, hipStream_t s);
+                               uint32_t BC, Epi epi, const PassEpi &ea, hipStream_t s);
 
 // Sets the message of mlem_last_error() (this thread).
 void set_last_error(const char *msg);

@@ -114,6 +114,14 @@ int mlem_server_add_matrix(mlem_server *s, mlem_matrix *m, uint32_t max_slots, u
     mlem_batch *b = nullptr;
     if (int st = mlem_batch_create(m, max_slots, &s->bopts, &b))
         return fail(st, "mlem_server_add_matrix: %s", std::string(mlem_last_error()).c_str());
+    // Under a budget the partial sums take no more than FP's and BP's of one
+    // pass: what several passes per launch would add goes to requests.
+    if (s->budget)
+        if (int st = mlem::abi::batch_alloc_part(b, b->passes, mlem::abi::batch_part_pair_bytes(b))) {
+            const std::string msg = mlem_last_error();
+            mlem_batch_destroy(b);
+            return fail(st, "mlem_server_add_matrix: %s", msg.c_str());
+        }
     const uint64_t bbytes = b->fixed_bytes(), pbytes = b->pass_bytes();
     mlem_matrix_info(m, nullptr, nullptr, nullptr, nullptr, &mbytes);  // with the tiles the batch built
     if (s->budget && s->used + mbytes + bbytes + pbytes > s->budget) {

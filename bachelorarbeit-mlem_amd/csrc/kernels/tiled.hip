@@ -494,16 +494,22 @@ __global__ __launch_bounds__(kWG, (min_waves<W, VT, BC>())) void blocked_spmv_ke
 // boundary.
 // wl[w] = {row block, first window, windows}; win[i] = {first group,
 // groups | split << 16 | slot of A << 31, segment of A, segment of B}.
-
-
+//
+// One launch takes several passes of a batch (px.n of BC right-hand sides
+// each): workgroup i is pass i % n of run order[i / n], with its own x and
+// its own partial sums, so the passes' arithmetic is what n launches do.
+// A small matrix cannot fill the chip with one pass (the 2D ring's windows
+// make 540 workgroups, each a chain of memory latencies): its four launches
+// of 8.4 us are one of 22.0; with 6.9e8 nonzeros four passes take 2.70 ms
+// instead of 2.76.
 template <int W, int VT, int BC, int NT>
 __global__ __launch_bounds__(NT) void stream_spmv_kernel(uint32_t R, uint32_t nseg,
                                                          const uint64_t *__restrict__ tile_off,
                                                          const uint4 *__restrict__ wl,
                                                          const uint32_t *__restrict__ order,
                                                          const uint4 *__restrict__ win,
-                                                         const uint8_t *__restrict__ tdata,
-                                                         const float *__restrict__ x, float *__restrict__ part) {
+                                                         const uint8_t *__restrict__ tdata, PassX px, uint32_t nwg,
+                                                         float *__restrict__ part) {
     constexpr int GPW = kSNT / NT;             // groups per work-item and window
     constexpr int NQ = 2 * GPW;                // quads per work-item
     constexpr int VB = VT == VAL_F32 ? 4 : 2;  // bytes per stored value
@@ -523,7 +529,9 @@ __global__ __launch_bounds__(NT) void stream_spmv_kernel(uint32_t R, uint32_t ns
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
     const uint32_t g0 = tid * GPW;  // the work-item's first group in a window
-    const uint32_t run = order[blockIdx.x];  // workgroups start in column order, runs keep their place
+    const uint32_t place = blockIdx.x / px.n, pass = blockIdx.x - place * px.n;
+    const uint32_t run = order[place];  // workgroups start in column order, runs keep their place
+    const float *__restrict__ x = px.x[pass];
     const uint4 w = wl[run];
     const uint64_t e0 = tile_off[(uint64_t)w.x * nseg], e1 = tile_off[(uint64_t)(w.x + 1) * nseg];
     const uint64_t G = (e1 - e0) / 8;  // groups of the row block
@@ -747,7 +755,7 @@ __global__ __launch_bounds__(NT) void stream_spmv_kernel(uint32_t R, uint32_t ns
         }
     }
     __syncthreads();
-    float *pw = part + (uint64_t)run * R * BC;
+    float *pw = part + ((uint64_t)pass * nwg + run) * R * BC;
     for (uint32_t i = tid; i < R * BC; i += NT) pw[i] = acc[i];
 }
 
@@ -837,12 +845,16 @@ __device__ __forceinline__ void sum_partials(float (&y)[BC], const float *__rest
 
 // Row r of block b = r / R sums the partials of the block's workgroups
 // wl_first[b] .. wl_first[b+1]-1 in order (for each of the BC right-hand
-// sides) and applies the epilogue.
+// sides) and applies the epilogue.  Pass blockIdx.y has its partials from
+// pass_part floats per pass on.
 template <int EPI, int BC>
-__global__ void blocked_reduce_kernel(const float *__restrict__ part, const uint32_t *__restrict__ wl_first,
-                                      uint32_t rshift, uint32_t rows, const float *__restrict__ scale, EpiArgs ea) {
+__global__ void blocked_reduce_kernel(const float *__restrict__ part, uint64_t pass_part,
+                                      const uint32_t *__restrict__ wl_first, uint32_t rshift, uint32_t rows,
+                                      const float *__restrict__ scale, PassEpi pe) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
+    const EpiArgs ea = pe.ea[blockIdx.y];
+    part += blockIdx.y * pass_part;
     const uint32_t b = r >> rshift, i = r & ((1u << rshift) - 1u);
     const ReduceIn<BC> in = reduce_load<EPI, BC>(r, scale, ea);
     float y[BC];
@@ -860,8 +872,10 @@ constexpr uint32_t kSlices = 8;
 constexpr uint32_t kSlicedRuns = 64;  // runs of a row block from which the sliced sum is used
 template <int EPI, int BC>
 __global__ __launch_bounds__(64 * kSlices) void blocked_reduce_sliced_kernel(
-    const float *__restrict__ part, const uint32_t *__restrict__ wl_first, uint32_t rshift, uint32_t rows,
-    const float *__restrict__ scale, EpiArgs ea) {
+    const float *__restrict__ part, uint64_t pass_part, const uint32_t *__restrict__ wl_first, uint32_t rshift,
+    uint32_t rows, const float *__restrict__ scale, PassEpi pe) {
+    const EpiArgs ea = pe.ea[blockIdx.y];
+    part += blockIdx.y * pass_part;
     __shared__ float s_y[kSlices][64][BC];
     const uint32_t x = threadIdx.x, j = threadIdx.y;
     const uint32_t r = blockIdx.x * 64 + x;
@@ -1273,16 +1287,17 @@ hipError_t launch_k(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk
 }
 
 template <int W, int VT, int BC, int NT>
-hipError_t launch_stream_nt(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *x, float *part,
+hipError_t launch_stream_nt(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
                             hipStream_t s) {
     if (!wk.order) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((stream_spmv_kernel<W, VT, BC, NT>), dim3(wk.nwg), dim3(NT), stream_lds_bytes(W, p.R, BC), s,
-                       p.R, p.nseg, tm.tile_off, wk.wl, wk.order, wk.tiles, tm.tdata, x, part);
+    hipLaunchKernelGGL((stream_spmv_kernel<W, VT, BC, NT>), dim3(wk.nwg * x.n), dim3(NT),
+                       stream_lds_bytes(W, p.R, BC), s, p.R, p.nseg, tm.tile_off, wk.wl, wk.order, wk.tiles, tm.tdata,
+                       x, wk.nwg, part);
     return hipGetLastError();
 }
 
 template <int W, int VT, int BC>
-hipError_t launch_stream(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *x, float *part,
+hipError_t launch_stream(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
                          uint32_t nt, hipStream_t s) {
     switch (nt) {
         case 128: return launch_stream_nt<W, VT, BC, 128>(p, tm, wk, x, part, s);
@@ -1294,11 +1309,12 @@ hipError_t launch_stream(const TilePlan &p, const TiledMatrix &tm, const TileWor
 }
 
 template <int VT>
-hipError_t launch_vt(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *x, float *part,
+hipError_t launch_vt(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
                      uint32_t BC, uint32_t nt, hipStream_t s) {
     if (p.quad != (BC > 1)) return hipErrorInvalidValue;  // quads (block streams) exactly for several
-    if (BC == 1 && p.W == 1024) return launch_k<1024, VT, 1>(p, tm, wk, x, part, s);
-    if (BC == 1 && p.W == 2048) return launch_k<2048, VT, 1>(p, tm, wk, x, part, s);
+    if (BC == 1 && x.n != 1) return hipErrorInvalidValue;
+    if (BC == 1 && p.W == 1024) return launch_k<1024, VT, 1>(p, tm, wk, x.x[0], part, s);
+    if (BC == 1 && p.W == 2048) return launch_k<2048, VT, 1>(p, tm, wk, x.x[0], part, s);
     if (BC == 4 && p.W == 512) return launch_stream<512, VT, 4>(p, tm, wk, x, part, nt, s);
     if (BC == 4 && p.W == 1024) return launch_stream<1024, VT, 4>(p, tm, wk, x, part, nt, s);
     if (BC == 8 && p.W == 512) return launch_stream<512, VT, 8>(p, tm, wk, x, part, nt, s);
@@ -1648,8 +1664,9 @@ hipError_t launch_tile_fill_into(const TilePlan &p, const uint64_t *rowptr, cons
     return hipStreamSynchronize(s);
 }
 
-hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *x,
+hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x,
                                  float *part, uint32_t BC, uint32_t nt, hipStream_t s) {
+    if (x.n == 0 || x.n > kMaxPasses) return hipErrorInvalidValue;
     if (p.rows == 0 || wk.nwg == 0) return hipSuccess;
     switch (p.vt) {
         case VAL_F32: return launch_vt<VAL_F32>(p, tm, wk, x, part, BC, nt, s);
@@ -1664,36 +1681,38 @@ bool valid_stream_threads(uint32_t nt) { return nt == 0 || nt == 128 || nt == 25
 namespace {
 template <int EPI, int BC>
 void launch_reduce_epi(const TilePlan &p, const TileWork &wk, const float *part, const float *scale, uint32_t rshift,
-                       const EpiArgs &ea, hipStream_t s) {
+                       const PassEpi &pe, hipStream_t s) {
+    const uint64_t pass_part = (uint64_t)wk.nwg * p.R * BC;
     if (wk.max_runs >= kSlicedRuns)
-        hipLaunchKernelGGL((blocked_reduce_sliced_kernel<EPI, BC>), dim3(blocks_for(p.rows, 64)), dim3(64, kSlices), 0,
-                           s, part, wk.wl_first, rshift, p.rows, scale, ea);
+        hipLaunchKernelGGL((blocked_reduce_sliced_kernel<EPI, BC>), dim3(blocks_for(p.rows, 64), pe.n),
+                           dim3(64, kSlices), 0, s, part, pass_part, wk.wl_first, rshift, p.rows, scale, pe);
     else
-        hipLaunchKernelGGL((blocked_reduce_kernel<EPI, BC>), dim3(blocks_for(p.rows, kWG)), dim3(kWG), 0, s, part,
-                           wk.wl_first, rshift, p.rows, scale, ea);
+        hipLaunchKernelGGL((blocked_reduce_kernel<EPI, BC>), dim3(blocks_for(p.rows, kWG), pe.n), dim3(kWG), 0, s,
+                           part, pass_part, wk.wl_first, rshift, p.rows, scale, pe);
 }
 
 template <int BC>
 hipError_t launch_reduce_bc(const TilePlan &p, const TileWork &wk, const float *part, const float *scale, Epi epi,
-                            const EpiArgs &ea, hipStream_t s) {
+                            const PassEpi &pe, hipStream_t s) {
     uint32_t rshift = 0;
     while ((1u << rshift) < p.R) ++rshift;
     switch (epi) {
-        case EPI_PLAIN: launch_reduce_epi<EPI_PLAIN, BC>(p, wk, part, scale, rshift, ea, s); break;
-        case EPI_RATIO: launch_reduce_epi<EPI_RATIO, BC>(p, wk, part, scale, rshift, ea, s); break;
-        default: launch_reduce_epi<EPI_UPDATE, BC>(p, wk, part, scale, rshift, ea, s); break;
+        case EPI_PLAIN: launch_reduce_epi<EPI_PLAIN, BC>(p, wk, part, scale, rshift, pe, s); break;
+        case EPI_RATIO: launch_reduce_epi<EPI_RATIO, BC>(p, wk, part, scale, rshift, pe, s); break;
+        default: launch_reduce_epi<EPI_UPDATE, BC>(p, wk, part, scale, rshift, pe, s); break;
     }
     return hipGetLastError();
 }
 }  // namespace
 
 hipError_t launch_tiled_reduce(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *part,
-                               uint32_t BC, Epi epi, const EpiArgs &ea, hipStream_t s) {
+                               uint32_t BC, Epi epi, const PassEpi &pe, hipStream_t s) {
+    if (pe.n == 0 || pe.n > kMaxPasses) return hipErrorInvalidValue;
     if (p.rows == 0) return hipSuccess;
     switch (BC) {
-        case 1: return launch_reduce_bc<1>(p, wk, part, tm.scale, epi, ea, s);
-        case 4: return launch_reduce_bc<4>(p, wk, part, tm.scale, epi, ea, s);
-        case 8: return launch_reduce_bc<8>(p, wk, part, tm.scale, epi, ea, s);
+        case 1: return launch_reduce_bc<1>(p, wk, part, tm.scale, epi, pe, s);
+        case 4: return launch_reduce_bc<4>(p, wk, part, tm.scale, epi, pe, s);
+        case 8: return launch_reduce_bc<8>(p, wk, part, tm.scale, epi, pe, s);
         default: return hipErrorInvalidValue;
     }
 }

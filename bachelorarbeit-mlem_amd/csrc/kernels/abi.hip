@@ -419,7 +419,7 @@ hipError_t enqueue_iteration(mlem_recon *r, IterEvents *ev) {
                                   m->col.as<uint32_t>(), m->val.as<float>(), r->f.as<float>(), EPI_RATIO, fa, s);
         else
             e = launch_csr_vector(r->lanes_fp, m->rowptr.as<uint64_t>(), m->col.as<uint32_t>(), m->val.as<float>(),
-                                  r->f.as<float>(), m->rows, EPI_RATIO, fa, s);
+                                  r->f.as<float>(), m->rows, m->nnz, EPI_RATIO, fa, s);
         if (e == hipSuccess) e = mark(1);
     }
     if (e != hipSuccess) return e;
@@ -443,12 +443,12 @@ hipError_t enqueue_iteration(mlem_recon *r, IterEvents *ev) {
                                       ba, s);
             else
                 e = launch_csr_vector(r->lanes_bp, m->rowptrT.as<uint64_t>(), m->colT.as<uint32_t>(),
-                                      m->valT.as<float>(), r->ratio.as<float>(), m->cols, EPI_UPDATE, ba, s);
+                                      m->valT.as<float>(), r->ratio.as<float>(), m->cols, m->nnz, EPI_UPDATE, ba, s);
             if (e == hipSuccess) e = mark(3);
         }
     } else {
         e = launch_scatter(r->lanes_fp, m->rowptr.as<uint64_t>(), m->col.as<uint32_t>(), m->val.as<float>(),
-                           r->ratio.as<float>(), r->bp.as<float>(), m->rows, s);
+                           r->ratio.as<float>(), r->bp.as<float>(), m->rows, m->cols, m->nnz, s);
         if (e == hipSuccess) e = mark(3);
         if (e == hipSuccess)
             e = launch_update_image(r->f.as<float>(), r->sens.as<float>(), r->bp.as<float>(), m->cols, s);
@@ -737,9 +737,8 @@ static int vector_call(const char *what, const uint64_t *rowptr, const uint32_t 
     if (rows == 0) return MLEM_OK;
     ARGCHK(rowptr && x && (nnz == 0 || (col && val)), "%s: null pointer", what);
     ARGCHK(aligned16(col) && aligned16(val), "%s: col and val must be 16-byte aligned", what);
-    if (lanes == 0) lanes = auto_lanes(rows, nnz);
-    ARGCHK(valid_lanes(lanes), "%s: lanes must be 4, 8, 16, 32 or 64 (got %u)", what, lanes);
-    HIPCHK(launch_csr_vector(lanes, rowptr, col, val, x, rows, epi, ea, S(stream)));
+    ARGCHK(lanes == 0 || valid_lanes(lanes), "%s: lanes must be 4, 8, 16, 32 or 64 (got %u)", what, lanes);
+    HIPCHK(launch_csr_vector(lanes, rowptr, col, val, x, rows, nnz, epi, ea, S(stream)));
     return MLEM_OK;
 }
 
@@ -786,9 +785,8 @@ int mlem_bp_scatter(const uint64_t *rowptr, const uint32_t *col, const float *va
     HIPCHK(launch_fill(bwproj, 0.0f, cols, S(stream)));
     if (rows == 0) return MLEM_OK;
     ARGCHK(rowptr && correl && (nnz == 0 || (col && val)), "mlem_bp_scatter: null pointer");
-    if (lanes == 0) lanes = auto_lanes(rows, nnz);
-    ARGCHK(valid_lanes(lanes), "mlem_bp_scatter: lanes must be 4, 8, 16, 32 or 64 (got %u)", lanes);
-    HIPCHK(launch_scatter(lanes, rowptr, col, val, correl, bwproj, rows, S(stream)));
+    ARGCHK(lanes == 0 || valid_lanes(lanes), "mlem_bp_scatter: lanes must be 4, 8, 16, 32 or 64 (got %u)", lanes);
+    HIPCHK(launch_scatter(lanes, rowptr, col, val, correl, bwproj, rows, cols, nnz, S(stream)));
     return MLEM_OK;
 }
 
@@ -1161,8 +1159,8 @@ int mlem_recon_create(const mlem_matrix *mc, const int32_t *g, const float *sens
     r->opts = o;
     r->opts.secsize_fp = clamp_secsize(o.secsize_fp);
     r->opts.secsize_bp = clamp_secsize(o.secsize_bp);
-    r->lanes_fp = o.fp_lanes ? o.fp_lanes : auto_lanes(m->rows, m->nnz);
-    r->lanes_bp = o.bp_lanes ? o.bp_lanes : auto_lanes(m->cols, m->nnz);
+    r->lanes_fp = o.fp_lanes;
+    r->lanes_bp = o.bp_lanes;
     r->bp_merge = o.bp_spmv == 0 ? o.spmv == 0 : o.bp_spmv == 1;
     HIPCHK(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
     struct StreamGuard {

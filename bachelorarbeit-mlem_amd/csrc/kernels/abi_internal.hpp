@@ -223,7 +223,7 @@ struct mlem_recon {
     const Tiled *tfp = nullptr, *tbp = nullptr;        // blocked LDS-tiled path, when used
     const TileWorkDev *wfp = nullptr, *wbp = nullptr;  // and its work lists
     mlem::abi::DevBuf part_fp, part_bp;
-    uint32_t lanes_fp = 64, lanes_bp = 64;
+    uint32_t lanes_fp = 0, lanes_bp = 0;  // 0: chosen at the launch
     bool bp_merge = true;  // BP on A^T: merge-based or CSR-vector
     std::vector<IterEvents> events;  // pool, one set per profiled iteration
     size_t events_used = 0;

@@ -50,12 +50,13 @@ hipError_t launch_merge_spmv(const MergePlan &p, const void *partition, void *sc
                              const uint32_t *col, const float *val, const float *x, Epi epi, const EpiArgs &ea,
                              hipStream_t s);
 
-uint32_t auto_lanes(uint32_t rows, uint64_t nnz);
 bool valid_lanes(uint32_t lanes);
+// lanes 0: chosen from the mean row length (launch_scatter: or the windowed
+// kernel).  out[cols] of the scatter is added to.
 hipError_t launch_csr_vector(uint32_t lanes, const uint64_t *rowptr, const uint32_t *col, const float *val,
-                             const float *x, uint32_t rows, Epi epi, const EpiArgs &ea, hipStream_t s);
+                             const float *x, uint32_t rows, uint64_t nnz, Epi epi, const EpiArgs &ea, hipStream_t s);
 hipError_t launch_scatter(uint32_t lanes, const uint64_t *rowptr, const uint32_t *col, const float *val,
-                          const float *xrow, float *out, uint32_t rows, hipStream_t s);
+                          const float *xrow, float *out, uint32_t rows, uint32_t cols, uint64_t nnz, hipStream_t s);
 hipError_t launch_ratio(const int32_t *g, float *fwproj, uint32_t rows, hipStream_t s);
 // In place over bwproj: bwproj = update(f, bwproj, norm)  (calcUpdate)
 hipError_t launch_update(const float *f, const float *norm, float *bwproj, uint32_t cols, hipStream_t s);

@@ -4,7 +4,7 @@
 //    (calcFwProj_csr_vector / calcBwProj_csr_vector, kernel.cu:118-153,
 //    297-336).  Consecutive 4-byte non-temporal loads of col/val, eight
 //    rounds in flight, fixed-order xor shuffle reduction, plain store
-//    through the epilogue.
+//    through the epilogue.  csr_long_rows_kernel<EPI>: the same for long rows.
 //  * merge_*: block-level merge-path SpMV (calcFwProj_merge_based /
 //    calcBwProj_merge_based, kernel.cu:52-105,190-286).  The merge path of
 //    (row ends, nonzeros) is cut into tiles of 256*S items; each workgroup
@@ -135,6 +135,92 @@ __global__ __launch_bounds__(kWG) void csr_vector_kernel(const uint64_t *__restr
     if (row >= rows) return;  // whole groups leave together
     const EpiIn in = epi_load<EPI>(row, ea);  // every work-item of the group: one address, one request
     const float acc = group_sum<G>(row_partial<G>(col, val, x, rowptr[row], rowptr[row + 1], lane));
+    if (lane == 0) emit_with<EPI>(row, acc, in, ea);
+}
+
+// Long rows, a wave each: chunks of 1024 entries are loaded 16 bytes per
+// work-item (a quarter of the load instructions) and turned in LDS, so that
+// a gather instruction still reads 64 consecutive entries, whose columns
+// share cache lines (gathering straight from the 16-byte pieces, four
+// entries apart, misses L1 more than the saved loads are worth).  16 gathers
+// per work-item are in flight, the next chunk's loads behind them.  Chunks
+// start at a multiple of four entries (aligned pieces); pieces that reach
+// past the row's end are read entry by entry.  A wave uses its own part of
+// LDS: no barriers.
+// Bound by L1 on the gathers of x (hits on lines still being fetched): on
+// the mid-sized scanner (1085 entries per row, 1.8e8 nonzeros) FP takes 0.475
+// ms (3.0 TB/s of matrix) and BP 0.461, csr_vector_kernel 0.549 and 0.560;
+// on the 12 GB scanner 4.16 and 3.92 ms against 4.59 and 4.56.  Six pieces per
+// chunk are within 1% of four, one or two 8% slower, eight (LDS for two
+// workgroups of 256) 30%.
+// Mean entries per row from which it is used (64 work-items per row by
+// default too): rows of 440 gain 5%, of 550-620 7-23%; shorter rows leave
+// most of a chunk empty.
+constexpr uint32_t kLongMean = 384;
+constexpr int kLongNT = 512;
+constexpr int kLongQ = 4;  // 16-byte pieces of col and of val per work-item and chunk
+template <int EPI>
+__global__ __launch_bounds__(kLongNT) void csr_long_rows_kernel(const uint64_t *__restrict__ rowptr,
+                                                                const uint32_t *__restrict__ col,
+                                                                const float *__restrict__ val,
+                                                                const float *__restrict__ x, uint32_t rows,
+                                                                EpiArgs ea) {
+    constexpr int Q = kLongQ, NW = kLongNT / 64;
+    constexpr uint32_t CH = 256 * Q;  // entries per chunk
+    __shared__ __attribute__((aligned(16))) uint32_t s_c[NW][CH];
+    __shared__ __attribute__((aligned(16))) float s_v[NW][CH];
+    const uint32_t wv = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const uint32_t row = blockIdx.x * (uint32_t)NW + wv;
+    if (row >= rows) return;
+    const EpiIn in = epi_load<EPI>(row, ea);
+    const uint64_t b = rowptr[row], e = rowptr[row + 1];
+    uint32_t *sc = s_c[wv];
+    float *sv = s_v[wv];
+    u32x4 c4[Q];
+    f32x4 v4[Q];
+    auto load = [&](uint64_t k) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const uint64_t i = k + 256 * q + 4 * lane;
+            if (i + 4 <= e) {
+                c4[q] = ldnt(reinterpret_cast<const u32x4 *>(col + i));
+                v4[q] = ldnt(reinterpret_cast<const f32x4 *>(val + i));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool ok = i + j < e;
+                    c4[q][j] = ok ? col[i + j] : 0u;
+                    v4[q][j] = ok ? val[i + j] : 0.0f;
+                }
+            }
+        }
+    };
+    float acc = 0.0f;
+    const uint64_t k0 = b & ~3ull;
+    if (b < e) load(k0);
+    for (uint64_t k = k0; k < e; k += CH) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            *reinterpret_cast<u32x4 *>(sc + 256 * q + 4 * lane) = c4[q];
+            *reinterpret_cast<f32x4 *>(sv + 256 * q + 4 * lane) = v4[q];
+        }
+        if (k + CH < e) load(k + CH);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        float xv[4 * Q], vv[4 * Q];
+#pragma unroll
+        for (int u = 0; u < 4 * Q; ++u) {
+            const uint64_t i = k + 64 * u + lane;
+            vv[u] = sv[64 * u + lane];
+            xv[u] = (i >= b && i < e) ? x[sc[64 * u + lane]] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4 * Q; ++u) {
+            const uint64_t i = k + 64 * u + lane;
+            if (i >= b && i < e) acc += vv[u] * xv[u];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    acc = group_sum<64>(acc);
     if (lane == 0) emit_with<EPI>(row, acc, in, ea);
 }
 
@@ -599,21 +685,37 @@ uint32_t auto_lanes(uint32_t rows, uint64_t nnz) {
     return 64;
 }
 
+template <int EPI>
+hipError_t launch_csr_long(const uint64_t *rowptr, const uint32_t *col, const float *val, const float *x,
+                           uint32_t rows, const EpiArgs &ea, hipStream_t s) {
+    hipLaunchKernelGGL(csr_long_rows_kernel<EPI>, dim3(blocks_for(rows, kLongNT / 64)), dim3(kLongNT), 0, s, rowptr, col,
+                       val, x, rows, ea);
+    return hipGetLastError();
+}
+
 hipError_t launch_csr_vector(uint32_t lanes, const uint64_t *rowptr, const uint32_t *col, const float *val,
-                             const float *x, uint32_t rows, Epi epi, const EpiArgs &ea, hipStream_t s) {
+                             const float *x, uint32_t rows, uint64_t nnz, Epi epi, const EpiArgs &ea, hipStream_t s) {
     if (rows == 0) return hipSuccess;
-    switch (lanes) {
+    switch (lanes ? lanes : auto_lanes(rows, nnz)) {
         case 4: return launch_csr_vector_g<4>(rowptr, col, val, x, rows, epi, ea, s);
         case 8: return launch_csr_vector_g<8>(rowptr, col, val, x, rows, epi, ea, s);
         case 16: return launch_csr_vector_g<16>(rowptr, col, val, x, rows, epi, ea, s);
         case 32: return launch_csr_vector_g<32>(rowptr, col, val, x, rows, epi, ea, s);
-        default: return launch_csr_vector_g<64>(rowptr, col, val, x, rows, epi, ea, s);
+        default: break;
+    }
+    if (nnz < (uint64_t)kLongMean * rows) return launch_csr_vector_g<64>(rowptr, col, val, x, rows, epi, ea, s);
+    switch (epi) {
+        case EPI_PLAIN: return launch_csr_long<EPI_PLAIN>(rowptr, col, val, x, rows, ea, s);
+        case EPI_RATIO: return launch_csr_long<EPI_RATIO>(rowptr, col, val, x, rows, ea, s);
+        default: return launch_csr_long<EPI_UPDATE>(rowptr, col, val, x, rows, ea, s);
     }
 }
 
 hipError_t launch_scatter(uint32_t lanes, const uint64_t *rowptr, const uint32_t *col, const float *val,
-                          const float *xrow, float *out, uint32_t rows, hipStream_t s) {
+                          const float *xrow, float *out, uint32_t rows, uint32_t cols, uint64_t nnz, hipStream_t s) {
+    (void)cols;
     if (rows == 0) return hipSuccess;
+    if (lanes == 0) lanes = auto_lanes(rows, nnz);
     switch (lanes) {
         case 4: return launch_scatter_g<4>(rowptr, col, val, xrow, out, rows, s);
         case 8: return launch_scatter_g<8>(rowptr, col, val, xrow, out, rows, s);

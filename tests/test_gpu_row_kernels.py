@@ -82,3 +82,39 @@ def test_long_rows(lens, cols, kind):
         dx, out = M.DeviceArray.from_numpy(x2), M.DeviceArray(A.rows, np.float32)
         M.fp_csr_vector(rp, ci, va, dx, out, A.rows, A.nnz)
         assert np.array_equal(np.isfinite(out.numpy()), np.isfinite(y2))
+
+
+@pytest.mark.parametrize("lens", LENS)
+@pytest.mark.parametrize("cols,kind", [(50000, "sorted"), (70000, "edges"), (32768, "sorted"), (33000, "unsorted"),
+                                       (40, "sorted")])
+def test_scatter_windows(lens, cols, kind):
+    lengths = LENS[lens]
+    A = matrix(lengths, cols, 4, kind)
+    rows_per_wg = -(-A.rows // 256)
+    windows = 16 * A.nnz >= -(-A.rows // rows_per_wg) * cols  # else one atomic per entry
+    r = np.random.default_rng(5).random(A.rows).astype(np.float32)
+    r[::5] = 0.0
+    m = A.to_scipy().astype(np.float64).T
+    y, mag = m @ r.astype(np.float64), m @ r.astype(np.float64)
+    n = np.bincount(A.col, minlength=cols)
+    with M.ResidentMatrix(A) as mm:
+        rp, ci, va = mm.device_arrays()[:3]
+        dr, out = M.DeviceArray.from_numpy(r), M.DeviceArray.from_numpy(np.full(cols, 7.0, np.float32))
+        for lanes in (0, 64):  # the automatic choice, one atomic per entry
+            M.bp_scatter(rp, ci, va, dr, out, A.rows, cols, A.nnz, lanes)
+            err = np.abs(out.numpy() - y)
+            assert np.all(err <= (n + 64) * EPS * mag), (lanes, windows)
+
+
+def test_scatter_windows_over_several_rounds_of_rows():
+    """More rows than one workgroup per CU holds (262,144)."""
+    lens = np.random.default_rng(6).integers(0, 12, 300001)
+    A = matrix(list(lens), 1500, 7, "unsorted")
+    r = np.random.default_rng(8).random(A.rows).astype(np.float32)
+    y = A.to_scipy().astype(np.float64).T @ r.astype(np.float64)
+    n = np.bincount(A.col, minlength=A.cols)
+    with M.ResidentMatrix(A) as mm:
+        rp, ci, va = mm.device_arrays()[:3]
+        dr, out = M.DeviceArray.from_numpy(r), M.DeviceArray(A.cols, np.float32)
+        M.bp_scatter(rp, ci, va, dr, out, A.rows, A.cols, A.nnz)
+        assert np.all(np.abs(out.numpy() - y) <= (n + 64) * EPS * y)

@@ -330,7 +330,7 @@ int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev *
 }
 
 // The blocked path for one side (0: A, 1: A^T): tiles (built on first use),
-// a work list of about `groups` runs (0: 24 per CU) and the partial-sum
+// a work list of about `groups` runs (0: the default) and the partial-sum
 // buffer for BC right-hand sides.  MLEM_ERR_UNSUPPORTED when the matrix or
 // the LDS does not allow the shape.
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
@@ -342,12 +342,10 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
     uint32_t flags = 0;
     const Tiled *t = nullptr;
     if (int st = get_tiled(m, which, W, R, vt, BC > 1, &t, &flags)) return st;
-    int dev = 0, lds_max = 65536, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
+    int dev = 0, lds_max = 65536;
+    if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    }
-    const uint32_t target = groups ? groups : 24u * (uint32_t)std::max(1, cus);
+    const uint32_t target = groups ? groups : default_tile_groups(m->nnz, vt, BC);
     const TileWorkDev *w = nullptr;
     if (int st = get_tile_work(m, const_cast<Tiled *>(t), target, &w)) return st;
     if (tiled_lds_bytes(t->plan, w->view.span, BC) + 4096 > (size_t)lds_max)
@@ -359,26 +357,51 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
     return MLEM_OK;
 }
 
-uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t BC) {
+static uint32_t device_cus() {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const uint64_t target = groups ? groups : (BC == 1 ? 24u : 8u) * (uint64_t)std::max(1, cus);
+    return (uint32_t)std::max(1, cus);
+}
+
+// Every run writes R partial sums that the reduction reads back, and fills
+// its pipeline once; a run also has to be long enough to pay for that, while
+// more runs than the chip holds at a time balance its end.  With u units of
+// 2048 entries per run at 24 runs per CU, one right-hand side, us per
+// iteration (2048 rows x 24 / 1024 x 12 / 2048 x 12):
+//   f32    u = 2.2   99.8 /  87.8 /  91.5    16-bit   84.6 /  75.8 /  77.3
+//   f32    u = 6.6  223.6 / 203.7 / 210.6    16-bit  173.8 / 165.7 / 165.0
+//   f32    u = 11   343.8 / 319.2 / 324.3    16-bit  264.3 / 264.0 / 258.2
+//   f32    u = 14   434.6 / 415.2 / 417.9    16-bit  329.7 / 343.5 / 327.1
+//   f32    u = 31   906.2 / 872.3 / 882.6    16-bit  678.2 / 718.5 / 674.1
+//   f32    u = 54    1437 /  1463 /  1448    16-bit   1095 /  1215 /  1136
+// so 12 runs per CU up to 40 units (24 with 16-bit values, which cost less
+// per entry), of 1024 rows (16-bit values: up to 8 units).  Under two units
+// a run's partial sums cost as much as its entries: 512 rows.
+uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
+    const uint32_t cus = device_cus();
+    if (BC != 1) return 8u * cus;
+    const uint64_t u = nnz / (24ull * cus * kTileUnit);
+    return (u >= 2 && u < (vt == VAL_F32 ? 40u : 24u) ? 12u : 24u) * cus;
+}
+
+uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC) {
+    const uint64_t target = groups ? groups : (BC == 1 ? 24u : 8u) * (uint64_t)device_cus();
     if (nnz < target * 2 * kTileUnit) return 512u;
-    return BC == 1 ? 2048u : 1024u;
+    if (BC != 1) return 1024u;
+    return !groups && nnz < target * (vt == VAL_F32 ? 40u : 8u) * kTileUnit ? 1024u : 2048u;
 }
 
 // Chooses the blocked (LDS-tiled) or the plain merge path for one side of
-// the iteration.  The blocked path (default tiles of 2048 rows, 512 for
-// small matrices, x 1024 columns) runs about tile_groups workgroups (0: 24
-// per CU); secsize applies to the plain merge path only.  16-bit values need
-// the blocked path.
+// the iteration.  The blocked path (default_tile_rows x 1024 columns) runs
+// about tile_groups workgroups (0: default_tile_groups); secsize applies to
+// the plain merge path only.  16-bit values need the blocked path.
 int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t secsize, const Tiled **tiled,
                      const TileWorkDev **work, DevBuf *part, const Partition **partn, DevBuf *scratch) {
     *tiled = nullptr;
     *work = nullptr;
     if (o.tile_width != 1) {
         const uint32_t W = o.tile_width == 0 ? 1024u : o.tile_width;
-        const uint32_t R = o.tile_rows == 0 ? default_tile_rows(m->nnz, o.tile_groups, 1) : o.tile_rows;
+        const uint32_t R = o.tile_rows == 0 ? default_tile_rows(m->nnz, o.tile_groups, o.values, 1) : o.tile_rows;
         const int st = setup_tiled(m, which, W, R, o.values, 1, o.tile_groups, tiled, work, part);
         if (st == MLEM_OK || m->tiles_only) return st;
         // Automatic width with f32 values: a matrix the tiles do not suit, or

@@ -253,13 +253,11 @@ int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t sec
                      const TileWorkDev **work, DevBuf *part, const Partition **partn, DevBuf *scratch);
 // FP64 column sums of A (s32 and s64 may be null).
 int sens_on_device(const mlem_matrix *m, float *s32, double *s64_or_null, hipStream_t s);
-// Rows per tile block of the blocked kernels for BC right-hand sides when
-// none is asked for, on the current device: 512 when the matrix's runs
-// (about `groups` of them; 0: 24 per CU for one right-hand side, 8 for
-// several) would hold under two units of entries each -- a run's partial
-// sums (4 bytes per row of its block and right-hand side) would then cost
-// about as much as its entries -- else 2048 (one) or 1024 (several).
-uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t BC);
+// Runs (workgroups) per blocked SpMV and rows per tile block for BC
+// right-hand sides and `vt` values when none are asked for, on the current
+// device (groups 0: the default runs).
+uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC);
+uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC);
 // Batch slots without waiting on the host (the serving loop): the set
 // copies g (rows) and f0 (cols) in and marks the slot active, allocating its
 // pass if that is the first slot set in it (*allocated = bytes allocated,

@@ -324,7 +324,7 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
         o.tile_rows = m->tile_R;
         o.values = m->tile_vt;
     }
-    // Defaults: 1024 x 2048 for one per pass, 1024 x 1024 for 4 (3.28x the
+    // Defaults: 1024 x 2048 (1024 up to mid sizes) for one per pass, 1024 x 1024 for 4 (3.28x the
     // single FP32 path at C2 against 3.17x for 512 x 2048), 512 x 1024 for 8;
     // 512 rows for small matrices (default_tile_rows).
     const uint32_t W = o.tile_width ? o.tile_width : (BC == 8 ? 512u : 1024u);
@@ -333,7 +333,7 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
            "mlem_batch_create: tile_rows must be 512 ... 16384 (a power of two)");
     ARGCHK(valid_stream_threads(o.tile_threads), "mlem_batch_create: tile_threads must be 0, 128, 256 or 512");
     HIPCHK(hipSetDevice(m->device));
-    const uint32_t R = o.tile_rows ? o.tile_rows : default_tile_rows(m->nnz, o.tile_groups, BC);
+    const uint32_t R = o.tile_rows ? o.tile_rows : default_tile_rows(m->nnz, o.tile_groups, o.values, BC);
     auto b = std::make_unique<mlem_batch>();
     b->m = m;
     b->slots = slots;
@@ -344,9 +344,7 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     b->rows_x = (m->rows + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
     b->cols_x = (m->cols + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
     HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const uint32_t groups = o.tile_groups ? o.tile_groups : (BC == 1 ? 24u : 8u) * (uint32_t)std::max(1, cus);
+    const uint32_t groups = o.tile_groups ? o.tile_groups : default_tile_groups(m->nnz, o.values, BC);
     if (int st = setup_tiled(m, 0, W, R, o.values, BC, groups, &b->tfp, &b->wfp, nullptr)) return st;
     if (int st = setup_tiled(m, 1, W, R, o.values, BC, groups, &b->tbp, &b->wbp, nullptr)) return st;
     if (int st = batch_alloc_part(b.get(), b->passes, 0)) return st;

@@ -207,14 +207,16 @@ typedef struct mlem_opts {
                              1 = plain merge path; 1024 or 2048 = blocked
                              with that segment width (an error if the
                              matrix does not allow it)                       */
-    uint32_t tile_rows;   /* rows per block of the blocked kernels: 0 = 2048
-                             (512 when nnz < 2 x 2048 x the workgroup
-                             count: a run's partial sums would cost as much
-                             as its entries), or 512, 1024, 2048, 4096,
-                             8192, 16384                                     */
+    uint32_t tile_rows;   /* rows per block of the blocked kernels: 0 = 2048,
+                             1024 for mid-sized matrices (nnz < 40 x 2048 x
+                             24 per CU with f32 values, a fifth of that with
+                             16-bit ones, and tile_groups 0), 512 for small
+                             ones (nnz < 2 x 2048 x the workgroup count: a
+                             run's partial sums would cost as much as its
+                             entries), or 512, 1024, 2048, 4096, 8192, 16384 */
     uint32_t tile_groups; /* workgroups per blocked SpMV (runs of equal
                              length over each row block's tiles):
-                             0 = 24 per CU                                   */
+                             0 = 24 per CU, 12 for mid-sized matrices       */
     uint32_t values;      /* stored matrix values of the blocked kernels:
                              0 = f32, 1 = bf16, 2 = fp16, 3 = uf16 (an
                              unsigned 16-bit float for nonnegative matrices:
@@ -380,8 +382,8 @@ typedef struct mlem_batch_opts {
     uint32_t per_pass;    /* slots per pass over the matrix: 1, 4, 8
                              (0 = 4)                                       */
     uint32_t tile_width;  /* 0 = automatic (512 for 8 per pass, else 1024) */
-    uint32_t tile_rows;   /* 0 = automatic (2048 for 1 per pass, else 1024;
-                             512 for small matrices, as in mlem_opts)        */
+    uint32_t tile_rows;   /* 0 = automatic (as in mlem_opts for 1 per pass,
+                             else 1024, 512 for small matrices)              */
     uint32_t tile_groups; /* workgroups per blocked SpMV, 0 = automatic    */
     uint32_t tile_threads; /* work-items per workgroup of the kernel for
                               4 or 8 per pass: 128, 256 or 512 (each takes

@@ -35,6 +35,88 @@ int hip_err(hipError_t e, const char *what, const char *file, int line) {
     return set_err(st, "%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
 }
 
+hipError_t DevBuf::alloc(size_t n) {
+    reset();
+    if (n == 0) return hipSuccess;
+    hipError_t e = hipMalloc(&p, n);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        scratch_trim();
+        e = hipMalloc(&p, n);
+    }
+    if (e == hipSuccess)
+        bytes = n;
+    else
+        p = nullptr;
+    return e;
+}
+
+// The kept scratch of one device.  Never destroyed: at process exit the HIP
+// runtime may be gone before it.
+struct Kept {
+    std::atomic<bool> busy{false};
+    void *p = nullptr;
+    size_t bytes = 0;
+    void free() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+};
+
+static Kept *kept_scratch() {
+    static std::mutex mu;
+    static auto *all = new std::map<int, Kept>;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    std::lock_guard<std::mutex> lk(mu);
+    return &(*all)[dev];
+}
+
+hipError_t Scratch::get(size_t n) {
+    Kept *k = n <= kKept ? kept_scratch() : nullptr;
+    if (k && !k->busy.exchange(true)) {
+        if (k->bytes < n) {
+            k->free();
+            const hipError_t e = hipMalloc(&k->p, n);
+            if (e != hipSuccess) {
+                k->p = nullptr;
+                k->busy = false;
+                return e;
+            }
+            k->bytes = n;
+        }
+        held = k;
+        p = k->p;
+        bytes = k->bytes;
+        return hipSuccess;
+    }
+    const hipError_t e = own.alloc(n);
+    p = own.p;
+    bytes = own.bytes;
+    return e;
+}
+
+Scratch::~Scratch() {
+    if (!held) return;
+    (void)hipStreamSynchronize(nullptr);  // also where the call failed half way
+    held->busy = false;
+}
+
+void scratch_trim() {
+    Kept *k = kept_scratch();
+    if (!k || k->busy.exchange(true)) return;
+    k->free();
+    k->busy = false;
+}
+
+hipError_t free_device_bytes(size_t *free_b) {
+    scratch_trim();
+    size_t total = 0;
+    *free_b = 0;
+    return hipMemGetInfo(free_b, &total);
+}
+
 // Host-side checks of a CSR's row pointers before it reaches the GPU (a bad
 // row pointer would make the kernels read outside their arrays); its column
 // indices are checked on the device once uploaded (check_columns_device).
@@ -67,47 +149,47 @@ int check_columns_device(const char *what, const uint32_t *col, uint64_t nnz, ui
                    (unsigned long long)k, cols);
 }
 
-// Host array -> device: small copies directly, large ones through four
-// pinned 64 MiB buffers in rotation, filled by the host library's OpenMP
-// threads while the previous buffers go to the device (pageable copies run
-// on the calling thread, which OpenMP may have bound to one core).
-int upload_h2d(void *dst, const void *src, size_t bytes) {
-    constexpr size_t kChunk = size_t(64) << 20;
-    if (bytes <= 2 * kChunk) {
+Upload::~Upload() {
+    if (s) (void)hipStreamSynchronize(s);
+    for (int i = 0; i < kBufs; ++i) {
+        if (host[i]) (void)hipHostFree(host[i]);
+        if (done[i]) (void)hipEventDestroy(done[i]);
+    }
+    if (s) (void)hipStreamDestroy(s);
+}
+
+int Upload::copy(void *dst, const void *src, size_t bytes) {
+    const int st = queue(dst, src, bytes);
+    if (st != MLEM_OK && s) (void)hipStreamSynchronize(s);  // nothing in flight into arrays the caller frees
+    return st;
+}
+
+int Upload::queue(void *dst, const void *src, size_t bytes) {
+    if (bytes <= kDirect) {
         if (bytes) HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
         return MLEM_OK;
     }
-    constexpr int kBufs = 4;
-    struct Staging {
-        void *host[kBufs] = {};
-        hipEvent_t done[kBufs] = {};
-        hipStream_t s = nullptr;
-        ~Staging() {
-            if (s) (void)hipStreamSynchronize(s);
-            for (int i = 0; i < kBufs; ++i) {
-                if (host[i]) (void)hipHostFree(host[i]);
-                if (done[i]) (void)hipEventDestroy(done[i]);
-            }
-            if (s) (void)hipStreamDestroy(s);
+    if (!s) {
+        HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        for (int i = 0; i < kBufs; ++i) {
+            HIPCHK(hipHostMalloc(&host[i], kChunk, hipHostMallocDefault));
+            HIPCHK(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
         }
-    } st;
-    HIPCHK(hipStreamCreateWithFlags(&st.s, hipStreamNonBlocking));
-    for (int i = 0; i < kBufs; ++i) {
-        HIPCHK(hipHostMalloc(&st.host[i], kChunk, hipHostMallocDefault));
-        HIPCHK(hipEventCreateWithFlags(&st.done[i], hipEventDisableTiming));
     }
-    bool used[kBufs] = {};
-    int i = 0;
-    for (size_t off = 0; off < bytes; off += kChunk, i = (i + 1) % kBufs) {
+    for (size_t off = 0; off < bytes; off += kChunk, next = (next + 1) % kBufs) {
         const size_t len = std::min(kChunk, bytes - off);
-        if (used[i]) HIPCHK(hipEventSynchronize(st.done[i]));
-        if (int e = mlem_host_copy(st.host[i], static_cast<const uint8_t *>(src) + off, len, 0))
+        if (used[next]) HIPCHK(hipEventSynchronize(done[next]));
+        if (int e = mlem_host_copy(host[next], static_cast<const uint8_t *>(src) + off, len, 0))
             return set_err(e, "upload: %s", mlem_host_last_error());
-        HIPCHK(hipMemcpyAsync(static_cast<uint8_t *>(dst) + off, st.host[i], len, hipMemcpyHostToDevice, st.s));
-        HIPCHK(hipEventRecord(st.done[i], st.s));
-        used[i] = true;
+        HIPCHK(hipMemcpyAsync(static_cast<uint8_t *>(dst) + off, host[next], len, hipMemcpyHostToDevice, s));
+        HIPCHK(hipEventRecord(done[next], s));
+        used[next] = true;
     }
-    HIPCHK(hipStreamSynchronize(st.s));
+    return MLEM_OK;
+}
+
+int Upload::wait() {
+    if (s) HIPCHK(hipStreamSynchronize(s));
     return MLEM_OK;
 }
 
@@ -172,7 +254,7 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     const uint64_t *rp = which == 0 ? m->rowptr.as<uint64_t>() : m->rowptrT.as<uint64_t>();
     const uint32_t *ci = which == 0 ? m->col.as<uint32_t>() : m->colT.as<uint32_t>();
     const float *va = which == 0 ? m->val.as<float>() : m->valT.as<float>();
-    size_t free_b = 0, total_b = 0;
+    size_t free_b = 0;
     const size_t margin = (size_t)1 << 30;
     uint32_t nr = 0;
     // A in the row order (A'), and for A^T its transpose: A^T's columns are
@@ -202,7 +284,7 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
             ci = trow.as<uint32_t>();
             if (vt == VAL_F32) {
                 HIPCHK(o_valT.alloc(sizeof(float) * std::max<uint64_t>(1, m->nnz)));
-                HIPCHK(hipMemGetInfo(&free_b, &total_b));
+                HIPCHK(free_device_bytes(&free_b));
                 HIPCHK(transpose_in_ranges(m->rows, m->cols, m->nnz, arp, aci, ava, tcp.as<uint64_t>(),
                                            trow.as<uint32_t>(), o_valT.as<float>(),
                                            free_b > margin ? free_b - margin : 0, &nr, nullptr));
@@ -231,7 +313,7 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
         uint64_t *tc = ordered ? tcp.as<uint64_t>() : tcp_l.as<uint64_t>();
         uint32_t *tr = ordered ? trow.as<uint32_t>() : trow_l.as<uint32_t>();
         HIPCHK(codesT.alloc(sizeof(float) * std::max<uint64_t>(1, m->nnz)));
-        HIPCHK(hipMemGetInfo(&free_b, &total_b));
+        HIPCHK(free_device_bytes(&free_b));
         HIPCHK(transpose_in_ranges(m->rows, m->cols, m->nnz, arp, aci, codes.as<float>(), tc, tr,
                                    codesT.as<float>(), free_b > margin ? free_b - margin : 0, &nr, nullptr));
         HIPCHK(t->sens.alloc(sizeof(float) * std::max<size_t>(1, m->cols)));
@@ -241,8 +323,12 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
         va = codesT.as<float>();
         t->plan.unit_scale = true;
     }
-    DevBuf scratch;
-    HIPCHK(scratch.alloc(tile_count_scratch_bytes(t->plan)));
+    // The fill's scratch behind the count's where the kept scratch holds
+    // both (its size is known after the count; the guess covers padding).
+    const size_t count_b = (tile_count_scratch_bytes(t->plan) + 255) & ~size_t(255);
+    const size_t both = count_b + m->nnz * (vt == VAL_F32 ? 5 : 7) + 4096;
+    Scratch scratch;
+    HIPCHK(scratch.get(both <= Scratch::kKept ? both : count_b));
     uint32_t fl = 0;
     HIPCHK(launch_tile_count(t->plan, rp, ci, scratch.p, &fl, nullptr));
     if (fl) {
@@ -254,9 +340,14 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     HIPCHK(t->mem.alloc(tiled_matrix_bytes(t->plan)));
     t->view = tiled_matrix_view(t->plan, t->mem.p);
     {
-        DevBuf fill_scratch;
-        HIPCHK(fill_scratch.alloc(tile_fill_scratch_bytes(t->plan)));
-        HIPCHK(launch_tile_fill(t->plan, rp, ci, va, t->mem.p, scratch.p, fill_scratch.p, &fl, nullptr));
+        const size_t fill_b = tile_fill_scratch_bytes(t->plan);
+        DevBuf own;
+        void *fill = static_cast<char *>(scratch.p) + count_b;
+        if (count_b + fill_b > scratch.bytes) {
+            HIPCHK(own.alloc(fill_b));
+            fill = own.p;
+        }
+        HIPCHK(launch_tile_fill(t->plan, rp, ci, va, t->mem.p, scratch.p, fill, &fl, nullptr));
     }
     if (fl & 8u) return set_err(MLEM_ERR_INVALID_ARGUMENT, "uf16 values need a matrix without negative values");
     if (fl) return set_err(MLEM_ERR_FORMAT, "tiling (width %u, rows %u): layout check failed (flags %u)", W, R, fl);
@@ -869,21 +960,24 @@ int mlem_matrix_create(int device, uint32_t rows, uint32_t cols, uint64_t nnz, c
     HIPCHK(m->rowptr.alloc(sizeof(uint64_t) * ((size_t)rows + 1)));
     HIPCHK(m->col.alloc(sizeof(uint32_t) * nnz));
     HIPCHK(m->val.alloc(sizeof(float) * nnz));
-    if (int st = upload_h2d(m->rowptr.p, rowptr, m->rowptr.bytes)) return st;
+    Upload up;
+    if (int st = up.copy(m->rowptr.p, rowptr, m->rowptr.bytes)) return st;
     if (nnz) {
-        if (int st = upload_h2d(m->col.p, col, m->col.bytes)) return st;
-        if (int st = upload_h2d(m->val.p, val, m->val.bytes)) return st;
+        if (int st = up.copy(m->col.p, col, m->col.bytes)) return st;
+        if (int st = up.copy(m->val.p, val, m->val.bytes)) return st;
     }
+    if (int st = up.wait()) return st;
     if (int st = check_columns_device("mlem_matrix_create (A)", m->col.as<uint32_t>(), nnz, cols)) return st;
     if (rowptrT) {
         HIPCHK(m->rowptrT.alloc(sizeof(uint64_t) * ((size_t)cols + 1)));
         HIPCHK(m->colT.alloc(sizeof(uint32_t) * nnz));
         HIPCHK(m->valT.alloc(sizeof(float) * nnz));
-        if (int st = upload_h2d(m->rowptrT.p, rowptrT, m->rowptrT.bytes)) return st;
+        if (int st = up.copy(m->rowptrT.p, rowptrT, m->rowptrT.bytes)) return st;
         if (nnz) {
-            if (int st = upload_h2d(m->colT.p, colT, m->colT.bytes)) return st;
-            if (int st = upload_h2d(m->valT.p, valT, m->valT.bytes)) return st;
+            if (int st = up.copy(m->colT.p, colT, m->colT.bytes)) return st;
+            if (int st = up.copy(m->valT.p, valT, m->valT.bytes)) return st;
         }
+        if (int st = up.wait()) return st;
         if (int st = check_columns_device("mlem_matrix_create (A^T)", m->colT.as<uint32_t>(), nnz, rows)) return st;
         m->has_T = true;
     }
@@ -925,13 +1019,14 @@ int mlem_matrix_load_csr4(int device, const char *path, int threads, mlem_matrix
         if (rows) std::memcpy(rp.data() + 1, ends, sizeof(uint64_t) * rows);
         HIPCHK(hipMemcpy(m->rowptr.p, rp.data(), m->rowptr.bytes, hipMemcpyHostToDevice));
     }
-    // Four pinned buffers of 128 MiB in rotation: while buffer i goes to the
+    // Four pinned buffers of 32 MiB in rotation (as in Upload, new pinned pages
+    // cost more than the copies through them): while buffer i goes to the
     // device (copy stream) and is split into col / val (split stream), the
     // host library's OpenMP threads fill buffer i+1 from the mapped file.
     // (Threads started here would inherit the one core that OpenMP binds a
     // process's initial thread to under OMP_PROC_BIND: a fifth of the rate.)
     constexpr int kBufs = 4;
-    constexpr size_t kChunk = size_t(128) << 20;  // a multiple of the 8-byte entry
+    constexpr size_t kChunk = size_t(32) << 20;  // a multiple of the 8-byte entry
     const uint64_t total = 8 * nnz;
     // Declared before the streams: on an early return the streams are
     // synchronized (Staging's destructor) before these are freed.
@@ -1013,20 +1108,27 @@ int mlem_matrix_build_transpose_limited(mlem_matrix *m, uint64_t scratch_bytes, 
            m->users.load());
     HIPCHK(hipSetDevice(m->device));
     if (ranges) *ranges = 0;
-    DevBuf scratch, rp, ci, va;
+    DevBuf rp, ci, va;
     HIPCHK(rp.alloc(sizeof(uint64_t) * ((size_t)m->cols + 1)));
     HIPCHK(ci.alloc(sizeof(uint32_t) * m->nnz));
     HIPCHK(va.alloc(sizeof(float) * m->nnz));
     const size_t whole = transpose_scratch_bytes(m->rows, m->cols, m->nnz);
     size_t budget = scratch_bytes;
-    if (budget == 0) {  // automatic: one sort when its scratch fits beside a margin, else ranges in what is free
-        size_t free_b = 0, total_b = 0;
-        HIPCHK(hipMemGetInfo(&free_b, &total_b));
+    // Automatic: one sort when its scratch fits beside a margin (or is small
+    // enough to be kept and can be had), else ranges in what is free.
+    Scratch scratch;
+    bool have = false;
+    if (budget == 0) {
         const size_t margin = (size_t)1 << 30;
-        budget = free_b > margin ? free_b - margin : 0;
+        have = whole <= Scratch::kKept && scratch.get(whole) == hipSuccess;
+        if (!have) {
+            (void)hipGetLastError();
+            HIPCHK(free_device_bytes(&budget));
+            budget = budget > margin ? budget - margin : 0;
+        }
     }
-    if (whole <= budget) {
-        HIPCHK(scratch.alloc(whole));
+    if (have || whole <= budget) {
+        if (!have) HIPCHK(scratch.get(whole));
         HIPCHK(launch_transpose(m->rows, m->cols, m->nnz, m->rowptr.as<uint64_t>(), m->col.as<uint32_t>(),
                                 m->val.as<float>(), rp.as<uint64_t>(), ci.as<uint32_t>(), va.as<float>(), scratch.p,
                                 nullptr));

@@ -70,17 +70,40 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
     }
-    hipError_t alloc(size_t n) {
-        reset();
-        bytes = n;
-        if (n == 0) return hipSuccess;
-        return hipMalloc(&p, n);
-    }
+    hipError_t alloc(size_t n);  // when memory is short, kept scratch (below) is freed first
     template <typename T>
     T *as() const {
         return static_cast<T *>(p);
     }
 };
+
+// Device scratch of a set-up call (the transpose's sort, the tile builder)
+// on the null stream, which has passed its last use when the call returns.
+// One buffer per device of up to kKept bytes is kept from call to call;
+// larger requests, and those that find it in use by another thread, get
+// memory of their own.  It is freed when an allocation fails or the free
+// memory is asked for (free_device_bytes).  Without it a one-shot
+// reconstruction on 1.8e8 nonzeros allocates and frees 13 GB, faster than
+// freed device memory comes back cleared: after a dozen of them calls of 56
+// ms took 0.3 to 3 s.
+struct Scratch {
+    static constexpr size_t kKept = size_t(8) << 30;
+    void *p = nullptr;
+    size_t bytes = 0;  // at least what was asked for
+    Scratch() = default;
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
+    ~Scratch();
+    hipError_t get(size_t n);
+
+private:
+    struct Kept *held = nullptr;
+    DevBuf own;
+};
+// Frees the kept scratch of the current device unless it is in use.
+void scratch_trim();
+// Free device memory with no scratch kept.
+hipError_t free_device_bytes(size_t *free_b);
 
 // Host-side checks of a CSR's row pointers before it reaches the GPU (a bad
 // one would make the kernels read outside their arrays); the column indices
@@ -90,8 +113,34 @@ int check_csr_host(const char *what, uint32_t rows, uint32_t cols, uint64_t nnz,
 // Column indices of an uploaded CSR: MLEM_ERR_INVALID_ARGUMENT naming the
 // first index >= cols.
 int check_columns_device(const char *what, const uint32_t *col, uint64_t nnz, uint32_t cols);
-// Host -> device copy, large ones through pinned buffers (waits).
-int upload_h2d(void *dst, const void *src, size_t bytes);
+// Host -> device copies of one call: small ones directly, large ones through
+// pinned buffers in rotation, filled by the host library's OpenMP threads
+// while the previous buffers go to the device (pageable copies run on the
+// calling thread, which OpenMP may have bound to one core).  The buffers are
+// small and serve all arrays of the call: a new pinned page costs the host
+// three times what the copy through it does (1.2 -> 4 ms per 64 MiB), and
+// 256 MiB of them per array were nearly half of a 1.6 GB upload (55 -> 32 ms,
+// 50 GB/s; the csr4 loader 57 -> 38 ms).
+// copy() returns with the source read; wait() (or the destructor) with the
+// device arrays written.
+struct Upload {
+    static constexpr size_t kChunk = size_t(16) << 20, kDirect = size_t(64) << 20;
+    static constexpr int kBufs = 4;
+    void *host[kBufs] = {};
+    hipEvent_t done[kBufs] = {};
+    bool used[kBufs] = {};
+    int next = 0;
+    hipStream_t s = nullptr;
+    Upload() = default;
+    Upload(const Upload &) = delete;
+    Upload &operator=(const Upload &) = delete;
+    ~Upload();
+    int copy(void *dst, const void *src, size_t bytes);
+    int wait();
+
+private:
+    int queue(void *dst, const void *src, size_t bytes);
+};
 
 inline uint32_t clamp_secsize(uint32_t s) { return std::min(std::max(s, 1u), kMaxSecsize); }
 

@@ -133,7 +133,6 @@ int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t limit) {
         const hipError_t e = b->part.alloc(n * one);
         b->group = n;
         if (e == hipSuccess) return MLEM_OK;
-        b->part.bytes = 0;
         if (n == 1 || e != hipErrorOutOfMemory) HIPCHK(e);
         (void)hipGetLastError();
     }

@@ -119,8 +119,8 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     m->tile_bc = BC;
     const size_t margin = (size_t)1 << 30;
     auto avail = [&](size_t *b) -> int {
-        size_t free_b = 0, total_b = 0;
-        HIPCHK(hipMemGetInfo(&free_b, &total_b));
+        size_t free_b = 0;
+        HIPCHK(free_device_bytes(&free_b));
         *b = free_b > margin ? (free_b - margin) / 20 * 17 : 0;  // 85%: the free memory is not one piece
         if (chunk_bytes) *b = std::min<size_t>(*b, chunk_bytes);
         return MLEM_OK;
@@ -134,6 +134,7 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     ChunkedTiles bT(pT, tT.get());
     ChunkedTiles bA(tile_plan(rows, cols, nnz, W, R, values, quad), tA.get());
     DevBuf scaleA;  // 16-bit values: A's row scales (for the sensitivity)
+    Upload up;
     {
         // A on the device; A^T's tiles from slabs of A^T's rows (column
         // ranges of A, whole row blocks of A^T), the sensitivity from the
@@ -142,11 +143,12 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
         HIPCHK(rp.alloc(sizeof(uint64_t) * ((size_t)rows + 1)));
         HIPCHK(ci.alloc(sizeof(uint32_t) * std::max<uint64_t>(1, nnz)));
         HIPCHK(va.alloc(sizeof(float) * std::max<uint64_t>(1, nnz)));
-        if (int st = upload_h2d(rp.p, rowptr, rp.bytes)) return st;
+        if (int st = up.copy(rp.p, rowptr, rp.bytes)) return st;
         if (nnz) {
-            if (int st = upload_h2d(ci.p, col, sizeof(uint32_t) * nnz)) return st;
-            if (int st = upload_h2d(va.p, val, sizeof(float) * nnz)) return st;
+            if (int st = up.copy(ci.p, col, sizeof(uint32_t) * nnz)) return st;
+            if (int st = up.copy(va.p, val, sizeof(float) * nnz)) return st;
         }
+        if (int st = up.wait()) return st;
         if (int st = check_columns_device("mlem_matrix_create_tiled", ci.as<uint32_t>(), nnz, cols)) return st;
         HIPCHK(colptrT.alloc(sizeof(uint64_t) * ((size_t)cols + 1)));
         HIPCHK(srp.alloc(sizeof(uint64_t) * ((size_t)cols + 1)));
@@ -229,12 +231,14 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             HIPCHK(rp.alloc(sizeof(uint64_t) * (rc + 1)));
             HIPCHK(ci.alloc(sizeof(uint32_t) * std::max<uint64_t>(1, n)));
             HIPCHK(hipMemcpy(rp.p, hrp.data(), rp.bytes, hipMemcpyHostToDevice));
-            if (n)
-                if (int st = upload_h2d(ci.p, col + rowptr[r0], sizeof(uint32_t) * n)) return st;
+            if (pass) HIPCHK(va.alloc(sizeof(float) * std::max<uint64_t>(1, n)));
+            if (n) {
+                if (int st = up.copy(ci.p, col + rowptr[r0], sizeof(uint32_t) * n)) return st;
+                if (pass)
+                    if (int st = up.copy(va.p, val + rowptr[r0], sizeof(float) * n)) return st;
+                if (int st = up.wait()) return st;
+            }
             if (pass == 0) return bA.count(r0, rc, n, rp.as<uint64_t>(), ci.as<uint32_t>());
-            HIPCHK(va.alloc(sizeof(float) * std::max<uint64_t>(1, n)));
-            if (n)
-                if (int st = upload_h2d(va.p, val + rowptr[r0], sizeof(float) * n)) return st;
             return bA.fill(r0, rc, n, rp.as<uint64_t>(), ci.as<uint32_t>(), va.as<float>());
         };
         for (uint32_t r0 = 0; r0 < rows; ++chunks) {

@@ -4,12 +4,13 @@
 // by column of the entries in nnz order keeps, inside every column, the
 // original nnz (= row) order, which is exactly sptrans' placement.
 //
-//   1. pack   (row, value bits) of every nonzero into one u64, in nnz order
+//   1. pack   (row, value bits) of every nonzero into one u64, in nnz order,
+//      beside a copy of its column
 //   2. stable LSD radix sort of (col, packed) pairs on the ceil(log2 cols)
-//      low key bits (rocPRIM radix_sort_pairs)
+//      low key bits (rocPRIM radix_sort_pairs between two pairs of buffers)
 //   3. unpack rowT / valT; colptrT[c] = lower_bound(sorted cols, c)
 //
-// That needs 20 bytes of scratch per nonzero.  Where it does not fit (the
+// That needs 24 bytes of scratch per nonzero.  Where it does not fit (the
 // 100 GB matrices), the same sort runs over column ranges one at a time:
 // colptrT from a column histogram and a scan; then for every range
 // [c0, c1) the nonzeros with a column in it are compacted in nnz order
@@ -27,14 +28,17 @@ namespace mlem {
 namespace {
 
 __global__ __launch_bounds__(kWG) void pack_rows_kernel(const uint64_t *__restrict__ rowptr,
+                                                        const uint32_t *__restrict__ col,
                                                         const float *__restrict__ val, uint32_t rows,
-                                                        uint64_t *__restrict__ packed) {
+                                                        uint32_t *__restrict__ keys, uint64_t *__restrict__ packed) {
     const uint32_t row = blockIdx.x * (kWG / 64) + threadIdx.x / 64;
     const uint32_t lane = threadIdx.x % 64;
     if (row >= rows) return;
     const uint64_t hi = (uint64_t)row << 32;
-    for (uint64_t k = rowptr[row] + lane; k < rowptr[row + 1]; k += 64)
+    for (uint64_t k = rowptr[row] + lane; k < rowptr[row + 1]; k += 64) {
+        keys[k] = col[k];
         packed[k] = hi | (uint64_t)__float_as_uint(val ? val[k] : 0.0f);
+    }
 }
 
 __global__ void unpack_kernel(const uint64_t *__restrict__ packed, uint64_t nnz, uint32_t *__restrict__ rowT,
@@ -122,6 +126,15 @@ size_t sort_temp_bytes(uint32_t cols, uint64_t nnz) {
     return bytes;
 }
 
+// The same between two pairs of buffers given by the caller.
+size_t sort_temp_bytes_db(uint32_t cols, uint64_t nnz) {
+    size_t bytes = 0;
+    rocprim::double_buffer<uint32_t> k(nullptr, nullptr);
+    rocprim::double_buffer<uint64_t> v(nullptr, nullptr);
+    (void)rocprim::radix_sort_pairs(nullptr, bytes, k, v, (size_t)nnz, 0u, key_bits(cols));
+    return bytes;
+}
+
 // Scratch of one column range of up to n nonzeros: keys and packed, in and
 // out, the sort's temporary storage.
 size_t range_scratch_bytes(uint32_t cols, uint64_t n) {
@@ -132,37 +145,40 @@ size_t range_scratch_bytes(uint32_t cols, uint64_t n) {
 
 size_t transpose_scratch_bytes(uint32_t rows, uint32_t cols, uint64_t nnz) {
     (void)rows;
-    return align256(nnz * 8) * 2 + align256(nnz * 4) + align256(sort_temp_bytes(cols, nnz));
+    return align256(nnz * 8) * 2 + align256(nnz * 4) * 2 + align256(sort_temp_bytes_db(cols, nnz));
 }
 
 hipError_t launch_transpose(uint32_t rows, uint32_t cols, uint64_t nnz, const uint64_t *rowptr, const uint32_t *col,
                             const float *val, uint64_t *colptrT, uint32_t *rowT, float *valT, void *scratch,
                             hipStream_t s) {
     char *p = static_cast<char *>(scratch);
-    uint64_t *packed_in = reinterpret_cast<uint64_t *>(p);
+    uint64_t *packed_a = reinterpret_cast<uint64_t *>(p);
     p += align256(nnz * 8);
-    uint64_t *packed_out = reinterpret_cast<uint64_t *>(p);
+    uint64_t *packed_b = reinterpret_cast<uint64_t *>(p);
     p += align256(nnz * 8);
-    uint32_t *keys_out = reinterpret_cast<uint32_t *>(p);
+    uint32_t *keys_a = reinterpret_cast<uint32_t *>(p);
     p += align256(nnz * 4);
-    size_t temp_bytes = sort_temp_bytes(cols, nnz);
+    uint32_t *keys_b = reinterpret_cast<uint32_t *>(p);
+    p += align256(nnz * 4);
+    size_t temp_bytes = sort_temp_bytes_db(cols, nnz);
     void *temp = p;
+    rocprim::double_buffer<uint32_t> keys(keys_a, keys_b);
+    rocprim::double_buffer<uint64_t> packed(packed_a, packed_b);
     if (nnz > 0) {
-        hipLaunchKernelGGL(pack_rows_kernel, dim3((rows + kWG / 64 - 1) / (kWG / 64)), dim3(kWG), 0, s, rowptr, val,
-                           rows, packed_in);
+        hipLaunchKernelGGL(pack_rows_kernel, dim3((rows + kWG / 64 - 1) / (kWG / 64)), dim3(kWG), 0, s, rowptr, col,
+                           val, rows, keys_a, packed_a);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        e = rocprim::radix_sort_pairs(temp, temp_bytes, col, keys_out, packed_in, packed_out, (size_t)nnz, 0u,
-                                      key_bits(cols), s);
+        e = rocprim::radix_sort_pairs(temp, temp_bytes, keys, packed, (size_t)nnz, 0u, key_bits(cols), s);
         if (e != hipSuccess) return e;
         uint64_t blocks = (nnz + kWG - 1) / kWG;
         if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL(unpack_kernel, dim3((uint32_t)blocks), dim3(kWG), 0, s, packed_out, nnz, rowT, valT);
+        hipLaunchKernelGGL(unpack_kernel, dim3((uint32_t)blocks), dim3(kWG), 0, s, packed.current(), nnz, rowT, valT);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(colptr_kernel, dim3((cols + 1 + kWG - 1) / kWG), dim3(kWG), 0, s, keys_out, nnz, cols,
-                       colptrT);
+    hipLaunchKernelGGL(colptr_kernel, dim3((cols + 1 + kWG - 1) / kWG), dim3(kWG), 0, s, keys.current(), nnz,
+                       cols, colptrT);
     return hipGetLastError();
 }
 

@@ -250,7 +250,7 @@ int mlem_matrix_create(int device, uint32_t rows, uint32_t cols, uint64_t nnz,
 /* Build A^T on the device from the resident A (stable counting sort,
  * bit-exact with the host transpose) instead of uploading one.  Replaces
  * sptrans_scanTrans_specialized (sptrans.h:397-545) as called at
- * main.cu:99-105.  The one sort needs 20 bytes of scratch per nonzero; when
+ * main.cu:99-105.  The one sort needs 24 bytes of scratch per nonzero; when
  * that is not free (the 100 GB matrices) the sort runs over column ranges
  * within the free memory, with the same result.  Refused
  * (MLEM_ERR_INVALID_ARGUMENT) while a reconstruction or batch of the matrix

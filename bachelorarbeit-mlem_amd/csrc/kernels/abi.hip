@@ -337,9 +337,41 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
         return set_err(MLEM_ERR_UNSUPPORTED, "tiling (width %u, rows %u) refused: a row is not sorted by column", W,
                        R);
     }
-    HIPCHK(t->mem.alloc(tiled_matrix_bytes(t->plan)));
-    t->view = tiled_matrix_view(t->plan, t->mem.p);
-    {
+    // Several right-hand sides: row slices where they suit the matrix.
+    if (slices_possible(t->plan)) {
+        const size_t ns = slice_stream_count(t->plan);
+        DevBuf wsteps;
+        HIPCHK(wsteps.alloc(4 * (ns + 3)));
+        uint32_t *flags = wsteps.as<uint32_t>() + ns, fh[2] = {};
+        HIPCHK(launch_slice_count(t->plan, tile_count_entries(t->plan, scratch.p), tile_count_rowpos(t->plan, scratch.p),
+                                  wsteps.as<uint32_t>(), flags, fh, nullptr));
+        std::vector<uint32_t> wb(ns + 1);
+        HIPCHK(hipMemcpy(wb.data(), wsteps.p, 4 * ns, hipMemcpyDeviceToHost));
+        uint64_t steps = 0;
+        if (!fh[0] && slice_prefix(&wb, &steps) && slices_suit(t->plan, steps, fh[1])) {
+            t->plan.slices = true;
+            t->plan.steps = steps;
+            t->plan.cap = steps * 64 + 8;
+            HIPCHK(t->mem.alloc(tiled_matrix_bytes(t->plan)));
+            t->view = tiled_matrix_view(t->plan, t->mem.p);
+            HIPCHK(hipMemcpy(t->view.wbase, wb.data(), 4 * wb.size(), hipMemcpyHostToDevice));
+            DevBuf q;
+            HIPCHK(launch_fill_u32(flags, 0u, 1, nullptr));
+            if (vt != VAL_F32) {
+                HIPCHK(q.alloc(sizeof(uint16_t) * std::max<uint64_t>(1, m->nnz)));
+                HIPCHK(launch_row_codes(t->plan, rp, va, t->view.scale, q.as<uint16_t>(), flags, nullptr));
+            }
+            HIPCHK(launch_slice_clear(t->plan, t->view, nullptr));
+            HIPCHK(launch_slice_scatter(t->plan, rp, ci, va, q.as<uint16_t>(),
+                                        tile_count_rowpos(t->plan, scratch.p), t->view.wbase, t->view.tdata, nullptr));
+            HIPCHK(hipMemcpy(&fl, flags, 4, hipMemcpyDeviceToHost));
+        } else {  // the quads' positions again
+            HIPCHK(launch_tile_count(t->plan, rp, ci, scratch.p, &fl, nullptr));
+        }
+    }
+    if (!t->plan.slices) {
+        HIPCHK(t->mem.alloc(tiled_matrix_bytes(t->plan)));
+        t->view = tiled_matrix_view(t->plan, t->mem.p);
         const size_t fill_b = tile_fill_scratch_bytes(t->plan);
         DevBuf own;
         void *fill = static_cast<char *>(scratch.p) + count_b;
@@ -352,12 +384,24 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     if (fl & 8u) return set_err(MLEM_ERR_INVALID_ARGUMENT, "uf16 values need a matrix without negative values");
     if (fl) return set_err(MLEM_ERR_FORMAT, "tiling (width %u, rows %u): layout check failed (flags %u)", W, R, fl);
     progress("tiles of %s: %u columns x %u rows, %s%s, values %u: %llu entries stored for %llu nonzeros (+%.1f%%)",
-             which ? "A^T" : "A", W, R, quad ? "quad groups" : "row steps", ordered ? " in the row order" : "", vt,
+             which ? "A^T" : "A", W, R, t->plan.slices ? "row slices" : quad ? "quad groups" : "row steps",
+             ordered ? " in the row order" : "", vt,
              (unsigned long long)(t->plan.cap - 8), (unsigned long long)m->nnz,
              m->nnz ? 100.0 * ((double)(t->plan.cap - 8) / (double)m->nnz - 1.0) : 0.0);
     *out = t.get();
     m->tiles.emplace(key, std::move(t));
     return MLEM_OK;
+}
+
+bool slice_prefix(std::vector<uint32_t> *w, uint64_t *steps) {
+    uint64_t run = 0;
+    for (uint32_t &v : *w) {  // the last element becomes the end
+        const uint32_t n = &v == &w->back() ? 0u : v;
+        v = (uint32_t)run;
+        run += n;
+    }
+    *steps = run;
+    return run < 0xffffff00ull;
 }
 
 // Progress of long builds on stderr when MLEM_VERBOSE is set (not empty, not 0).
@@ -387,13 +431,20 @@ int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev *
         return MLEM_OK;
     }
     const TilePlan &p = t->plan;
-    std::vector<uint32_t> nz(p.ntiles);
-    std::vector<uint64_t> off(p.ntiles + 1);
-    if (p.ntiles) {
-        HIPCHK(hipMemcpy(nz.data(), t->view.tile_nz, 4 * p.ntiles, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(off.data(), t->view.tile_off, 8 * (p.ntiles + 1), hipMemcpyDeviceToHost));
+    TileWorkList L;
+    if (p.slices) {
+        std::vector<uint32_t> wb(slice_stream_count(p) + 1);
+        HIPCHK(hipMemcpy(wb.data(), t->view.wbase, 4 * wb.size(), hipMemcpyDeviceToHost));
+        L = slice_work_list(p, wb.data(), target);
+    } else {
+        std::vector<uint32_t> nz(p.ntiles);
+        std::vector<uint64_t> off(p.ntiles + 1);
+        if (p.ntiles) {
+            HIPCHK(hipMemcpy(nz.data(), t->view.tile_nz, 4 * p.ntiles, hipMemcpyDeviceToHost));
+            HIPCHK(hipMemcpy(off.data(), t->view.tile_off, 8 * (p.ntiles + 1), hipMemcpyDeviceToHost));
+        }
+        L = tile_work_list(p, nz.data(), off.data(), target);
     }
-    const TileWorkList L = tile_work_list(p, nz.data(), off.data(), target);
     if (L.bad) return set_err(MLEM_ERR_FORMAT, "tiles (width %u, rows %u) are not aligned for the stream kernel", p.W, p.R);
     auto w = std::make_unique<TileWorkDev>();
     const size_t b_wl = 4 * L.wl.size(), b_tl = 4 * L.tiles.size(), b_first = 4 * L.wl_first.size(),
@@ -468,6 +519,14 @@ static uint32_t device_cus() {
 // so 12 runs per CU up to 40 units (24 with 16-bit values, which cost less
 // per entry), of 1024 rows (16-bit values: up to 8 units).  Under two units
 // a run's partial sums cost as much as its entries: 512 rows.
+//   Four right-hand sides in row slices, 8 runs per CU: a tile ends when the
+// longest of its streams does, and taller tiles balance better; two of their
+// workgroups still fit a CU.  us per iteration of 8 slots, 1024 / 2048 rows:
+//   f32    u =  32   678 /  667    16-bit   580 /  579
+//   f32    u =  43   854 /  835    16-bit   718 /  697
+//   f32    u = 163  3188 / 2841    16-bit  2671 / 2334
+// (u counts 8 runs per CU): 2048 rows from 40 units.  Eight right-hand sides
+// of 2048 rows leave one workgroup per CU (u = 163: 2798 / 4153).
 uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
     const uint32_t cus = device_cus();
     if (BC != 1) return 8u * cus;
@@ -478,6 +537,7 @@ uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
 uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC) {
     const uint64_t target = groups ? groups : (BC == 1 ? 24u : 8u) * (uint64_t)device_cus();
     if (nnz < target * 2 * kTileUnit) return 512u;
+    if (BC == 4) return nnz < target * 40 * kTileUnit ? 1024u : 2048u;
     if (BC != 1) return 1024u;
     return !groups && nnz < target * (vt == VAL_F32 ? 40u : 8u) * kTileUnit ? 1024u : 2048u;
 }

@@ -291,6 +291,10 @@ int get_partition(mlem_matrix *m, int which, uint32_t secsize, const Partition *
 // tiles-only matrix has only the ones it was built with).
 int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bool quad, const Tiled **out,
               uint32_t *flags);
+// The steps of the slices of quad tiles (wsteps of launch_slice_count, host
+// copy) as first steps in place, and their sum; false when they are too many
+// for the layout.
+bool slice_prefix(std::vector<uint32_t> *w, uint64_t *steps);
 // Work list of t for about `target` workgroups, built on first use.
 int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev **out);
 // Tiles, work list and partial-sum buffer (part null: none) of one side for

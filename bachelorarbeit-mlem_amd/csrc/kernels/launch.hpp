@@ -137,6 +137,10 @@ struct TilePlan {
     // 16-bit values that are codes already (the transposed tiles hold the
     // codes of A's tiles, so both sides use one quantized matrix): scale 1.
     bool unit_scale = false;
+    // Quad tiles stored as row slices instead (slices.hip): steps of 64
+    // entries, `steps` of them; cap counts their entries.
+    bool slices = false;
+    uint64_t steps = 0;
     uint32_t vb() const { return vt == VAL_F32 ? 4u : 2u; }  // bytes per stored value
 };
 struct TiledMatrix {
@@ -144,6 +148,7 @@ struct TiledMatrix {
     uint32_t *tile_nz = nullptr;   // [ntiles] entries including padding
     uint8_t *tdata = nullptr;      // vb+2 bytes per entry: per unit, values then group words
     float *scale = nullptr;        // [rows] value scales (16-bit values only)
+    uint32_t *wbase = nullptr;     // slices: first step of every (row block, stream, segment), and the end
 };
 // Work list on the host: 4 u32 per run {row block, first tile (index into
 // tiles), first unit in that tile, units}; 4 u32 per non-empty tile
@@ -206,6 +211,9 @@ hipError_t launch_tile_fill_into(const TilePlan &p, const uint64_t *rowptr, cons
 // it left in `scratch` (device pointers).
 const uint64_t *tile_count_offsets(const TilePlan &p, void *scratch);
 const uint32_t *tile_count_sizes(const TilePlan &p, void *scratch);
+// And the entries of every row and segment, and the rows' positions.
+const uint32_t *tile_count_entries(const TilePlan &p, void *scratch);
+uint32_t *tile_count_rowpos(const TilePlan &p, void *scratch);
 // Runs for about target_wgs workgroups from the host copies of tile_nz and
 // tile_off.
 TileWorkList tile_work_list(const TilePlan &p, const uint32_t *tile_nz, const uint64_t *tile_off,
@@ -244,6 +252,36 @@ hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const
 bool valid_stream_threads(uint32_t nt);
 hipError_t launch_tiled_reduce(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *part,
                                uint32_t BC, Epi epi, const PassEpi &ea, hipStream_t s);
+
+// Row slices (slices.hip), the other layout of quad tiles.  After
+// launch_tile_count with quads (its counts in `scratch`): the steps of every
+// (row block, stream, segment) into wsteps (slice_stream_count(p), device)
+// and the rows' places into rowloc (tile_count_rowpos: the quads' positions
+// are gone then); flags_host[0] bit 16: the layout cannot hold a row or a
+// tile, [1]: the most steps of a stream in a tile.  flags: 8 bytes on the
+// device.  The call waits.
+bool slices_possible(const TilePlan &p);
+size_t slice_stream_count(const TilePlan &p);
+hipError_t launch_slice_count(const TilePlan &p, const uint32_t *cnt, uint32_t *rowloc, uint32_t *wsteps,
+                              uint32_t *flags, uint32_t *flags_host, hipStream_t s);
+// Whether slices with `steps` steps beat the quad tiles of plan `quads`.
+bool slices_suit(const TilePlan &quads, uint64_t steps, uint32_t most);
+size_t slice_data_bytes(const TilePlan &p);                    // wbase and the steps (p.steps set)
+void slice_view(const TilePlan &p, void *mem, TiledMatrix *t);  // tm.wbase, tm.tdata within them
+size_t slice_lds_bytes(const TilePlan &p, uint32_t BC);
+// The whole matrix's steps cleared, then the rows of a CSR of whole row
+// blocks placed (wbase: of its first row block); qval: 16-bit codes or null.
+hipError_t launch_slice_clear(const TilePlan &p, const TiledMatrix &tm, hipStream_t s);
+hipError_t launch_slice_scatter(const TilePlan &p, const uint64_t *rowptr, const uint32_t *col, const float *val,
+                                const uint16_t *qval, const uint32_t *rowloc, const uint32_t *wbase, uint8_t *tdata,
+                                hipStream_t s);
+TileWorkList slice_work_list(const TilePlan &p, const uint32_t *wbase, uint32_t target_wgs);
+hipError_t launch_slice_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x,
+                                 float *part, uint32_t BC, hipStream_t s);
+// The scales (p.unit_scale: 1) and codes of a CSR's rows as the tiles store
+// them; *bad bit 8: a negative value for uf16.
+hipError_t launch_row_codes(const TilePlan &p, const uint64_t *rowptr, const float *val, float *scale, uint16_t *q,
+                            uint32_t *bad, hipStream_t s);
 
 // Sets the message of mlem_last_error() (this thread).
 void set_last_error(const char *msg);

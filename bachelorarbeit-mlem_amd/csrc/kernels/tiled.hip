@@ -61,21 +61,10 @@
 #include <cstdlib>
 #include <cstring>
 
-#include <hip/hip_fp16.h>
-
-#include "launch.hpp"
+#include "tiled_common.hpp"
 
 namespace mlem {
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-
-template <typename T>
-__device__ __forceinline__ T ldnt(const T *p) {
-    return __builtin_nontemporal_load(p);
-}
 
 constexpr uint32_t kE = kTileE;          // entries per work-item of a unit
 constexpr uint32_t kSNT = 512;           // groups per window of stream_spmv_kernel
@@ -900,34 +889,6 @@ __global__ __launch_bounds__(64 * kSlices) void blocked_reduce_sliced_kernel(
 }
 
 // ----------------------------------------------------------------- builder
-// A wave walking the entries of one row, 64 at a time, in rows sorted by
-// column: where the run of entries in the same segment that each entry
-// belongs to started (`head`, an entry index) and whether it ends there.
-struct SegWalk {
-    uint64_t head;    // start of the run that the last step ended in
-    uint32_t prev_c;  // column of the last step's last entry
-    // Entries k0..k0+63 of the row [rs, re) with column c in lane k - k0
-    // (lanes past re: any); next_c: the column of entry k0 + 64 where it is
-    // in the row.  Returns the head of this lane's run.
-    __device__ __forceinline__ uint64_t step(uint64_t rs, uint64_t re, uint64_t k0, uint32_t lane, uint32_t c,
-                                             uint32_t next_c, uint32_t wshift, bool *last, bool *unsorted) {
-        const uint64_t k = k0 + lane;
-        const bool in = k < re;
-        uint32_t p = __shfl_up(c, 1), n = __shfl_down(c, 1);
-        if (lane == 0) p = prev_c;
-        if (lane == 63) n = next_c;
-        const uint32_t seg = c >> wshift;
-        const bool starts = in && (k == rs || (p >> wshift) != seg);
-        *unsorted = in && k != rs && c < p;
-        *last = in && (k + 1 == re || (n >> wshift) != seg);
-        const uint64_t m = __ballot(starts), below = m & (~0ull >> (63u - lane));
-        const uint64_t mine = below ? k0 + (63u - __clzll(below)) : head;
-        if (m) head = k0 + (63u - __clzll(m));
-        prev_c = __shfl(c, 63);
-        return mine;
-    }
-};
-
 // cnt[r*nseg + s] = entries of row r in segment s (cnt zeroed before); bit 2
 // of *bad: a row not sorted by column, whose segment runs are not contiguous
 // (cnt is then meaningless, the writes stay inside it).  A wave per row: the
@@ -1265,9 +1226,6 @@ __global__ void fill_u16_kernel(uint16_t *__restrict__ p, uint16_t v, uint64_t n
         p[i] = v;
 }
 
-inline uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)((n + per - 1) / per); }
-constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
-
 size_t lds_bytes(uint32_t W, uint32_t R, uint32_t span, uint32_t BC) {
     return ((size_t)W + 4 + R + (BC == 1 ? kWG : 0)) * BC * 4 + (size_t)span * 16;
 }
@@ -1383,10 +1341,12 @@ bool valid_tile_config(uint32_t W, uint32_t BC) {
 bool valid_tile_rows(uint32_t R) { return R == 512 || R == 1024 || R == 2048 || R == 4096 || R == 8192 || R == 16384; }
 
 size_t tiled_lds_bytes(const TilePlan &p, uint32_t span, uint32_t BC) {
+    if (p.slices) return slice_lds_bytes(p, BC);
     return p.quad ? stream_lds_bytes(p.W, p.R, BC) : lds_bytes(p.W, p.R, span, BC);
 }
 
 size_t tiled_matrix_bytes(const TilePlan &p) {
+    if (p.slices) return slice_data_bytes(p) + align256(4 * (size_t)p.rows);
     return align256(8 * (p.ntiles + 1)) + align256(4 * p.ntiles) + align256((p.vb() + 2) * p.cap) +
            align256(4 * (size_t)p.rows);
 }
@@ -1548,6 +1508,11 @@ size_t tile_fill_scratch_bytes(const TilePlan &p) {
 TiledMatrix tiled_matrix_view(const TilePlan &p, void *mem) {
     TiledMatrix t;
     char *c = static_cast<char *>(mem);
+    if (p.slices) {
+        slice_view(p, mem, &t);
+        t.scale = p.vt == VAL_F32 ? nullptr : reinterpret_cast<float *>(c + slice_data_bytes(p));
+        return t;
+    }
     t.tile_off = reinterpret_cast<uint64_t *>(c);
     c += align256(8 * (p.ntiles + 1));
     t.tile_nz = reinterpret_cast<uint32_t *>(c);
@@ -1597,6 +1562,23 @@ hipError_t launch_tile_count(TilePlan &p, const uint64_t *rowptr, const uint32_t
 
 const uint64_t *tile_count_offsets(const TilePlan &p, void *scratch) { return count_scratch(p, scratch).tile_off; }
 const uint32_t *tile_count_sizes(const TilePlan &p, void *scratch) { return count_scratch(p, scratch).tile_nz; }
+const uint32_t *tile_count_entries(const TilePlan &p, void *scratch) { return count_scratch(p, scratch).cnt; }
+uint32_t *tile_count_rowpos(const TilePlan &p, void *scratch) { return count_scratch(p, scratch).rowpos; }
+
+hipError_t launch_row_codes(const TilePlan &p, const uint64_t *rowptr, const float *val, float *scale, uint16_t *q,
+                            uint32_t *bad, hipStream_t s) {
+    if (!p.rows) return hipSuccess;
+    hipError_t e;
+    if (p.unit_scale) {  // the values are 16-bit codes already: stored as they are
+        if ((e = launch_fill(scale, 1.0f, p.rows, s)) != hipSuccess) return e;
+    } else {
+        hipLaunchKernelGGL(row_absmax_kernel, dim3(blocks_for(p.rows, kWG / 64)), dim3(kWG), 0, s, rowptr, val, p.rows,
+                           value_scale_mult(p.vt), scale);
+    }
+    hipLaunchKernelGGL(quantize_rows_kernel, dim3(blocks_for(p.rows, kWG / 64)), dim3(kWG), 0, s, rowptr, val, p.rows,
+                       scale, p.vt, q, bad);
+    return hipGetLastError();
+}
 
 hipError_t launch_tile_fill(const TilePlan &p, const uint64_t *rowptr, const uint32_t *col, const float *val,
                             void *mem, void *scratch, void *fill_scratch, uint32_t *flags_host, hipStream_t s) {
@@ -1624,14 +1606,7 @@ hipError_t launch_tile_fill_into(const TilePlan &p, const uint64_t *rowptr, cons
     uint16_t *qval = nullptr;
     if (tm.scale && p.rows) {
         qval = reinterpret_cast<uint16_t *>(static_cast<char *>(fill_scratch) + 2 * align256(2 * p.cap));
-        if (p.unit_scale) {  // the values are 16-bit codes already: stored as they are
-            if ((e = launch_fill(tm.scale, 1.0f, p.rows, s)) != hipSuccess) return e;
-        } else {
-            hipLaunchKernelGGL(row_absmax_kernel, dim3(blocks_for(p.rows, kWG / 64)), dim3(kWG), 0, s, rowptr, val,
-                               p.rows, value_scale_mult(p.vt), tm.scale);
-        }
-        hipLaunchKernelGGL(quantize_rows_kernel, dim3(blocks_for(p.rows, kWG / 64)), dim3(kWG), 0, s, rowptr, val, p.rows,
-                           tm.scale, p.vt, qval, c.bad);
+        if ((e = launch_row_codes(p, rowptr, val, tm.scale, qval, c.bad, s)) != hipSuccess) return e;
     }
     if ((e = hipMemsetAsync(rtmp, 0xff, 2 * p.cap, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(fill_u16_kernel, dim3(1024), dim3(kWG), 0, s, ctmp, (uint16_t)p.W, p.cap);
@@ -1668,6 +1643,7 @@ hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const
                                  float *part, uint32_t BC, uint32_t nt, hipStream_t s) {
     if (x.n == 0 || x.n > kMaxPasses) return hipErrorInvalidValue;
     if (p.rows == 0 || wk.nwg == 0) return hipSuccess;
+    if (p.slices) return launch_slice_partials(p, tm, wk, x, part, BC, s);
     switch (p.vt) {
         case VAL_F32: return launch_vt<VAL_F32>(p, tm, wk, x, part, BC, nt, s);
         case VAL_BF16: return launch_vt<VAL_BF16>(p, tm, wk, x, part, BC, nt, s);

@@ -14,14 +14,34 @@ namespace {
 // over the same row blocks (the chunks may differ between them): the counts
 // give every tile's size and so the offsets of the whole layout; then, the
 // tiles allocated, each chunk fills its part.  The bytes are those that one
-// build over the whole CSR writes (every tile is laid out on its own).
+// build over the whole CSR writes (every tile is laid out on its own, and
+// the choice of row slices is made from the whole matrix's counts).
 struct ChunkedTiles {
     TilePlan P;
-    std::vector<uint64_t> size;  // padded entries per tile, then (allocate) offsets
-    std::vector<uint32_t> nz;    // entries per tile
+    std::vector<uint64_t> size;   // padded entries per tile, then (allocate) offsets
+    std::vector<uint32_t> nz;     // entries per tile
+    std::vector<uint32_t> wbase;  // row slices: steps per (row block, stream, segment), then (allocate) first steps
+    uint32_t most = 0;            // the most steps of a stream in a tile
+    bool slices;                  // still possible; from allocate() on: taken
     Tiled *t = nullptr;
 
-    ChunkedTiles(const TilePlan &p, Tiled *tiled) : P(p), size(p.ntiles + 1, 0), nz(p.ntiles, 0), t(tiled) {}
+    ChunkedTiles(const TilePlan &p, Tiled *tiled)
+        : P(p), size(p.ntiles + 1, 0), nz(p.ntiles, 0), slices(slices_possible(p)), t(tiled) {
+        if (slices) wbase.assign(slice_stream_count(p) + 1, 0);
+    }
+
+    // Where the row blocks from r0 on begin in wbase.
+    size_t stream_at(uint32_t r0) const { return slice_stream_count(P) / P.nblk * (r0 / P.R); }
+
+    // The chunk's rows placed in their slices, after count_chunk; fl as
+    // launch_slice_count leaves it.
+    int count_slices(const TilePlan &pc, const DevBuf &scratch, DevBuf *wsteps, uint32_t fl[2]) {
+        const size_t ns = slice_stream_count(pc);
+        HIPCHK(wsteps->alloc(4 * (ns + 2)));
+        HIPCHK(launch_slice_count(pc, tile_count_entries(pc, scratch.p), tile_count_rowpos(pc, scratch.p),
+                                  wsteps->as<uint32_t>(), wsteps->as<uint32_t>() + ns, fl, nullptr));
+        return MLEM_OK;
+    }
 
     // The chunk's own plan, its count into `scratch` (allocated here).
     int count_chunk(uint32_t r0, uint32_t rows_c, uint64_t nnz_c, const uint64_t *rp, const uint32_t *ci,
@@ -45,6 +65,14 @@ struct ChunkedTiles {
         if (pc.ntiles)
             HIPCHK(hipMemcpy(nz.data() + t0, tile_count_sizes(pc, scratch.p), 4 * pc.ntiles, hipMemcpyDeviceToHost));
         for (uint64_t i = 0; i < pc.ntiles; ++i) size[t0 + i] = off[i + 1] - off[i];
+        if (slices && pc.ntiles) {
+            DevBuf wsteps;
+            uint32_t cf[2] = {};
+            if (int st = count_slices(pc, scratch, &wsteps, cf)) return st;
+            HIPCHK(hipMemcpy(wbase.data() + stream_at(r0), wsteps.p, 4 * slice_stream_count(pc), hipMemcpyDeviceToHost));
+            slices = !cf[0];
+            most = std::max(most, cf[1]);
+        }
         return MLEM_OK;
     }
 
@@ -56,9 +84,21 @@ struct ChunkedTiles {
             run += n;
         }
         P.cap = run + 8;  // as one build: a multiple of 8, at least one group
+        uint64_t steps = 0;
+        slices = slices && slice_prefix(&wbase, &steps) && slices_suit(P, steps, most);
+        if (slices) {
+            P.slices = true;
+            P.steps = steps;
+            P.cap = steps * 64 + 8;
+        }
         t->plan = P;
         HIPCHK(t->mem.alloc(tiled_matrix_bytes(P)));
         t->view = tiled_matrix_view(P, t->mem.p);
+        if (slices) {
+            HIPCHK(hipMemcpy(t->view.wbase, wbase.data(), 4 * wbase.size(), hipMemcpyHostToDevice));
+            HIPCHK(launch_slice_clear(P, t->view, nullptr));
+            return MLEM_OK;
+        }
         HIPCHK(hipMemcpy(t->view.tile_off, size.data(), 8 * (P.ntiles + 1), hipMemcpyHostToDevice));
         if (P.ntiles) HIPCHK(hipMemcpy(t->view.tile_nz, nz.data(), 4 * P.ntiles, hipMemcpyHostToDevice));
         return MLEM_OK;
@@ -68,6 +108,7 @@ struct ChunkedTiles {
         TilePlan pc;
         DevBuf scratch, local_off, fill_scratch;
         if (int st = count_chunk(r0, rows_c, nnz_c, rp, ci, &pc, &scratch)) return st;
+        if (slices) return fill_slices(r0, pc, rp, ci, va, scratch);
         const uint64_t t0 = (uint64_t)(r0 / P.R) * P.nseg;
         HIPCHK(local_off.alloc(8 * (pc.ntiles + 1)));
         HIPCHK(fill_scratch.alloc(tile_fill_scratch_bytes(pc)));
@@ -78,6 +119,24 @@ struct ChunkedTiles {
         v.scale = t->view.scale ? t->view.scale + r0 : nullptr;
         uint32_t fl = 0;
         HIPCHK(launch_tile_fill_into(pc, rp, ci, va, v, scratch.p, fill_scratch.p, &fl, nullptr));
+        if (fl & 8u) return set_err(MLEM_ERR_INVALID_ARGUMENT, "uf16 values need a matrix without negative values");
+        if (fl) return set_err(MLEM_ERR_FORMAT, "tiling: layout check failed (flags %u, rows from %u)", fl, r0);
+        return MLEM_OK;
+    }
+
+    int fill_slices(uint32_t r0, const TilePlan &pc, const uint64_t *rp, const uint32_t *ci, const float *va,
+                    const DevBuf &scratch) {
+        DevBuf wsteps, q;
+        uint32_t cf[2] = {};
+        if (int st = count_slices(pc, scratch, &wsteps, cf)) return st;
+        uint32_t *bad = wsteps.as<uint32_t>() + slice_stream_count(pc), fl = 0;
+        if (P.vt != VAL_F32) {
+            HIPCHK(q.alloc(sizeof(uint16_t) * std::max<uint64_t>(1, pc.nnz)));
+            HIPCHK(launch_row_codes(pc, rp, va, t->view.scale + r0, q.as<uint16_t>(), bad, nullptr));
+        }
+        HIPCHK(launch_slice_scatter(pc, rp, ci, va, q.as<uint16_t>(), tile_count_rowpos(pc, scratch.p),
+                                    t->view.wbase + stream_at(r0), t->view.tdata, nullptr));
+        HIPCHK(hipMemcpy(&fl, bad, 4, hipMemcpyDeviceToHost));
         if (fl & 8u) return set_err(MLEM_ERR_INVALID_ARGUMENT, "uf16 values need a matrix without negative values");
         if (fl) return set_err(MLEM_ERR_FORMAT, "tiling: layout check failed (flags %u, rows from %u)", fl, r0);
         return MLEM_OK;

@@ -383,12 +383,15 @@ typedef struct mlem_batch_opts {
                              (0 = 4)                                       */
     uint32_t tile_width;  /* 0 = automatic (512 for 8 per pass, else 1024) */
     uint32_t tile_rows;   /* 0 = automatic (as in mlem_opts for 1 per pass,
-                             else 1024, 512 for small matrices)              */
+                             else 1024, 512 for small matrices, 2048 for
+                             large ones with 4 per pass)                   */
     uint32_t tile_groups; /* workgroups per blocked SpMV, 0 = automatic    */
-    uint32_t tile_threads; /* work-items per workgroup of the kernel for
-                              4 or 8 per pass: 128, 256 or 512 (each takes
-                              512 / tile_threads groups of 8 entries of a
-                              window), 0 = automatic (512)               */
+    uint32_t tile_threads; /* work-items per workgroup of the block-stream
+                              kernel for 4 or 8 per pass: 128, 256 or 512
+                              (each takes 512 / tile_threads groups of 8
+                              entries of a window), 0 = automatic (512);
+                              without effect on tiles kept as row slices
+                              (which most matrices' are)                  */
     uint32_t use_graph;    /* 1: each mlem_batch_iterate call replays one
                               iteration captured as a hipGraph (captured
                               again when the set of passes holding an

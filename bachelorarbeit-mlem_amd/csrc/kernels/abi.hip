@@ -348,7 +348,7 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
         std::vector<uint32_t> wb(ns + 1);
         HIPCHK(hipMemcpy(wb.data(), wsteps.p, 4 * ns, hipMemcpyDeviceToHost));
         uint64_t steps = 0;
-        if (!fh[0] && slice_prefix(&wb, &steps) && slices_suit(t->plan, steps, fh[1])) {
+        if (!fh[0] && slice_prefix(W, &wb, &steps, &t->plan.group) && slices_suit(t->plan, steps, fh[1])) {
             t->plan.slices = true;
             t->plan.steps = steps;
             t->plan.cap = steps * 64 + 8;
@@ -391,17 +391,6 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     *out = t.get();
     m->tiles.emplace(key, std::move(t));
     return MLEM_OK;
-}
-
-bool slice_prefix(std::vector<uint32_t> *w, uint64_t *steps) {
-    uint64_t run = 0;
-    for (uint32_t &v : *w) {  // the last element becomes the end
-        const uint32_t n = &v == &w->back() ? 0u : v;
-        v = (uint32_t)run;
-        run += n;
-    }
-    *steps = run;
-    return run < 0xffffff00ull;
 }
 
 // Progress of long builds on stderr when MLEM_VERBOSE is set (not empty, not 0).
@@ -519,25 +508,31 @@ static uint32_t device_cus() {
 // so 12 runs per CU up to 40 units (24 with 16-bit values, which cost less
 // per entry), of 1024 rows (16-bit values: up to 8 units).  Under two units
 // a run's partial sums cost as much as its entries: 512 rows.
-//   Four right-hand sides in row slices, 8 runs per CU: a tile ends when the
-// longest of its streams does, and taller tiles balance better; two of their
-// workgroups still fit a CU.  us per iteration of 8 slots, 1024 / 2048 rows:
-//   f32    u =  32   678 /  667    16-bit   580 /  579
-//   f32    u =  43   854 /  835    16-bit   718 /  697
-//   f32    u = 163  3188 / 2841    16-bit  2671 / 2334
-// (u counts 8 runs per CU): 2048 rows from 40 units.  Eight right-hand sides
-// of 2048 rows leave one workgroup per CU (u = 163: 2798 / 4153).
+//   Four right-hand sides in row slices: a tile ends when the longest of its
+// streams does, and taller tiles balance better; two of their workgroups
+// still fit a CU.  One pass alone is best at 4 runs per CU (u = 44 at 1024
+// rows, f32: 349 / 335 / 341 us per iteration with 2 / 4 / 8), several passes
+// at 2 or 4 (616 / 627 / 694).  us per iteration at 4 runs per CU, 1024 /
+// 2048 rows (u counts those):
+//   f32    u = 0.9 (8 slots)    38 /  42    16-bit     35 /  39
+//   f32    u =  13 (16 slots)  233 / 268    16-bit    200 / 234
+//   f32    u =  44 (16 slots)  627 / 617    16-bit    513 / 512
+//   f32    u =  64 (8 slots)   588 / 564    16-bit    453 / 434
+//   f32    u = 326 (8 slots)  2767 / 2492   16-bit   2098 / 1898
+// 2048 rows from 48 units.  512 rows lose at every size (u = 0.9: 39 and
+// 37).  Eight right-hand sides of 2048 rows leave one workgroup per CU
+// (u = 163 at 8 runs per CU: 2798 / 4153).
 uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
     const uint32_t cus = device_cus();
-    if (BC != 1) return 8u * cus;
+    if (BC != 1) return (BC == 4 ? 4u : 8u) * cus;
     const uint64_t u = nnz / (24ull * cus * kTileUnit);
     return (u >= 2 && u < (vt == VAL_F32 ? 40u : 24u) ? 12u : 24u) * cus;
 }
 
 uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC) {
-    const uint64_t target = groups ? groups : (BC == 1 ? 24u : 8u) * (uint64_t)device_cus();
+    const uint64_t target = groups ? groups : (BC == 1 ? 24u : BC == 4 ? 4u : 8u) * (uint64_t)device_cus();
+    if (BC == 4) return nnz < target * 48 * kTileUnit ? 1024u : 2048u;
     if (nnz < target * 2 * kTileUnit) return 512u;
-    if (BC == 4) return nnz < target * 40 * kTileUnit ? 1024u : 2048u;
     if (BC != 1) return 1024u;
     return !groups && nnz < target * (vt == VAL_F32 ? 40u : 8u) * kTileUnit ? 1024u : 2048u;
 }

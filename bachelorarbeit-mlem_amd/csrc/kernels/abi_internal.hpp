@@ -291,10 +291,6 @@ int get_partition(mlem_matrix *m, int which, uint32_t secsize, const Partition *
 // tiles-only matrix has only the ones it was built with).
 int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bool quad, const Tiled **out,
               uint32_t *flags);
-// The steps of the slices of quad tiles (wsteps of launch_slice_count, host
-// copy) as first steps in place, and their sum; false when they are too many
-// for the layout.
-bool slice_prefix(std::vector<uint32_t> *w, uint64_t *steps);
 // Work list of t for about `target` workgroups, built on first use.
 int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev **out);
 // Tiles, work list and partial-sum buffer (part null: none) of one side for
@@ -326,11 +322,8 @@ int batch_deactivate_async(mlem_batch *b, uint32_t slot);
 // place, so the images are bitwise those it would have had in `from`.
 int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to);
 // The partial-sum buffer for up to `passes` passes per launch (at most
-// kMaxPasses), fewer where the memory for them is not free; `limit` (0:
-// none) bounds its bytes, one pass always allowed.
-int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t limit);
-// What one pass of FP and one of BP would take in buffers of their own.
-uint64_t batch_part_pair_bytes(const mlem_batch *b);
+// kMaxPasses), fewer where the memory for them is not free.
+int batch_alloc_part(mlem_batch *b, uint32_t passes);
 // Frees pass p when none of its slots is active (returns the bytes freed).
 uint64_t batch_release_pass(mlem_batch *b, uint32_t p);
 // Progress of long builds on stderr when MLEM_VERBOSE is set.

@@ -118,17 +118,11 @@ int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to) {
     return MLEM_OK;
 }
 
-uint64_t batch_part_pair_bytes(const mlem_batch *b) {
-    return tiled_part_bytes(b->tfp->plan, b->wfp->view.nwg, b->BC) +
-           tiled_part_bytes(b->tbp->plan, b->wbp->view.nwg, b->BC);
-}
-
-int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t limit) {
+int batch_alloc_part(mlem_batch *b, uint32_t passes) {
     const uint64_t one = std::max<uint64_t>(4, std::max(tiled_part_bytes(b->tfp->plan, b->wfp->view.nwg, b->BC),
                                                         tiled_part_bytes(b->tbp->plan, b->wbp->view.nwg, b->BC)));
     // One right-hand side per pass: the blocked kernel takes one pass per launch.
     uint32_t n = b->BC == 1 ? 1u : std::max(1u, std::min(passes, kMaxPasses));
-    while (n > 1 && limit && n * one > limit) --n;
     for (;; n = (n + 1) / 2) {
         const hipError_t e = b->part.alloc(n * one);
         b->group = n;
@@ -346,7 +340,7 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     const uint32_t groups = o.tile_groups ? o.tile_groups : default_tile_groups(m->nnz, o.values, BC);
     if (int st = setup_tiled(m, 0, W, R, o.values, BC, groups, &b->tfp, &b->wfp, nullptr)) return st;
     if (int st = setup_tiled(m, 1, W, R, o.values, BC, groups, &b->tbp, &b->wbp, nullptr)) return st;
-    if (int st = batch_alloc_part(b.get(), b->passes, 0)) return st;
+    if (int st = batch_alloc_part(b.get(), b->passes)) return st;
     if (b->tfp->ordered != b->tbp->ordered)  // a row order set from another thread between the two builds
         return set_err(MLEM_ERR_INVALID_ARGUMENT, "mlem_batch_create: the row order changed while the tiles were built");
     if (b->tfp->ordered) b->row_order = m->row_order.as<uint32_t>();

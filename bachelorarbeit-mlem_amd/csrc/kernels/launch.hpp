@@ -141,6 +141,7 @@ struct TilePlan {
     // entries, `steps` of them; cap counts their entries.
     bool slices = false;
     uint64_t steps = 0;
+    uint32_t group = 1;  // steps taken together
     uint32_t vb() const { return vt == VAL_F32 ? 4u : 2u; }  // bytes per stored value
 };
 struct TiledMatrix {
@@ -264,6 +265,10 @@ bool slices_possible(const TilePlan &p);
 size_t slice_stream_count(const TilePlan &p);
 hipError_t launch_slice_count(const TilePlan &p, const uint32_t *cnt, uint32_t *rowloc, uint32_t *wsteps,
                               uint32_t *flags, uint32_t *flags_host, hipStream_t s);
+// The steps of the slices of tiles W columns wide (wsteps, host copy, one
+// element more) as first steps in place, their sum and the steps taken
+// together; false when they are too many for the layout.
+bool slice_prefix(uint32_t W, std::vector<uint32_t> *w, uint64_t *steps, uint32_t *group);
 // Whether slices with `steps` steps beat the quad tiles of plan `quads`.
 bool slices_suit(const TilePlan &quads, uint64_t steps, uint32_t most);
 size_t slice_data_bytes(const TilePlan &p);                    // wbase and the steps (p.steps set)

@@ -114,10 +114,10 @@ int mlem_server_add_matrix(mlem_server *s, mlem_matrix *m, uint32_t max_slots, u
     mlem_batch *b = nullptr;
     if (int st = mlem_batch_create(m, max_slots, &s->bopts, &b))
         return fail(st, "mlem_server_add_matrix: %s", std::string(mlem_last_error()).c_str());
-    // Under a budget the partial sums take no more than FP's and BP's of one
-    // pass: what several passes per launch would add goes to requests.
+    // Under a budget the partial sums are those of one pass: what several
+    // passes per launch would add goes to requests.
     if (s->budget)
-        if (int st = mlem::abi::batch_alloc_part(b, b->passes, mlem::abi::batch_part_pair_bytes(b))) {
+        if (int st = mlem::abi::batch_alloc_part(b, 1)) {
             const std::string msg = mlem_last_error();
             mlem_batch_destroy(b);
             return fail(st, "mlem_server_add_matrix: %s", msg.c_str());

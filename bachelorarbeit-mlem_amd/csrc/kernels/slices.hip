@@ -40,8 +40,8 @@
 // number of passes.  Partial sums, their reduction and the epilogue are
 // those of tiled.hip.
 //
-// What bounds it: instructions (VALU about half of the time, 12 per step)
-// and the LDS gather (16 bytes per entry and 4 right-hand sides, 40%), then
+// What bounds it: instructions (VALU two thirds of the time, 12 per step)
+// and the LDS gather (16 bytes per entry and 4 right-hand sides, 60%), then
 // the barriers (a tile waits for its longest stream).  us per launch, 4
 // passes of 4 right-hand sides over 683 M entries (16-bit) and 2 passes of 8
 // over 135 M (f32):
@@ -52,10 +52,12 @@
 //   serves all but the first; HBM reads of one pass)     2518 / 495
 //   slices to the stream with the fewest steps, 2048
 //   rows (4 right-hand sides), four staging waves        2116 / 474
-// (us per iteration of the last: 4940 / 964 before it, 4740 / 946 with the
+//   steps taken in groups, 16-24 in flight               1589 / 430
+// (us per iteration before the fifth: 4940 / 964, 4740 / 946 with the
 // dealing, 4190 with 2048 rows, 4144 / 935 with four staging waves.)
-// Sixteen steps in flight instead of eight cost registers (8544 us), and
-// non-temporal loads of the steps lose the L2 (2769).
+// Non-temporal loads of the steps lose the L2 (2769); x of two or three tiles
+// in flight instead of one, and 32-row slices of two work-items per row,
+// gained nothing.
 #include <algorithm>
 #include <vector>
 
@@ -72,8 +74,12 @@ constexpr uint32_t kRowSteps = 255;            // steps of a row in a tile at mo
 constexpr uint32_t kStreamSteps = 1u << 14;    // steps of a stream in a tile below this
 constexpr uint32_t kSliceMaxR = 2048;          // rows per block at most
 constexpr uint32_t kRunTiles = 64;             // tiles per run at most (one per lane)
-constexpr int kDepth = 8;                      // steps in flight per wave
-constexpr uint32_t kPadSteps = 2 * kDepth;     // readable past the last step
+// Steps in flight per wave, G taken together.  683 M entries in 16 bits, 4
+// right-hand sides, fours, us per iteration with 8 / 12 / 16 / 24 in flight:
+// 3600 / 3340 / 3216 / 3109.  (A loop of more groups than these is not
+// unrolled, and then the steps are not in registers: 8544.)
+constexpr int step_depth(uint32_t vt, uint32_t G) { return G == 1 ? 8 : G == 2 || vt == VAL_F32 ? 16 : 24; }
+constexpr uint32_t kPadSteps = 48;         // readable past the last step
 
 constexpr uint32_t step_bytes(uint32_t vt) { return vt == VAL_F32 ? 384u : 256u; }
 
@@ -99,18 +105,17 @@ template <int CTRL>
 __device__ __forceinline__ uint32_t quad_get(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
 }
-// The sum over the four lanes of a quad, in every lane.
-__device__ __forceinline__ float quad_sum(float v) {
-    v += __uint_as_float(quad_get<0xB1>(__float_as_uint(v)));  // lane ^ 1
-    v += __uint_as_float(quad_get<0x4E>(__float_as_uint(v)));  // lane ^ 2
-    return v;
+template <int CTRL>
+__device__ __forceinline__ float quad_getf(float v) {
+    return __uint_as_float(quad_get<CTRL>(__float_as_uint(v)));
 }
 
 // wl[run] = {row block, first tile (index into tiles), tiles}; tiles[i].x =
 // segment.  One launch takes several passes of a batch, as
 // stream_spmv_kernel does: workgroups go round the 8 XCDs, so 8 runs of one
 // pass are followed by the same runs of the next, each on its XCD.
-template <int W, int VT, int BC>
+// G steps are taken together, their gathers in flight at once.
+template <int W, int VT, int BC, int G>
 __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32_t nseg,
                                                               const uint32_t *__restrict__ wbase,
                                                               const uint4 *__restrict__ wl,
@@ -119,6 +124,8 @@ __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32
                                                               const uint8_t *__restrict__ tdata, PassX px,
                                                               uint32_t nwg, float *__restrict__ part) {
     constexpr uint32_t SB = step_bytes(VT);
+    constexpr int kDepth = step_depth(VT, G);
+    static_assert(kDepth % G == 0 && 2 * kDepth <= (int)kPadSteps, "whole groups in flight, nothing read past the end");
     constexpr uint32_t XS = (W + 4) * BC;  // floats per x slot (column W holds 0)
     constexpr int XP = W * BC / 4 / (64 * kStagers);  // 16-byte pieces of an x segment per staging work-item
     static_assert(XP * 4 * 64 * kStagers == W * BC && (BC == 4 || BC == 8), "x moves in 16-byte pieces");
@@ -195,48 +202,59 @@ __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32
     for (int b = 0; b < BC; ++b) a[b] = 0.0f;
     for (uint32_t done = 0; done < total;) {
 #pragma unroll
-        for (int j = 0; j < kDepth; ++j) {
+        for (int j0 = 0; j0 < kDepth; j0 += G) {
             if (done == total) break;
             while (left == 0) enter();  // ends: a tile with steps is left
-            const uint32_t m = rw[j];
-            float v;
-            if constexpr (VT == VAL_F32)
-                v = rv[j];
-            else
-                v = word_val<VT>(m);
-            const float *xg = reinterpret_cast<const float *>(xw + (m & 0x7ff0u) * (BC / 4));
+            f32x4 xv[G][BC / 4];
+            float v[G];
 #pragma unroll
-            for (int q = 0; q < BC / 4; ++q) {
-                const f32x4 xv = *reinterpret_cast<const f32x4 *>(xg + 4 * q);
+            for (int i = 0; i < G; ++i) {
+                const float *xg = reinterpret_cast<const float *>(xw + (rw[j0 + i] & 0x7ff0u) * (BC / 4));
 #pragma unroll
-                for (int b = 0; b < 4; ++b) a[4 * q + b] = fmaf(v, xv[b], a[4 * q + b]);
+                for (int q = 0; q < BC / 4; ++q) xv[i][q] = *reinterpret_cast<const f32x4 *>(xg + 4 * q);
+                if constexpr (VT == VAL_F32)
+                    v[i] = rv[j0 + i];
+                else
+                    v[i] = word_val<VT>(rw[j0 + i]);
             }
-            ++done;
-            --left;
-            if (__builtin_amdgcn_readfirstlane(m) & 0x8000u) {  // the slice ends: its 16 rows
-                uint32_t row = (m & 15u) << (4u * (lane & 3u));
-                row |= quad_get<0xB1>(row);
-                row |= quad_get<0x4E>(row);
+            done += G;
+            left -= G;
 #pragma unroll
-                for (int b = 0; b < BC; ++b) a[b] = quad_sum(a[b]);
-                const bool o1 = lane & 1u, o2 = lane & 2u;
-                if constexpr (BC == 4) {  // lane q of the quad: right-hand side q
-                    const float lo = o1 ? a[1] : a[0], hi = o1 ? a[3] : a[2];
-                    acc[row * 4 + (lane & 3u)] += o2 ? hi : lo;
-                } else {  // right-hand sides 2q, 2q + 1
-                    typedef float f32x2 __attribute__((ext_vector_type(2)));
-                    f32x2 *p = reinterpret_cast<f32x2 *>(acc + row * 8 + 2 * (lane & 3u));
-                    f32x2 o = *p;
-                    o.x += o2 ? (o1 ? a[6] : a[4]) : (o1 ? a[2] : a[0]);
-                    o.y += o2 ? (o1 ? a[7] : a[5]) : (o1 ? a[3] : a[1]);
-                    *p = o;
+            for (int i = 0; i < G; ++i) {
+                const uint32_t m = rw[j0 + i];
+#pragma unroll
+                for (int q = 0; q < BC / 4; ++q)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) a[4 * q + b] = fmaf(v[i], xv[i][q][b], a[4 * q + b]);
+                if (__builtin_amdgcn_readfirstlane(m) & 0x8000u) {  // the slice ends: its 16 rows
+                    uint32_t row = (m & 15u) << (4u * (lane & 3u));
+                    row |= quad_get<0xB1>(row);
+                    row |= quad_get<0x4E>(row);
+                    // Sums over the row's four work-items, halved between
+                    // neighbours: work-item q keeps BC/4 right-hand sides.
+                    const bool o1 = lane & 1u, o2 = lane & 2u;
+                    float h[BC / 2];
+#pragma unroll
+                    for (int b = 0; b < BC / 2; ++b)
+                        h[b] = (o1 ? a[b + BC / 2] : a[b]) + quad_getf<0xB1>(o1 ? a[b] : a[b + BC / 2]);
+                    float *p = acc + row * BC + (o1 ? BC / 2 : 0) + (o2 ? BC / 4 : 0);
+                    if constexpr (BC == 4) {
+                        *p += (o2 ? h[1] : h[0]) + quad_getf<0x4E>(o2 ? h[0] : h[1]);
+                    } else {
+                        typedef float f32x2 __attribute__((ext_vector_type(2)));
+                        f32x2 o = *reinterpret_cast<f32x2 *>(p);
+                        o.x += (o2 ? h[2] : h[0]) + quad_getf<0x4E>(o2 ? h[0] : h[2]);
+                        o.y += (o2 ? h[3] : h[1]) + quad_getf<0x4E>(o2 ? h[1] : h[3]);
+                        *reinterpret_cast<f32x2 *>(p) = o;
+                    }
+#pragma unroll
+                    for (int b = 0; b < BC; ++b) a[b] = 0.0f;
                 }
-#pragma unroll
-                for (int b = 0; b < BC; ++b) a[b] = 0.0f;
             }
-            // The step's registers are used up: loading into them earlier
+            // The steps' registers are used up: loading into them earlier
             // would make the compiler copy them, and a copy waits.
-            fetch(j, src + (kDepth + j) * SB);
+#pragma unroll
+            for (int i = 0; i < G; ++i) fetch(j0 + i, src + (kDepth + j0 + i) * SB);
         }
         src += kDepth * SB;
     }
@@ -422,10 +440,10 @@ __global__ __launch_bounds__(kWG) void slice_scatter_kernel(const uint64_t *__re
     }
 }
 
-template <int W, int VT, int BC>
+template <int W, int VT, int BC, int G>
 hipError_t launch_slices(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
                          hipStream_t s) {
-    hipLaunchKernelGGL((slice_spmv_kernel<W, VT, BC>), dim3((wk.nwg + 7) / 8 * 8 * x.n), dim3(kSliceNT),
+    hipLaunchKernelGGL((slice_spmv_kernel<W, VT, BC, G>), dim3((wk.nwg + 7) / 8 * 8 * x.n), dim3(kSliceNT),
                        slice_lds_bytes(p, BC), s, p.R, p.nseg, tm.wbase, wk.wl, wk.order, wk.tiles, tm.tdata, x, wk.nwg,
                        part);
     return hipGetLastError();
@@ -434,9 +452,19 @@ hipError_t launch_slices(const TilePlan &p, const TiledMatrix &tm, const TileWor
 template <int VT>
 hipError_t launch_slices_vt(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
                             uint32_t BC, hipStream_t s) {
-    if (BC == 4 && p.W == 512) return launch_slices<512, VT, 4>(p, tm, wk, x, part, s);
-    if (BC == 4 && p.W == 1024) return launch_slices<1024, VT, 4>(p, tm, wk, x, part, s);
-    if (BC == 8 && p.W == 512) return launch_slices<512, VT, 8>(p, tm, wk, x, part, s);
+    if (BC == 4 && p.W == 1024) {
+        switch (p.group) {
+            case 1: return launch_slices<1024, VT, 4, 1>(p, tm, wk, x, part, s);
+            case 2: return launch_slices<1024, VT, 4, 2>(p, tm, wk, x, part, s);
+            case 4: return launch_slices<1024, VT, 4, 4>(p, tm, wk, x, part, s);
+        }
+    } else if (BC == 4 && p.W == 512) {
+        if (p.group == 1) return launch_slices<512, VT, 4, 1>(p, tm, wk, x, part, s);
+        if (p.group == 2) return launch_slices<512, VT, 4, 2>(p, tm, wk, x, part, s);
+    } else if (BC == 8 && p.W == 512) {
+        if (p.group == 1) return launch_slices<512, VT, 8, 1>(p, tm, wk, x, part, s);
+        if (p.group == 2) return launch_slices<512, VT, 8, 2>(p, tm, wk, x, part, s);
+    }
     return hipErrorInvalidValue;
 }
 
@@ -448,6 +476,30 @@ size_t slice_lds_bytes(const TilePlan &p, uint32_t BC) { return (2 * ((size_t)p.
 // up to 1024 rows: with 2048 one is left, and the block streams win.
 bool slices_possible(const TilePlan &p) { return p.quad && p.R <= (p.W == 512 ? kSliceMaxR / 2 : kSliceMaxR) && p.ntiles > 0; }
 
+// A stream's part of a tile is padded to whole groups of steps: up to four
+// (two of 512 columns, whose x of 8 right-hand sides takes the registers of
+// four), as long as that adds at most an eighth.  us per iteration in single
+// steps / pairs / fours, 8 steps in flight: 16 slots of 4 over 683 M entries
+// 4242 / 3728 / 3600; 13 slots of 8 over 135 M, about 5 steps per part,
+// 935 / 870 (+9% padding) / 1262 (+28%).
+bool slice_prefix(uint32_t W, std::vector<uint32_t> *w, uint64_t *steps, uint32_t *group) {
+    w->back() = 0;  // becomes the end
+    uint64_t sum[3] = {};
+    for (uint32_t n : *w)
+        for (uint32_t i = 0; i < 3; ++i) sum[i] += (n + (1u << i) - 1) >> i << i;
+    uint32_t i = W == 512 ? 1u : 2u;
+    while (i && sum[i] * 8 > sum[0] * 9) --i;
+    *group = 1u << i;
+    uint64_t run = 0;
+    for (uint32_t &v : *w) {
+        const uint32_t n = (v + (1u << i) - 1) >> i << i;
+        v = (uint32_t)run;
+        run += n;
+    }
+    *steps = run;
+    return run < 0xffffff00ull;
+}
+
 size_t slice_stream_count(const TilePlan &p) { return (size_t)p.nblk * kStreams * p.nseg; }
 
 // Slices unless they store over a quarter more entries than the quads (a few
@@ -456,10 +508,10 @@ size_t slice_stream_count(const TilePlan &p) { return (size_t)p.nblk * kStreams 
 // block stream may hold part of a tile).  Within the rule they were the
 // faster on every matrix tried; us per iteration of 8 slots in 16-bit
 // values, 4 / 8 right-hand sides per pass, block streams -> slices:
-//   20000 x 2000, 200 a row, uniform     73 -> 43 /  53 ->  40
-//   300000 x 300000, 60 a row, a band   151 -> 112 / 138 ->  88
-//   100000 x 100000, 200 a row, uniform 239 -> 230 / 263 -> 243
-//   200000 x 200000, 40 a row, uniform  556 -> 398 / 808 -> 405
+//   20000 x 2000, 200 a row, uniform     73 ->  34 /  53 ->  39
+//   300000 x 300000, 60 a row, a band   151 ->  91 / 138 ->  91
+//   100000 x 100000, 200 a row, uniform 239 -> 217 / 263 -> 234
+//   200000 x 200000, 40 a row, uniform  556 -> 400 / 808 -> 403
 bool slices_suit(const TilePlan &quads, uint64_t steps, uint32_t most) {
     const uint64_t per_run = std::max<uint64_t>(1, steps / 2048);
     return steps * 64 * 4 <= (quads.cap - 8) * 5 && (most <= 256 || most <= per_run);

@@ -85,7 +85,7 @@ struct ChunkedTiles {
         }
         P.cap = run + 8;  // as one build: a multiple of 8, at least one group
         uint64_t steps = 0;
-        slices = slices && slice_prefix(&wbase, &steps) && slices_suit(P, steps, most);
+        slices = slices && slice_prefix(P.W, &wbase, &steps, &P.group) && slices_suit(P, steps, most);
         if (slices) {
             P.slices = true;
             P.steps = steps;

@@ -852,9 +852,7 @@ static int merge_call(const char *what, const uint64_t *rowptr, const uint32_t *
     MergePlan p = merge_plan(rows, nnz, secsize);
     const size_t need = merge_partition_bytes(p) + merge_scratch_bytes(p);
     ARGCHK(ws && ws_bytes >= need, "%s: workspace of %zu bytes needed (mlem_merge_workspace_bytes)", what, need);
-    HIPCHK(launch_merge_partition(p, rowptr, ws, S(stream)));
-    HIPCHK(launch_merge_spmv(p, ws, static_cast<char *>(ws) + merge_partition_bytes(p), rowptr, col, val, x, epi, ea,
-                             S(stream)));
+    HIPCHK(launch_merge_once(p, ws, rowptr, col, val, x, epi, ea, S(stream)));
     return MLEM_OK;
 }
 

@@ -49,6 +49,10 @@ hipError_t launch_merge_partition(const MergePlan &p, const uint64_t *rowptr, vo
 hipError_t launch_merge_spmv(const MergePlan &p, const void *partition, void *scratch, const uint64_t *rowptr,
                              const uint32_t *col, const float *val, const float *x, Epi epi, const EpiArgs &ea,
                              hipStream_t s);
+// Partition and product in one call, for a matrix seen once: ws holds
+// merge_partition_bytes(p) + merge_scratch_bytes(p).
+hipError_t launch_merge_once(const MergePlan &p, void *ws, const uint64_t *rowptr, const uint32_t *col,
+                             const float *val, const float *x, Epi epi, const EpiArgs &ea, hipStream_t s);
 
 bool valid_lanes(uint32_t lanes);
 // lanes 0: chosen from the mean row length (launch_scatter: or the windowed

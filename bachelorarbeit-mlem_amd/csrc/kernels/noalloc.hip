@@ -62,9 +62,7 @@ int mlem_fp_merge_noalloc(const uint64_t *rowptr, const uint32_t *col, const flo
     if (int st = scratch_address(&ws)) return st;
     EpiArgs ea{};
     ea.out = fwproj;
-    HIPCHK(launch_merge_partition(p, rowptr, ws, S(stream)));
-    HIPCHK(launch_merge_spmv(p, ws, static_cast<char *>(ws) + merge_partition_bytes(p), rowptr, col, val, f,
-                             EPI_PLAIN, ea, S(stream)));
+    HIPCHK(launch_merge_once(p, ws, rowptr, col, val, f, EPI_PLAIN, ea, S(stream)));
     return MLEM_OK;
 }
 

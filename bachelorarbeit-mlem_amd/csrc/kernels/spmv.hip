@@ -256,35 +256,81 @@ __global__ void merge_partition_kernel(const uint64_t *__restrict__ rowptr, uint
     tile_nz[t] = d - lo;
 }
 
-template <int EPI>
+// The same split point found by a wave: 64 probes per round (three rounds of
+// loads for 41,000 rows where one work-item takes sixteen).  Every lane gets
+// it.
+__device__ __forceinline__ uint32_t merge_split_wave(const uint64_t *__restrict__ rowptr, uint32_t rows, uint64_t nnz,
+                                                     uint64_t d, uint32_t lane) {
+    uint64_t lo = d > nnz ? d - nnz : 0, hi = d < rows ? d : rows;
+    while (lo < hi) {  // ends: the range shrinks to less than a 64th, at least by one
+        const uint64_t step = (hi - lo + 63) / 64, at = lo + lane * step;
+        const bool past = at >= hi || rowptr[at + 1] + at >= d;
+        const uint64_t m = __ballot(past);
+        const uint32_t f = m ? (uint32_t)__builtin_ctzll(m) : 64u;  // the first probe at or past the split
+        hi = f == 64u ? hi : (lo + f * step < hi ? lo + f * step : hi);
+        lo = f == 0u ? lo : lo + (f - 1) * step + 1;
+    }
+    return (uint32_t)lo;
+}
+
+// SEARCH: the partition does not exist yet.  Two waves find the tile's two
+// split points and the tile stores its own for the fix-up.
+template <int EPI, bool SEARCH>
 __global__ __launch_bounds__(kWG) void merge_spmv_kernel(const uint64_t *__restrict__ rowptr,
                                                          const uint32_t *__restrict__ col,
                                                          const float *__restrict__ val, const float *__restrict__ x,
-                                                         uint32_t S, const uint32_t *__restrict__ tile_row,
-                                                         const uint64_t *__restrict__ tile_nz,
-                                                         float *__restrict__ tile_carry,
+                                                         uint32_t S, uint32_t rows, uint64_t nnz, uint32_t *tile_row,
+                                                         uint64_t *tile_nz, float *__restrict__ tile_carry,
                                                          float *__restrict__ tile_head, EpiArgs ea) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     __shared__ float s_wv[kWG / 64];
     __shared__ int s_wf[kWG / 64];
+    __shared__ uint32_t s_row[2];
 
     const uint32_t t = blockIdx.x;
     const uint32_t tid = threadIdx.x;
-    const uint32_t i0 = tile_row[t], i1 = tile_row[t + 1];
-    const uint64_t j0 = tile_nz[t], j1 = tile_nz[t + 1];
+    uint32_t i0, i1;
+    uint64_t j0, j1;
+    if constexpr (SEARCH) {
+        const uint64_t L = (uint64_t)rows + nnz, T = (uint64_t)kWG * S;
+        const uint64_t d0 = t * T, d1 = d0 + T < L ? d0 + T : L;  // t * T < L
+        const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+        if (w < 2) {
+            const uint32_t r = merge_split_wave(rowptr, rows, nnz, w ? d1 : d0, tid & 63u);
+            if ((tid & 63u) == 0) s_row[w] = r;
+        }
+        __syncthreads();
+        i0 = s_row[0];
+        i1 = s_row[1];
+        j0 = d0 - i0;
+        j1 = d1 - i1;
+        if (tid < 2 && (tid == 0 || t + 1 == gridDim.x)) {
+            tile_row[t + tid] = tid ? i1 : i0;
+            tile_nz[t + tid] = tid ? j1 : j0;
+        }
+    } else {
+        i0 = tile_row[t];
+        i1 = tile_row[t + 1];
+        j0 = tile_nz[t];
+        j1 = tile_nz[t + 1];
+    }
     const uint32_t nr = i1 - i0;              // row ends in this tile
     const uint32_t nz = (uint32_t)(j1 - j0);  // nonzeros in this tile
     const uint32_t h = (uint32_t)(j0 & 3u);   // s_val[h + jl] holds nonzero j0 + jl
     float *s_val = smem;
     uint32_t *s_end = reinterpret_cast<uint32_t *>(smem + ((h + nz + 3u) & ~3u));
 
-    // Stage products val*x[col] with aligned 16-byte loads (partial quads at
-    // the tile edges element by element) and the local row ends.
+    // Stage products val*x[col] with aligned 16-byte loads and the local row
+    // ends.  The tile's edge quads: on its own (SEARCH, a small matrix whose
+    // tile is one chain of latencies) loaded whole, a neighbour's entries in
+    // them unused; else element by element, which costs the chain another
+    // round trip but was the faster on large matrices (mid-sized scanner,
+    // 87,811 tiles, FP + BP: 1046 against 1110 us; 2D ring 36.7 against 35.0).
     const uint64_t ja = j0 - h;
     const uint32_t nq = (h + nz + 3u) >> 2;
     for (uint32_t q = tid; q < nq; q += kWG) {
         const uint64_t jq = ja + 4ull * q;
-        if (jq >= j0 && jq + 4 <= j1) {
+        if (SEARCH ? jq + 4 <= nnz : jq >= j0 && jq + 4 <= j1) {
             const u32x4 c = ldnt(reinterpret_cast<const u32x4 *>(col + jq));
             const f32x4 v = ldnt(reinterpret_cast<const f32x4 *>(val + jq));
             f32x4 p;
@@ -707,14 +753,18 @@ __global__ __launch_bounds__(kWG) void loglik_kernel(const uint64_t *__restrict_
 inline uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)((n + per - 1) / per); }
 
 template <int EPI>
-hipError_t launch_merge_epi(const MergePlan &p, const uint32_t *tile_row, const uint64_t *tile_nz, float *carry,
+hipError_t launch_merge_epi(const MergePlan &p, bool search, uint32_t *tile_row, uint64_t *tile_nz, float *carry,
                             float *head, const uint64_t *rowptr, const uint32_t *col, const float *val,
                             const float *x, const EpiArgs &ea, hipStream_t s) {
     const size_t lds = (p.tile_items + 8) * sizeof(float);
-    hipLaunchKernelGGL(merge_spmv_kernel<EPI>, dim3(p.ntiles), dim3(kWG), lds, s, rowptr, col, val, x, p.secsize,
-                       tile_row, tile_nz, carry, head, ea);
+    if (search)
+        hipLaunchKernelGGL((merge_spmv_kernel<EPI, true>), dim3(p.ntiles), dim3(kWG), lds, s, rowptr, col, val, x,
+                           p.secsize, p.rows, p.nnz, tile_row, tile_nz, carry, head, ea);
+    else
+        hipLaunchKernelGGL((merge_spmv_kernel<EPI, false>), dim3(p.ntiles), dim3(kWG), lds, s, rowptr, col, val, x,
+                           p.secsize, p.rows, p.nnz, tile_row, tile_nz, carry, head, ea);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || p.ntiles == 1) return e;  // one tile: no row spans two
     hipLaunchKernelGGL(merge_fixup_kernel<EPI>, dim3(blocks_for(p.ntiles, kWG)), dim3(kWG), 0, s, rowptr, p.ntiles,
                        tile_row, tile_nz, carry, head, ea);
     return hipGetLastError();
@@ -779,20 +829,46 @@ hipError_t launch_merge_partition(const MergePlan &p, const uint64_t *rowptr, vo
     return hipGetLastError();
 }
 
+namespace {
+hipError_t merge_launch(const MergePlan &p, bool search, void *partition, void *scratch, const uint64_t *rowptr,
+                        const uint32_t *col, const float *val, const float *x, Epi epi, const EpiArgs &ea,
+                        hipStream_t s) {
+    uint32_t *tile_row = static_cast<uint32_t *>(partition);
+    uint64_t *tile_nz = reinterpret_cast<uint64_t *>(static_cast<char *>(partition) +
+                                                     align256(sizeof(uint32_t) * ((size_t)p.ntiles + 1)));
+    float *carry = static_cast<float *>(scratch);
+    float *head = reinterpret_cast<float *>(static_cast<char *>(scratch) + align256(sizeof(float) * ((size_t)p.ntiles + 1)));
+    switch (epi) {
+        case EPI_PLAIN: return launch_merge_epi<EPI_PLAIN>(p, search, tile_row, tile_nz, carry, head, rowptr, col, val, x, ea, s);
+        case EPI_RATIO: return launch_merge_epi<EPI_RATIO>(p, search, tile_row, tile_nz, carry, head, rowptr, col, val, x, ea, s);
+        default: return launch_merge_epi<EPI_UPDATE>(p, search, tile_row, tile_nz, carry, head, rowptr, col, val, x, ea, s);
+    }
+}
+}  // namespace
+
 hipError_t launch_merge_spmv(const MergePlan &p, const void *partition, void *scratch, const uint64_t *rowptr,
                              const uint32_t *col, const float *val, const float *x, Epi epi, const EpiArgs &ea,
                              hipStream_t s) {
     if (p.rows == 0) return hipSuccess;
-    const uint32_t *tile_row = static_cast<const uint32_t *>(partition);
-    const uint64_t *tile_nz = reinterpret_cast<const uint64_t *>(
-        static_cast<const char *>(partition) + align256(sizeof(uint32_t) * ((size_t)p.ntiles + 1)));
-    float *carry = static_cast<float *>(scratch);
-    float *head = reinterpret_cast<float *>(static_cast<char *>(scratch) + align256(sizeof(float) * ((size_t)p.ntiles + 1)));
-    switch (epi) {
-        case EPI_PLAIN: return launch_merge_epi<EPI_PLAIN>(p, tile_row, tile_nz, carry, head, rowptr, col, val, x, ea, s);
-        case EPI_RATIO: return launch_merge_epi<EPI_RATIO>(p, tile_row, tile_nz, carry, head, rowptr, col, val, x, ea, s);
-        default: return launch_merge_epi<EPI_UPDATE>(p, tile_row, tile_nz, carry, head, rowptr, col, val, x, ea, s);
+    return merge_launch(p, false, const_cast<void *>(partition), scratch, rowptr, col, val, x, epi, ea, s);
+}
+
+// A small product is a chain of launches: the partition's own launch and its
+// binary search (one work-item per tile, a memory latency per step) took as
+// long as the search by waves inside the product takes for thousands of
+// tiles.  FP + ratio + BP + update, us, partition launch / search: 2D ring
+// (987 tiles) 36.7 / 30.5, 4262 tiles 74.0 / 69.1, 7804 tiles 116.7 / 113.0,
+// 24497 tiles 301 / 319.
+constexpr uint32_t kSearchTiles = 8192;
+hipError_t launch_merge_once(const MergePlan &p, void *ws, const uint64_t *rowptr, const uint32_t *col,
+                             const float *val, const float *x, Epi epi, const EpiArgs &ea, hipStream_t s) {
+    if (p.rows == 0) return hipSuccess;
+    const bool search = p.ntiles <= kSearchTiles;
+    if (!search) {
+        const hipError_t e = launch_merge_partition(p, rowptr, ws, s);
+        if (e != hipSuccess) return e;
     }
+    return merge_launch(p, search, ws, static_cast<char *>(ws) + merge_partition_bytes(p), rowptr, col, val, x, epi, ea, s);
 }
 
 // Rows per workgroup of the windowed scatter: whole rounds of a workgroup per

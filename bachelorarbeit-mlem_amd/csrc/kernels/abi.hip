@@ -241,7 +241,7 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     }
     if (m->tiles_only)
         return set_err(MLEM_ERR_UNSUPPORTED, "a tiles-only matrix holds tiles of width %u and %u rows (values %u) only",
-                       m->tile_W, m->tile_R, m->tile_vt);
+                       m->tile_W, m->tile_R[which], m->tile_vt);
     auto ref = m->tile_refused.find(key);
     if (ref != m->tile_refused.end()) {
         *flags = ref->second;
@@ -451,6 +451,7 @@ int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev *
     w->view.ntl = L.ntl;
     for (size_t b = 0; b + 1 < L.wl_first.size(); ++b)
         w->view.max_runs = std::max(w->view.max_runs, L.wl_first[b + 1] - L.wl_first[b]);
+    w->view.direct = p.slices && w->view.max_runs == 1 && L.nwg == p.nblk;
     w->view.wl = reinterpret_cast<const uint4 *>(base);
     w->view.tiles = reinterpret_cast<const uint4 *>(base + o_tl);
     w->view.wl_first = reinterpret_cast<const uint32_t *>(base + o_first);
@@ -461,7 +462,8 @@ int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev *
 }
 
 // The blocked path for one side (0: A, 1: A^T): tiles (built on first use),
-// a work list of about `groups` runs (0: the default) and the partial-sum
+// a work list of about `groups` runs (0: the default, one run per row block
+// where slices_direct says so) and the partial-sum
 // buffer for BC right-hand sides.  MLEM_ERR_UNSUPPORTED when the matrix or
 // the LDS does not allow the shape.
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
@@ -476,7 +478,8 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
     int dev = 0, lds_max = 65536;
     if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-    const uint32_t target = groups ? groups : default_tile_groups(m->nnz, vt, BC);
+    uint32_t target = groups ? groups : default_tile_groups(m->nnz, vt, BC);
+    if (!groups && t->plan.slices && slices_direct(t->plan.cols, W, R, t->plan.rows, m->nnz, BC)) target = 1;
     const TileWorkDev *w = nullptr;
     if (int st = get_tile_work(m, const_cast<Tiled *>(t), target, &w)) return st;
     if (tiled_lds_bytes(t->plan, w->view.span, BC) + 4096 > (size_t)lds_max)
@@ -519,9 +522,10 @@ static uint32_t device_cus() {
 //   f32    u =  44 (16 slots)  627 / 617    16-bit    513 / 512
 //   f32    u =  64 (8 slots)   588 / 564    16-bit    453 / 434
 //   f32    u = 326 (8 slots)  2767 / 2492   16-bit   2098 / 1898
-// 2048 rows from 48 units.  512 rows lose at every size (u = 0.9: 39 and
-// 37).  Eight right-hand sides of 2048 rows leave one workgroup per CU
-// (u = 163 at 8 runs per CU: 2798 / 4153).
+// 2048 rows from 48 units.  512 rows (u = 0.9: 39 and 37) where every row
+// block is then one run and needs no partial sums (slices_direct).  Eight
+// right-hand sides of 2048 rows leave one workgroup per CU (u = 163 at 8
+// runs per CU: 2798 / 4153).
 uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
     const uint32_t cus = device_cus();
     if (BC != 1) return (BC == 4 ? 4u : 8u) * cus;
@@ -529,8 +533,10 @@ uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
     return (u >= 2 && u < (vt == VAL_F32 ? 40u : 24u) ? 12u : 24u) * cus;
 }
 
-uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC) {
+uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC) {
     const uint64_t target = groups ? groups : (BC == 1 ? 24u : BC == 4 ? 4u : 8u) * (uint64_t)device_cus();
+    const uint32_t W = BC == 8 ? 512u : 1024u;
+    if (BC != 1 && !groups && slices_direct(cols, W, 512, rows, nnz, BC)) return 512u;
     if (BC == 4) return nnz < target * 48 * kTileUnit ? 1024u : 2048u;
     if (nnz < target * 2 * kTileUnit) return 512u;
     if (BC != 1) return 1024u;
@@ -547,7 +553,7 @@ int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t sec
     *work = nullptr;
     if (o.tile_width != 1) {
         const uint32_t W = o.tile_width == 0 ? 1024u : o.tile_width;
-        const uint32_t R = o.tile_rows == 0 ? default_tile_rows(m->nnz, o.tile_groups, o.values, 1) : o.tile_rows;
+        const uint32_t R = o.tile_rows == 0 ? default_tile_rows(m->rows, m->cols, m->nnz, o.tile_groups, o.values, 1) : o.tile_rows;
         const int st = setup_tiled(m, which, W, R, o.values, 1, o.tile_groups, tiled, work, part);
         if (st == MLEM_OK || m->tiles_only) return st;
         // Automatic width with f32 values: a matrix the tiles do not suit, or
@@ -1323,12 +1329,12 @@ int mlem_recon_create(const mlem_matrix *mc, const int32_t *g, const float *sens
         ARGCHK(o.spmv == 0 && o.using_trans == 0 && o.bp_spmv <= 1,
                "mlem_recon_create: a tiles-only matrix takes merge-based FP and BP on A^T");
         ARGCHK(m->tile_bc == 1, "mlem_recon_create: the matrix holds the tiles of batches of %u per pass", m->tile_bc);
-        ARGCHK((o.tile_width == 0 || o.tile_width == m->tile_W) && (o.tile_rows == 0 || o.tile_rows == m->tile_R) &&
+        ARGCHK((o.tile_width == 0 || o.tile_width == m->tile_W) && (o.tile_rows == 0 || o.tile_rows == m->tile_R[0]) &&
                    (o.values == 0 || o.values == m->tile_vt),
                "mlem_recon_create: the matrix holds tiles of width %u and %u rows with values %u", m->tile_W,
-               m->tile_R, m->tile_vt);
+               m->tile_R[0], m->tile_vt);
         o.tile_width = m->tile_W;
-        o.tile_rows = m->tile_R;
+        o.tile_rows = m->tile_R[0];
         o.values = m->tile_vt;
     }
     HIPCHK(hipSetDevice(m->device));

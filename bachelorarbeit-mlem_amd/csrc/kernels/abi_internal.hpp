@@ -182,10 +182,10 @@ struct mlem_matrix {
     mlem::abi::DevBuf rowptrT, colT, valT;
     bool has_T = false;
     // Tiles only (mlem_matrix_create_tiled): no CSR copies on the device, the
-    // tiles of A and A^T (width tile_W, tile_R rows, f32) and the
+    // tiles of A and A^T (width tile_W, tile_R[0] and [1] rows) and the
     // sensitivity taken while they were built.
     bool tiles_only = false;
-    uint32_t tile_W = 0, tile_R = 0, tile_vt = 0, tile_bc = 1;  // tile_bc: right-hand sides per pass
+    uint32_t tile_W = 0, tile_R[2] = {}, tile_vt = 0, tile_bc = 1;  // tile_bc: right-hand sides per pass
     mlem::abi::DevBuf sens32, sens64;
     // Row order for the batched (quad) tiles: row_order[i] = place of row i
     // of A (mlem_matrix_set_row_order); has_order false: A's own order.
@@ -306,7 +306,7 @@ int sens_on_device(const mlem_matrix *m, float *s32, double *s64_or_null, hipStr
 // right-hand sides and `vt` values when none are asked for, on the current
 // device (groups 0: the default runs).
 uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC);
-uint32_t default_tile_rows(uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC);
+uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC);
 // Batch slots without waiting on the host (the serving loop): the set
 // copies g (rows) and f0 (cols) in and marks the slot active, allocating its
 // pass if that is the first slot set in it (*allocated = bytes allocated,

@@ -30,10 +30,8 @@ int enqueue_batch_iteration(mlem_batch *b, const std::vector<uint8_t> &passes) {
         fe.n = bx.n = be.n = fx.n;
         if (!fx.n) break;
         float *part = b->part.as<float>();
-        HIPCHK(launch_tiled_partials(b->tfp->plan, b->tfp->view, b->wfp->view, fx, part, BC, b->nt, s));
-        HIPCHK(launch_tiled_reduce(b->tfp->plan, b->tfp->view, b->wfp->view, part, BC, EPI_RATIO, fe, s));
-        HIPCHK(launch_tiled_partials(b->tbp->plan, b->tbp->view, b->wbp->view, bx, part, BC, b->nt, s));
-        HIPCHK(launch_tiled_reduce(b->tbp->plan, b->tbp->view, b->wbp->view, part, BC, EPI_UPDATE, be, s));
+        HIPCHK(launch_tiled_spmv(b->tfp->plan, b->tfp->view, b->wfp->view, fx, part, BC, b->nt, EPI_RATIO, fe, s));
+        HIPCHK(launch_tiled_spmv(b->tbp->plan, b->tbp->view, b->wbp->view, bx, part, BC, b->nt, EPI_UPDATE, be, s));
     }
     return MLEM_OK;
 }
@@ -119,8 +117,10 @@ int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to) {
 }
 
 int batch_alloc_part(mlem_batch *b, uint32_t passes) {
-    const uint64_t one = std::max<uint64_t>(4, std::max(tiled_part_bytes(b->tfp->plan, b->wfp->view.nwg, b->BC),
-                                                        tiled_part_bytes(b->tbp->plan, b->wbp->view.nwg, b->BC)));
+    auto bytes = [&](const Tiled *t, const TileWorkDev *w) {
+        return w->view.direct ? 0 : tiled_part_bytes(t->plan, w->view.nwg, b->BC);
+    };
+    const uint64_t one = std::max<uint64_t>(4, std::max(bytes(b->tfp, b->wfp), bytes(b->tbp, b->wbp)));
     // One right-hand side per pass: the blocked kernel takes one pass per launch.
     uint32_t n = b->BC == 1 ? 1u : std::max(1u, std::min(passes, kMaxPasses));
     for (;; n = (n + 1) / 2) {
@@ -219,9 +219,8 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
         ea.out = y;
         for (int rep = 0; rep < 4; ++rep) {
             if (rep == 1 && hipEventRecord(e0, s) != hipSuccess) return hipErrorUnknown;
-            hipError_t e = launch_tiled_partials(t->plan, t->view, w->view, one_pass(x), part.as<float>(), BC, nt, s);
-            if (e == hipSuccess)
-                e = launch_tiled_reduce(t->plan, t->view, w->view, part.as<float>(), BC, EPI_PLAIN, one_pass(ea), s);
+            const hipError_t e = launch_tiled_spmv(t->plan, t->view, w->view, one_pass(x), part.as<float>(), BC, nt,
+                                                   EPI_PLAIN, one_pass(ea), s);
             if (e != hipSuccess) return e;
         }
         hipError_t e = hipEventRecord(e1, s);
@@ -310,23 +309,27 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     ARGCHK(m->has_T || m->tiles_only, "mlem_batch_create: the transpose must be resident (upload it or build it)");
     if (m->tiles_only) {
         ARGCHK(BC == m->tile_bc && (o.tile_width == 0 || o.tile_width == m->tile_W) &&
-                   (o.tile_rows == 0 || o.tile_rows == m->tile_R) && (o.values == 0 || o.values == m->tile_vt),
+                   (o.tile_rows == 0 || o.tile_rows == m->tile_R[0] || o.tile_rows == m->tile_R[1]) &&
+                   (o.values == 0 || o.values == m->tile_vt),
                "mlem_batch_create: the matrix holds tiles of width %u and %u rows with values %u for %u per pass",
-               m->tile_W, m->tile_R, m->tile_vt, m->tile_bc);
+               m->tile_W, m->tile_R[0], m->tile_vt, m->tile_bc);
         o.tile_width = m->tile_W;
-        o.tile_rows = m->tile_R;
         o.values = m->tile_vt;
     }
-    // Defaults: 1024 x 2048 (1024 up to mid sizes) for one per pass, 1024 x 1024 for 4 (3.28x the
-    // single FP32 path at C2 against 3.17x for 512 x 2048), 512 x 1024 for 8;
-    // 512 rows for small matrices (default_tile_rows).
+    // Widths: 1024, 512 for 8 per pass (whose x of 1024 columns would leave
+    // one workgroup per CU); rows: default_tile_rows, for FP and BP by itself.
     const uint32_t W = o.tile_width ? o.tile_width : (BC == 8 ? 512u : 1024u);
     ARGCHK(valid_tile_config(W, BC), "mlem_batch_create: no blocked kernel for width %u with %u per pass", W, BC);
     ARGCHK(o.tile_rows == 0 || valid_tile_rows(o.tile_rows),
            "mlem_batch_create: tile_rows must be 512 ... 16384 (a power of two)");
     ARGCHK(valid_stream_threads(o.tile_threads), "mlem_batch_create: tile_threads must be 0, 128, 256 or 512");
     HIPCHK(hipSetDevice(m->device));
-    const uint32_t R = o.tile_rows ? o.tile_rows : default_tile_rows(m->nnz, o.tile_groups, o.values, BC);
+    auto side_rows = [&](int which) {
+        if (m->tiles_only) return m->tile_R[which];
+        if (o.tile_rows) return o.tile_rows;
+        return which ? default_tile_rows(m->cols, m->rows, m->nnz, o.tile_groups, o.values, BC)
+                     : default_tile_rows(m->rows, m->cols, m->nnz, o.tile_groups, o.values, BC);
+    };
     auto b = std::make_unique<mlem_batch>();
     b->m = m;
     b->slots = slots;
@@ -337,9 +340,8 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     b->rows_x = (m->rows + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
     b->cols_x = (m->cols + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
     HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-    const uint32_t groups = o.tile_groups ? o.tile_groups : default_tile_groups(m->nnz, o.values, BC);
-    if (int st = setup_tiled(m, 0, W, R, o.values, BC, groups, &b->tfp, &b->wfp, nullptr)) return st;
-    if (int st = setup_tiled(m, 1, W, R, o.values, BC, groups, &b->tbp, &b->wbp, nullptr)) return st;
+    if (int st = setup_tiled(m, 0, W, side_rows(0), o.values, BC, o.tile_groups, &b->tfp, &b->wfp, nullptr)) return st;
+    if (int st = setup_tiled(m, 1, W, side_rows(1), o.values, BC, o.tile_groups, &b->tbp, &b->wbp, nullptr)) return st;
     if (int st = batch_alloc_part(b.get(), b->passes)) return st;
     if (b->tfp->ordered != b->tbp->ordered)  // a row order set from another thread between the two builds
         return set_err(MLEM_ERR_INVALID_ARGUMENT, "mlem_batch_create: the row order changed while the tiles were built");

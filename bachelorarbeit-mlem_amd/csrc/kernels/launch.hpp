@@ -169,6 +169,7 @@ struct TileWorkList {
 struct TileWork {
     uint32_t span = 1, nwg = 0, ntl = 0;
     uint32_t max_runs = 0;  // the most runs of one row block
+    bool direct = false;    // row slices, one run per row block: no partial sums (launch_tiled_spmv)
     const uint4 *wl = nullptr;
     const uint4 *tiles = nullptr;
     const uint32_t *wl_first = nullptr;
@@ -254,6 +255,9 @@ inline PassEpi one_pass(const EpiArgs &ea) {
 }
 hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x,
                                  float *part, uint32_t BC, uint32_t nt, hipStream_t s);
+// Both; in one launch, without `part`, where every row block is one run.
+hipError_t launch_tiled_spmv(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
+                             uint32_t BC, uint32_t nt, Epi epi, const PassEpi &ea, hipStream_t s);
 bool valid_stream_threads(uint32_t nt);
 hipError_t launch_tiled_reduce(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const float *part,
                                uint32_t BC, Epi epi, const PassEpi &ea, hipStream_t s);
@@ -273,6 +277,8 @@ hipError_t launch_slice_count(const TilePlan &p, const uint32_t *cnt, uint32_t *
 // element more) as first steps in place, their sum and the steps taken
 // together; false when they are too many for the layout.
 bool slice_prefix(uint32_t W, std::vector<uint32_t> *w, uint64_t *steps, uint32_t *group);
+// One run per row block (launch_tiled_spmv then needs no partial sums).
+bool slices_direct(uint32_t cols, uint32_t W, uint32_t R, uint64_t rows, uint64_t nnz, uint32_t BC);
 // Whether slices with `steps` steps beat the quad tiles of plan `quads`.
 bool slices_suit(const TilePlan &quads, uint64_t steps, uint32_t most);
 size_t slice_data_bytes(const TilePlan &p);                    // wbase and the steps (p.steps set)
@@ -285,8 +291,14 @@ hipError_t launch_slice_scatter(const TilePlan &p, const uint64_t *rowptr, const
                                 const uint16_t *qval, const uint32_t *rowloc, const uint32_t *wbase, uint8_t *tdata,
                                 hipStream_t s);
 TileWorkList slice_work_list(const TilePlan &p, const uint32_t *wbase, uint32_t target_wgs);
-hipError_t launch_slice_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x,
-                                 float *part, uint32_t BC, hipStream_t s);
+// direct 0: partial sums into part; else the epilogue of whole row blocks.
+struct SliceEpi {
+    uint32_t direct, epi, rows;
+    const float *scale;
+    PassEpi pe;
+};
+hipError_t launch_slice_spmv(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
+                             uint32_t BC, const SliceEpi &se, hipStream_t s);
 // The scales (p.unit_scale: 1) and codes of a CSR's rows as the tiles store
 // them; *bad bit 8: a negative value for uf16.
 hipError_t launch_row_codes(const TilePlan &p, const uint64_t *rowptr, const float *val, float *scale, uint16_t *q,

@@ -110,19 +110,36 @@ __device__ __forceinline__ float quad_getf(float v) {
     return __uint_as_float(quad_get<CTRL>(__float_as_uint(v)));
 }
 
+// The epilogue of the rows r0 .. r0 + R - 1 from their sums: what
+// blocked_reduce_kernel makes of one run's partial sums.
+template <int EPI, int BC>
+__device__ __forceinline__ void finish_rows(uint32_t r0, uint32_t R, const float *acc, const SliceEpi &se,
+                                            const EpiArgs &ea) {
+    const uint32_t nr = min(R, se.rows - r0);
+    for (uint32_t i = threadIdx.x; i < nr; i += kSliceNT) {
+        const ReduceIn<BC> in = reduce_load<EPI, BC>(r0 + i, se.scale, ea);
+        float y[BC];
+#pragma unroll
+        for (int q = 0; q < BC; ++q) y[q] = acc[i * BC + q];
+        reduce_epilogue<EPI, BC>(r0 + i, y, in, se.scale != nullptr, ea);
+    }
+}
+
 // wl[run] = {row block, first tile (index into tiles), tiles}; tiles[i].x =
 // segment.  One launch takes several passes of a batch, as
 // stream_spmv_kernel does: workgroups go round the 8 XCDs, so 8 runs of one
 // pass are followed by the same runs of the next, each on its XCD.
-// G steps are taken together, their gathers in flight at once.
-template <int W, int VT, int BC, int G>
+// G steps are taken together, their gathers in flight at once.  DIRECT: whole
+// row blocks and their epilogue instead of partial sums (a variant of its
+// own: as a branch it cost launches that do not take it 1%).
+template <int W, int VT, int BC, int G, bool DIRECT>
 __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32_t nseg,
                                                               const uint32_t *__restrict__ wbase,
                                                               const uint4 *__restrict__ wl,
                                                               const uint32_t *__restrict__ order,
                                                               const uint4 *__restrict__ tiles,
                                                               const uint8_t *__restrict__ tdata, PassX px,
-                                                              uint32_t nwg, float *__restrict__ part) {
+                                                              uint32_t nwg, float *__restrict__ part, SliceEpi se) {
     constexpr uint32_t SB = step_bytes(VT);
     constexpr int kDepth = step_depth(VT, G);
     static_assert(kDepth % G == 0 && 2 * kDepth <= (int)kPadSteps, "whole groups in flight, nothing read past the end");
@@ -148,7 +165,6 @@ __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32
         xs[W * BC + tid] = 0.0f;
         xs[XS + W * BC + tid] = 0.0f;
     }
-    float *pw = part + ((uint64_t)pass * nwg + run) * R * BC;
     // Every wave passes nt + 1 barriers.  Barrier t: x of tile t is staged and
     // tile t - 1 is done, so that its slot may be written.
     if (wv >= kStreams) {
@@ -164,103 +180,111 @@ __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32
             for (int q = 0; q < XP; ++q) slot[st + 64 * kStagers * q] = r[q];
             __syncthreads();
         }
-        __syncthreads();
-        for (uint32_t i = tid; i < R * BC; i += kSliceNT) pw[i] = acc[i];
-        return;
-    }
-    // Lane i: this wave's steps in tile i.
-    const uint64_t wb = ((uint64_t)w.x * kStreams + wv) * nseg + seg;
-    const uint32_t s0 = wbase[wb], s1 = wbase[wb + 1], cnt = s1 - s0;
-    const uint32_t first = __builtin_amdgcn_readfirstlane(s0);
-    const uint32_t total = __builtin_amdgcn_readlane(s1, nt - 1) - first;
-    // The wave's steps, kDepth in flight (past its last step: whatever follows).
-    const uint8_t *src = tdata + (uint64_t)first * SB;
-    uint32_t rw[kDepth];  // 16-bit values: the words; f32: the metas
-    float rv[kDepth];
-    auto fetch = [&](int j, const uint8_t *at) {
-        if constexpr (VT == VAL_F32) {
-            rv[j] = reinterpret_cast<const float *>(at)[lane];
-            rw[j] = reinterpret_cast<const uint16_t *>(at + 256)[lane];
-        } else {
-            rw[j] = reinterpret_cast<const uint32_t *>(at)[lane];
-        }
-    };
-#pragma unroll
-    for (int j = 0; j < kDepth; ++j) fetch(j, src + j * SB);
-
-    const char *xw = reinterpret_cast<const char *>(xs);
-    uint32_t t = 0, left = 0;  // the next tile; this wave's steps left in the current one
-    auto enter = [&]() {
-        __syncthreads();
-        xw = reinterpret_cast<const char *>(xs + (t & 1u) * XS);
-        left = __builtin_amdgcn_readlane(cnt, t);
-        ++t;
-    };
-
-    float a[BC];
-#pragma unroll
-    for (int b = 0; b < BC; ++b) a[b] = 0.0f;
-    for (uint32_t done = 0; done < total;) {
-#pragma unroll
-        for (int j0 = 0; j0 < kDepth; j0 += G) {
-            if (done == total) break;
-            while (left == 0) enter();  // ends: a tile with steps is left
-            f32x4 xv[G][BC / 4];
-            float v[G];
-#pragma unroll
-            for (int i = 0; i < G; ++i) {
-                const float *xg = reinterpret_cast<const float *>(xw + (rw[j0 + i] & 0x7ff0u) * (BC / 4));
-#pragma unroll
-                for (int q = 0; q < BC / 4; ++q) xv[i][q] = *reinterpret_cast<const f32x4 *>(xg + 4 * q);
-                if constexpr (VT == VAL_F32)
-                    v[i] = rv[j0 + i];
-                else
-                    v[i] = word_val<VT>(rw[j0 + i]);
+    } else {
+        // Lane i: this wave's steps in tile i.
+        const uint64_t wb = ((uint64_t)w.x * kStreams + wv) * nseg + seg;
+        const uint32_t s0 = wbase[wb], s1 = wbase[wb + 1], cnt = s1 - s0;
+        const uint32_t first = __builtin_amdgcn_readfirstlane(s0);
+        const uint32_t total = __builtin_amdgcn_readlane(s1, nt - 1) - first;
+        // The wave's steps, kDepth in flight (past its last step: whatever follows).
+        const uint8_t *src = tdata + (uint64_t)first * SB;
+        uint32_t rw[kDepth];  // 16-bit values: the words; f32: the metas
+        float rv[kDepth];
+        auto fetch = [&](int j, const uint8_t *at) {
+            if constexpr (VT == VAL_F32) {
+                rv[j] = reinterpret_cast<const float *>(at)[lane];
+                rw[j] = reinterpret_cast<const uint16_t *>(at + 256)[lane];
+            } else {
+                rw[j] = reinterpret_cast<const uint32_t *>(at)[lane];
             }
-            done += G;
-            left -= G;
+        };
 #pragma unroll
-            for (int i = 0; i < G; ++i) {
-                const uint32_t m = rw[j0 + i];
+        for (int j = 0; j < kDepth; ++j) fetch(j, src + j * SB);
+
+        const char *xw = reinterpret_cast<const char *>(xs);
+        uint32_t t = 0, left = 0;  // the next tile; this wave's steps left in the current one
+        auto enter = [&]() {
+            __syncthreads();
+            xw = reinterpret_cast<const char *>(xs + (t & 1u) * XS);
+            left = __builtin_amdgcn_readlane(cnt, t);
+            ++t;
+        };
+
+        float a[BC];
 #pragma unroll
-                for (int q = 0; q < BC / 4; ++q)
+        for (int b = 0; b < BC; ++b) a[b] = 0.0f;
+        for (uint32_t done = 0; done < total;) {
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) a[4 * q + b] = fmaf(v[i], xv[i][q][b], a[4 * q + b]);
-                if (__builtin_amdgcn_readfirstlane(m) & 0x8000u) {  // the slice ends: its 16 rows
-                    uint32_t row = (m & 15u) << (4u * (lane & 3u));
-                    row |= quad_get<0xB1>(row);
-                    row |= quad_get<0x4E>(row);
-                    // Sums over the row's four work-items, halved between
-                    // neighbours: work-item q keeps BC/4 right-hand sides.
-                    const bool o1 = lane & 1u, o2 = lane & 2u;
-                    float h[BC / 2];
+            for (int j0 = 0; j0 < kDepth; j0 += G) {
+                if (done == total) break;
+                while (left == 0) enter();  // ends: a tile with steps is left
+                f32x4 xv[G][BC / 4];
+                float v[G];
 #pragma unroll
-                    for (int b = 0; b < BC / 2; ++b)
-                        h[b] = (o1 ? a[b + BC / 2] : a[b]) + quad_getf<0xB1>(o1 ? a[b] : a[b + BC / 2]);
-                    float *p = acc + row * BC + (o1 ? BC / 2 : 0) + (o2 ? BC / 4 : 0);
-                    if constexpr (BC == 4) {
-                        *p += (o2 ? h[1] : h[0]) + quad_getf<0x4E>(o2 ? h[0] : h[1]);
-                    } else {
-                        typedef float f32x2 __attribute__((ext_vector_type(2)));
-                        f32x2 o = *reinterpret_cast<f32x2 *>(p);
-                        o.x += (o2 ? h[2] : h[0]) + quad_getf<0x4E>(o2 ? h[0] : h[2]);
-                        o.y += (o2 ? h[3] : h[1]) + quad_getf<0x4E>(o2 ? h[1] : h[3]);
-                        *reinterpret_cast<f32x2 *>(p) = o;
-                    }
+                for (int i = 0; i < G; ++i) {
+                    const float *xg = reinterpret_cast<const float *>(xw + (rw[j0 + i] & 0x7ff0u) * (BC / 4));
 #pragma unroll
-                    for (int b = 0; b < BC; ++b) a[b] = 0.0f;
+                    for (int q = 0; q < BC / 4; ++q) xv[i][q] = *reinterpret_cast<const f32x4 *>(xg + 4 * q);
+                    if constexpr (VT == VAL_F32)
+                        v[i] = rv[j0 + i];
+                    else
+                        v[i] = word_val<VT>(rw[j0 + i]);
                 }
-            }
-            // The steps' registers are used up: loading into them earlier
-            // would make the compiler copy them, and a copy waits.
+                done += G;
+                left -= G;
 #pragma unroll
-            for (int i = 0; i < G; ++i) fetch(j0 + i, src + (kDepth + j0 + i) * SB);
+                for (int i = 0; i < G; ++i) {
+                    const uint32_t m = rw[j0 + i];
+#pragma unroll
+                    for (int q = 0; q < BC / 4; ++q)
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) a[4 * q + b] = fmaf(v[i], xv[i][q][b], a[4 * q + b]);
+                    if (__builtin_amdgcn_readfirstlane(m) & 0x8000u) {  // the slice ends: its 16 rows
+                        uint32_t row = (m & 15u) << (4u * (lane & 3u));
+                        row |= quad_get<0xB1>(row);
+                        row |= quad_get<0x4E>(row);
+                        // Sums over the row's four work-items, halved between
+                        // neighbours: work-item q keeps BC/4 right-hand sides.
+                        const bool o1 = lane & 1u, o2 = lane & 2u;
+                        float h[BC / 2];
+#pragma unroll
+                        for (int b = 0; b < BC / 2; ++b)
+                            h[b] = (o1 ? a[b + BC / 2] : a[b]) + quad_getf<0xB1>(o1 ? a[b] : a[b + BC / 2]);
+                        float *p = acc + row * BC + (o1 ? BC / 2 : 0) + (o2 ? BC / 4 : 0);
+                        if constexpr (BC == 4) {
+                            *p += (o2 ? h[1] : h[0]) + quad_getf<0x4E>(o2 ? h[0] : h[1]);
+                        } else {
+                            typedef float f32x2 __attribute__((ext_vector_type(2)));
+                            f32x2 o = *reinterpret_cast<f32x2 *>(p);
+                            o.x += (o2 ? h[2] : h[0]) + quad_getf<0x4E>(o2 ? h[0] : h[2]);
+                            o.y += (o2 ? h[3] : h[1]) + quad_getf<0x4E>(o2 ? h[1] : h[3]);
+                            *reinterpret_cast<f32x2 *>(p) = o;
+                        }
+#pragma unroll
+                        for (int b = 0; b < BC; ++b) a[b] = 0.0f;
+                    }
+                }
+                // The steps' registers are used up: loading into them earlier
+                // would make the compiler copy them, and a copy waits.
+#pragma unroll
+                for (int i = 0; i < G; ++i) fetch(j0 + i, src + (kDepth + j0 + i) * SB);
+            }
+            src += kDepth * SB;
         }
-        src += kDepth * SB;
+        while (t < nt) enter();  // tiles without steps for this wave
     }
-    while (t < nt) enter();  // tiles without steps for this wave
     __syncthreads();
-    for (uint32_t i = tid; i < R * BC; i += kSliceNT) pw[i] = acc[i];
+    if constexpr (DIRECT) {
+        const EpiArgs ea = se.pe.ea[pass];
+        switch (se.epi) {
+            case EPI_PLAIN: finish_rows<EPI_PLAIN, BC>(w.x * R, R, acc, se, ea); break;
+            case EPI_RATIO: finish_rows<EPI_RATIO, BC>(w.x * R, R, acc, se, ea); break;
+            default: finish_rows<EPI_UPDATE, BC>(w.x * R, R, acc, se, ea); break;
+        }
+    } else {
+        float *pw = part + ((uint64_t)pass * nwg + run) * R * BC;
+        for (uint32_t i = tid; i < R * BC; i += kSliceNT) pw[i] = acc[i];
+    }
 }
 
 // ----------------------------------------------------------------- builder
@@ -442,28 +466,32 @@ __global__ __launch_bounds__(kWG) void slice_scatter_kernel(const uint64_t *__re
 
 template <int W, int VT, int BC, int G>
 hipError_t launch_slices(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
-                         hipStream_t s) {
-    hipLaunchKernelGGL((slice_spmv_kernel<W, VT, BC, G>), dim3((wk.nwg + 7) / 8 * 8 * x.n), dim3(kSliceNT),
-                       slice_lds_bytes(p, BC), s, p.R, p.nseg, tm.wbase, wk.wl, wk.order, wk.tiles, tm.tdata, x, wk.nwg,
-                       part);
+                         const SliceEpi &se, hipStream_t s) {
+    const dim3 grid((wk.nwg + 7) / 8 * 8 * x.n);
+    if (se.direct)
+        hipLaunchKernelGGL((slice_spmv_kernel<W, VT, BC, G, true>), grid, dim3(kSliceNT), slice_lds_bytes(p, BC), s, p.R,
+                           p.nseg, tm.wbase, wk.wl, wk.order, wk.tiles, tm.tdata, x, wk.nwg, part, se);
+    else
+        hipLaunchKernelGGL((slice_spmv_kernel<W, VT, BC, G, false>), grid, dim3(kSliceNT), slice_lds_bytes(p, BC), s,
+                           p.R, p.nseg, tm.wbase, wk.wl, wk.order, wk.tiles, tm.tdata, x, wk.nwg, part, se);
     return hipGetLastError();
 }
 
 template <int VT>
 hipError_t launch_slices_vt(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
-                            uint32_t BC, hipStream_t s) {
+                            uint32_t BC, const SliceEpi &se, hipStream_t s) {
     if (BC == 4 && p.W == 1024) {
         switch (p.group) {
-            case 1: return launch_slices<1024, VT, 4, 1>(p, tm, wk, x, part, s);
-            case 2: return launch_slices<1024, VT, 4, 2>(p, tm, wk, x, part, s);
-            case 4: return launch_slices<1024, VT, 4, 4>(p, tm, wk, x, part, s);
+            case 1: return launch_slices<1024, VT, 4, 1>(p, tm, wk, x, part, se, s);
+            case 2: return launch_slices<1024, VT, 4, 2>(p, tm, wk, x, part, se, s);
+            case 4: return launch_slices<1024, VT, 4, 4>(p, tm, wk, x, part, se, s);
         }
     } else if (BC == 4 && p.W == 512) {
-        if (p.group == 1) return launch_slices<512, VT, 4, 1>(p, tm, wk, x, part, s);
-        if (p.group == 2) return launch_slices<512, VT, 4, 2>(p, tm, wk, x, part, s);
+        if (p.group == 1) return launch_slices<512, VT, 4, 1>(p, tm, wk, x, part, se, s);
+        if (p.group == 2) return launch_slices<512, VT, 4, 2>(p, tm, wk, x, part, se, s);
     } else if (BC == 8 && p.W == 512) {
-        if (p.group == 1) return launch_slices<512, VT, 8, 1>(p, tm, wk, x, part, s);
-        if (p.group == 2) return launch_slices<512, VT, 8, 2>(p, tm, wk, x, part, s);
+        if (p.group == 1) return launch_slices<512, VT, 8, 1>(p, tm, wk, x, part, se, s);
+        if (p.group == 2) return launch_slices<512, VT, 8, 2>(p, tm, wk, x, part, se, s);
     }
     return hipErrorInvalidValue;
 }
@@ -515,6 +543,24 @@ size_t slice_stream_count(const TilePlan &p) { return (size_t)p.nblk * kStreams 
 bool slices_suit(const TilePlan &quads, uint64_t steps, uint32_t most) {
     const uint64_t per_run = std::max<uint64_t>(1, steps / 2048);
     return steps * 64 * 4 <= (quads.cap - 8) * 5 && (most <= 256 || most <= per_run);
+}
+
+// A row block summed by one workgroup needs no partial sums and no reduction
+// (two launches in one), but its tiles are one chain: up to 16 segments, and
+// as many entries per block as there are other blocks to run beside it.
+// 4 right-hand sides per pass, 16 bits, us per iteration (FP and BP, FP's
+// blocks of 512 rows as one run or not), one pass / four / eight:
+//   64 x 64, 81 blocks of 24 Ki entries      32.7 -> 33.2 / 43.4 -> 39.7 / 55.8 -> 53.4
+//   40 x 40, 22 blocks of 15 Ki              24.2 -> 21.3 / 25.1 -> 22.1 / 26.7 -> 23.1
+//   96 x 96, 156 blocks of 36 Ki             47.0 -> 47.4 / 79.5 -> 73.9 /  129 ->  117
+//   128 x 128, 324 blocks of 48 Ki           75.5 -> 74.5 /  156 ->  146 /  310 ->  285
+//   128 x 128, 88 blocks of 48 Ki            43.0 -> 51.4 /  73  ->   69 /  119 ->  107
+// With 8 right-hand sides 24 Ki entries lose (one pass 40.4 -> 44.3, four
+// 70.8 -> 61.0) and 10 Ki win (977 blocks: 113 -> 94).
+bool slices_direct(uint32_t cols, uint32_t W, uint32_t R, uint64_t rows, uint64_t nnz, uint32_t BC) {
+    const uint64_t blocks = (rows + R - 1) / R;
+    const uint64_t most = BC == 8 ? 12288 : std::min<uint64_t>(65536, std::max<uint64_t>(16384, 400 * blocks));
+    return cols <= 16ull * W && nnz <= blocks * most;
 }
 
 size_t slice_data_bytes(const TilePlan &p) {
@@ -603,13 +649,13 @@ TileWorkList slice_work_list(const TilePlan &p, const uint32_t *wbase, uint32_t 
     return L;
 }
 
-hipError_t launch_slice_partials(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x,
-                                 float *part, uint32_t BC, hipStream_t s) {
+hipError_t launch_slice_spmv(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
+                             uint32_t BC, const SliceEpi &se, hipStream_t s) {
     switch (p.vt) {
-        case VAL_F32: return launch_slices_vt<VAL_F32>(p, tm, wk, x, part, BC, s);
-        case VAL_BF16: return launch_slices_vt<VAL_BF16>(p, tm, wk, x, part, BC, s);
-        case VAL_UF16: return launch_slices_vt<VAL_UF16>(p, tm, wk, x, part, BC, s);
-        default: return launch_slices_vt<VAL_F16>(p, tm, wk, x, part, BC, s);
+        case VAL_F32: return launch_slices_vt<VAL_F32>(p, tm, wk, x, part, BC, se, s);
+        case VAL_BF16: return launch_slices_vt<VAL_BF16>(p, tm, wk, x, part, BC, se, s);
+        case VAL_UF16: return launch_slices_vt<VAL_UF16>(p, tm, wk, x, part, BC, se, s);
+        default: return launch_slices_vt<VAL_F16>(p, tm, wk, x, part, BC, se, s);
     }
 }
 

@@ -748,61 +748,6 @@ __global__ __launch_bounds__(NT) void stream_spmv_kernel(uint32_t R, uint32_t ns
     for (uint32_t i = tid; i < R * BC; i += NT) pw[i] = acc[i];
 }
 
-// The epilogue of row r from its sum y over the block's workgroups: the
-// row's value scale (16-bit values), then the ratio, the update or the plain
-// sum.  Vectors are [rows][BC].  Its inputs are read by reduce_load before
-// the partials are summed, so that their memory round trip overlaps the
-// sum's instead of following it (a small matrix's reduction is a chain of
-// dependent round trips).
-template <int BC>
-struct ReduceIn {
-    float sc;     // the row's value scale (1 without scales)
-    float a[BC];  // RATIO: the counts; UPDATE: the image values
-    float n;      // UPDATE: the sensitivity
-    bool act[BC]; // UPDATE: the right-hand side is active
-};
-
-template <int EPI, int BC>
-__device__ __forceinline__ ReduceIn<BC> reduce_load(uint32_t r, const float *__restrict__ scale, const EpiArgs &ea) {
-    ReduceIn<BC> in;
-    in.sc = scale ? scale[r] : 1.0f;
-    in.n = 0.0f;
-#pragma unroll
-    for (int q = 0; q < BC; ++q) {
-        const uint64_t k = (uint64_t)r * BC + q;
-        in.a[q] = 0.0f;
-        in.act[q] = true;
-        if constexpr (EPI == EPI_RATIO) in.a[q] = (float)ea.g[k];
-        if constexpr (EPI == EPI_UPDATE) {
-            in.a[q] = ea.f[k];
-            in.act[q] = !ea.active || ea.active[q];
-        }
-    }
-    if constexpr (EPI == EPI_UPDATE) in.n = ea.norm[r];
-    return in;
-}
-
-template <int EPI, int BC>
-__device__ __forceinline__ void reduce_epilogue(uint32_t r, const float (&y)[BC], const ReduceIn<BC> &in,
-                                                bool scaled, const EpiArgs &ea) {
-#pragma unroll
-    for (int q = 0; q < BC; ++q) {
-        const uint64_t k = (uint64_t)r * BC + q;
-        const float yq = scaled ? y[q] * in.sc : y[q];
-        if constexpr (EPI == EPI_PLAIN) {
-            ea.out[k] = yq;
-        } else if constexpr (EPI == EPI_RATIO) {
-            // 16-bit values: the back projection's tiles hold the same codes
-            // without the row scales, so the ratio g / (scale * sum) goes on
-            // multiplied by the scale, that is g / sum.
-            ea.out[k] = (y[q] != 0.0f) ? in.a[q] / y[q] : 0.0f;
-        } else {
-            const float v = in.a[q] * yq;
-            if (in.act[q]) ea.f[k] = (in.n == 0.0f) ? v : v / in.n;
-        }
-    }
-}
-
 // y += the partials of row i (of R = 2^rshift) in workgroups w0, w0 + S,
 // ... below we, in that order.  The partials of U workgroups are loaded
 // together, then added in order: one memory latency per U workgroups
@@ -1643,13 +1588,29 @@ hipError_t launch_tiled_partials(const TilePlan &p, const TiledMatrix &tm, const
                                  float *part, uint32_t BC, uint32_t nt, hipStream_t s) {
     if (x.n == 0 || x.n > kMaxPasses) return hipErrorInvalidValue;
     if (p.rows == 0 || wk.nwg == 0) return hipSuccess;
-    if (p.slices) return launch_slice_partials(p, tm, wk, x, part, BC, s);
+    if (p.slices) return launch_slice_spmv(p, tm, wk, x, part, BC, SliceEpi{}, s);
     switch (p.vt) {
         case VAL_F32: return launch_vt<VAL_F32>(p, tm, wk, x, part, BC, nt, s);
         case VAL_BF16: return launch_vt<VAL_BF16>(p, tm, wk, x, part, BC, nt, s);
         case VAL_UF16: return launch_vt<VAL_UF16>(p, tm, wk, x, part, BC, nt, s);
         default: return launch_vt<VAL_F16>(p, tm, wk, x, part, BC, nt, s);
     }
+}
+
+hipError_t launch_tiled_spmv(const TilePlan &p, const TiledMatrix &tm, const TileWork &wk, const PassX &x, float *part,
+                             uint32_t BC, uint32_t nt, Epi epi, const PassEpi &pe, hipStream_t s) {
+    if (!wk.direct || p.rows == 0) {
+        const hipError_t e = launch_tiled_partials(p, tm, wk, x, part, BC, nt, s);
+        return e != hipSuccess ? e : launch_tiled_reduce(p, tm, wk, part, BC, epi, pe, s);
+    }
+    if (x.n == 0 || x.n > kMaxPasses || pe.n != x.n) return hipErrorInvalidValue;
+    SliceEpi se{};
+    se.direct = 1;
+    se.epi = epi;
+    se.rows = p.rows;
+    se.scale = tm.scale;
+    se.pe = pe;
+    return launch_slice_spmv(p, tm, wk, x, nullptr, BC, se, s);
 }
 
 bool valid_stream_threads(uint32_t nt) { return nt == 0 || nt == 128 || nt == 256 || nt == 512; }

@@ -49,5 +49,60 @@ struct SegWalk {
     }
 };
 
+// The epilogue of row r from its sum y over the block's workgroups: the
+// row's value scale (16-bit values), then the ratio, the update or the plain
+// sum.  Vectors are [rows][BC].  Its inputs are read by reduce_load before
+// the partials are summed, so that their memory round trip overlaps the
+// sum's instead of following it (a small matrix's reduction is a chain of
+// dependent round trips).
+template <int BC>
+struct ReduceIn {
+    float sc;     // the row's value scale (1 without scales)
+    float a[BC];  // RATIO: the counts; UPDATE: the image values
+    float n;      // UPDATE: the sensitivity
+    bool act[BC]; // UPDATE: the right-hand side is active
+};
+
+template <int EPI, int BC>
+__device__ __forceinline__ ReduceIn<BC> reduce_load(uint32_t r, const float *__restrict__ scale, const EpiArgs &ea) {
+    ReduceIn<BC> in;
+    in.sc = scale ? scale[r] : 1.0f;
+    in.n = 0.0f;
+#pragma unroll
+    for (int q = 0; q < BC; ++q) {
+        const uint64_t k = (uint64_t)r * BC + q;
+        in.a[q] = 0.0f;
+        in.act[q] = true;
+        if constexpr (EPI == EPI_RATIO) in.a[q] = (float)ea.g[k];
+        if constexpr (EPI == EPI_UPDATE) {
+            in.a[q] = ea.f[k];
+            in.act[q] = !ea.active || ea.active[q];
+        }
+    }
+    if constexpr (EPI == EPI_UPDATE) in.n = ea.norm[r];
+    return in;
+}
+
+template <int EPI, int BC>
+__device__ __forceinline__ void reduce_epilogue(uint32_t r, const float (&y)[BC], const ReduceIn<BC> &in,
+                                                bool scaled, const EpiArgs &ea) {
+#pragma unroll
+    for (int q = 0; q < BC; ++q) {
+        const uint64_t k = (uint64_t)r * BC + q;
+        const float yq = scaled ? y[q] * in.sc : y[q];
+        if constexpr (EPI == EPI_PLAIN) {
+            ea.out[k] = yq;
+        } else if constexpr (EPI == EPI_RATIO) {
+            // 16-bit values: the back projection's tiles hold the same codes
+            // without the row scales, so the ratio g / (scale * sum) goes on
+            // multiplied by the scale, that is g / sum.
+            ea.out[k] = (y[q] != 0.0f) ? in.a[q] / y[q] : 0.0f;
+        } else {
+            const float v = in.a[q] * yq;
+            if (in.act[q]) ea.f[k] = (in.n == 0.0f) ? v : v / in.n;
+        }
+    }
+}
+
 }  // namespace
 }  // namespace mlem

@@ -165,7 +165,8 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     ARGCHK(values <= VAL_UF16, "mlem_matrix_create_tiled: values must be 0 (f32), 1 (bf16), 2 (fp16) or 3 (uf16)");
     HIPCHK(hipSetDevice(device));
     // as a reconstruction over the resident CSR would choose
-    const uint32_t R = tile_rows ? tile_rows : default_tile_rows(nnz, 0, values, BC);
+    const uint32_t R = tile_rows ? tile_rows : default_tile_rows(rows, cols, nnz, 0, values, BC),
+                   RT = tile_rows ? tile_rows : default_tile_rows(cols, rows, nnz, 0, values, BC);
     auto m = std::make_unique<mlem_matrix>();
     m->device = device;
     m->rows = rows;
@@ -173,7 +174,8 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     m->nnz = nnz;
     m->tiles_only = true;
     m->tile_W = W;
-    m->tile_R = R;
+    m->tile_R[0] = R;
+    m->tile_R[1] = RT;
     m->tile_vt = values;
     m->tile_bc = BC;
     const size_t margin = (size_t)1 << 30;
@@ -188,7 +190,7 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     HIPCHK(m->sens64.alloc(sizeof(double) * cols));
     auto tT = std::make_unique<Tiled>();
     auto tA = std::make_unique<Tiled>();
-    TilePlan pT = tile_plan(cols, rows, nnz, W, R, values, quad);
+    TilePlan pT = tile_plan(cols, rows, nnz, W, RT, values, quad);
     pT.unit_scale = values != VAL_F32;  // A^T's tiles hold A's codes (decoded below, in place)
     ChunkedTiles bT(pT, tT.get());
     ChunkedTiles bA(tile_plan(rows, cols, nnz, W, R, values, quad), tA.get());
@@ -253,10 +255,10 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             uint32_t nr = 0;
             const hipError_t e = transpose_ranges_to(rows, cols, nnz, rp.as<uint64_t>(), ci.as<uint32_t>(),
                                                      va.as<float>(), colptrT.as<uint64_t>(), nullptr, nullptr,
-                                                     budget / 2, R, sink, &nr, nullptr);
+                                                     budget / 2, RT, sink, &nr, nullptr);
             if (st_sink != MLEM_OK) return st_sink;
             if (e == hipErrorOutOfMemory)
-                return set_err(MLEM_ERR_OUT_OF_MEMORY, "mlem_matrix_create_tiled: %u rows of A^T do not fit", R);
+                return set_err(MLEM_ERR_OUT_OF_MEMORY, "mlem_matrix_create_tiled: %u rows of A^T do not fit", RT);
             HIPCHK(e);
             progress("A^T tiles %s over %u column ranges (%.1f GB of range scratch)", pass ? "filled" : "counted", nr,
                      budget / 2 / 1e9);
@@ -330,7 +332,7 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
         HIPCHK(hipMemcpy(tT->sens.p, m->sens32.p, sizeof(float) * cols, hipMemcpyDeviceToDevice));
     }
     m->tiles.emplace(std::make_tuple(0, W, R, values, quad, false), std::move(tA));
-    m->tiles.emplace(std::make_tuple(1, W, R, values, quad, false), std::move(tT));
+    m->tiles.emplace(std::make_tuple(1, W, RT, values, quad, false), std::move(tT));
     *out = m.release();
     return MLEM_OK;
 }

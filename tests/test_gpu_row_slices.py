@@ -71,3 +71,32 @@ def test_edges_of_slices_and_runs(name, values, per_pass, width, rows, groups):
             assert rel_l2(img, ref) <= (2e-6 if values else 1e-5)
         else:
             assert np.array_equal(img, images[k % 2])  # the slot does not matter
+
+
+@pytest.mark.parametrize("per_pass,values", [(4, 0), (4, 3), (8, 1)])
+@pytest.mark.parametrize("rows,cols,gap", [(1, 40, 0), (511, 1025, 0), (512, 16 * 512, 0), (513, 16 * 512 + 1, 0),
+                                           (1537, 16 * 1024, 0), (1537, 16 * 1024 + 1, 0), (2000, 300, 600)])
+def test_row_blocks_as_one_run(rows, cols, gap, per_pass, values):
+    """Default tiles of small matrices, whose row blocks are one run each (no partial sums): a last block of one
+    row or one short of a block, as many column segments as such a run takes and one more, and a block without any
+    entries (rows 512 .. 512 + gap empty), which takes the reduction."""
+    rng = np.random.default_rng(rows + cols)
+    lens = rng.integers(0, 1 + min(cols, 24), rows)
+    lens[0] = 3
+    if gap:
+        lens[512:512 + gap] = 0
+    A = csr(lens, rng.integers(0, max(1, cols // 2), rows), cols, stride=1)
+    g = rng.integers(0, 50, A.rows).astype(np.int32)
+    f0 = np.ones(A.cols, np.float32)
+    val = O.quantize_values(A.rowptr, A.val, A.rows, values).astype(np.float32) if values else A.val
+    sens = O.colsum_f64(A.rowptr, A.col, val, A.rows, A.cols).astype(np.float32).astype(np.float64)
+    ref = O.mlem_f64(A.rowptr, A.col, val, A.rows, A.cols, g, sens, f0, 5)
+    with M.ResidentMatrix(A, M.transpose(A)) as m:
+        with M.Batch(m, 3 * per_pass, values=values, per_pass=per_pass, use_graph=1) as b:
+            for k in range(3 * per_pass):
+                b.set(k, g, f0)
+            for n in (2, 1, 2):
+                b.iterate(n)
+                b.sync()
+            for k in (0, per_pass - 1, 2 * per_pass, 3 * per_pass - 1):
+                assert rel_l2(b.image(k), ref) <= (2e-6 if values else 1e-5)

@@ -466,39 +466,50 @@ __global__ __launch_bounds__(kWG) void scatter_kernel(const uint64_t *__restrict
 
 // Scatter BP with the sums of a window of columns in LDS: a workgroup owns up
 // to kWinRows rows (one per lane of its waves) and walks them window by
-// window; in a window every wave takes its rows that reach into it, 64
-// entries at a time, kWinSlots rows in flight, and adds into LDS.  The
+// window; in a window every wave takes its rows that reach into it, a piece
+// of 64 U entries at a time, S rows in flight, and adds into LDS.  The
 // window's sums then go out as one run of consecutive atomics instead of one
 // scattered atomic per entry (a wave's 64 entries touch 25 lines; the
 // device-wide adds are done per line).  P is the next entry of the lane's
 // row, NC its column.  A row leaves a window at its first entry outside it;
 // what an unsorted row still holds after the last window is added entry by
-// entry.  The walk ends: a slot advances 64 entries or closes, and each
-// window opens a row once.
-// Bound by the LDS atomics (about 4 clocks per entry and CU): the mid-sized
-// scanner (1.8e8 nonzeros, every row's factor nonzero) takes 1.15 ms against
-// 4.16 with scattered atomics, the 12 GB scanner 9.3 against 34.3, the 2D
-// ring 24 against 132 us.  4 rows in flight per wave are as fast as 8 or 12,
-// 16,384-column windows (two workgroups per CU) as 32,768.
+// entry.  The walk ends: a slot advances a piece or closes, and each window
+// opens a row once.
+//
+// The sums are FP64 where a row has many entries in a window: the LDS adds an
+// FP32 value of one lane after the other (193 clocks per wave instruction
+// whatever the addresses, measured), FP64 values in 20 to 60.  Half as many
+// columns fit, so rows open twice as often, which is what short rows cost.
+// Bound by the loads then (without the adds 0.50 ms, without what goes out
+// 0.51 of the 0.55).  us, every row's factor nonzero; FP32 sums / FP64 with
+// U = 1, S = 4 / FP64 with U = 2, S = 3, by the mean entries e of a row in
+// 32,768 columns:
+//   1e6 rows x 200,000, e = 3          938 / 1300 / 1581
+//   200,000 x 100,000, e = 12          164 /  191 /  218
+//   200,000 x 100,000, e = 25          212 /  208 /  241
+//   200,000 x 100,000, e = 50          311 /  216 /  263
+//   mid-sized scanner, e = 155        1153 /  574 /  550  (scattered atomics 4165)
+//   500 rows x 100,000, e = 1000       103 /  102 /   85
+// The 12 GB scanner takes 5.1 ms (FP32 sums 9.3, scattered atomics 34.7).
 constexpr int kWinNT = 1024;
-constexpr uint32_t kWinCols = 32768;               // columns per window
 constexpr uint32_t kWinRows = 64 * (kWinNT / 64);  // rows per workgroup at most
-constexpr int kWinSlots = 4;
-constexpr size_t kWinLds = kWinCols * sizeof(float);
+constexpr uint32_t kWinColsF32 = 32768, kWinColsF64 = 20224;  // columns per window (128 and 158 KB)
 
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, uint32_t k) {
     return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), k) << 32) |
            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, k);
 }
 
+template <typename T, uint32_t kWinCols, int U, int S>
 __global__ __launch_bounds__(kWinNT) void scatter_window_kernel(const uint64_t *__restrict__ rowptr,
                                                                 const uint32_t *__restrict__ col,
                                                                 const float *__restrict__ val,
                                                                 const float *__restrict__ xrow,
                                                                 float *__restrict__ out, uint32_t rows, uint32_t cols,
                                                                 uint32_t per_wg) {
-    extern __shared__ __attribute__((aligned(16))) float win[];  // [kWinCols]
-    constexpr uint32_t NW = kWinNT / 64;
+    extern __shared__ __attribute__((aligned(16))) char win_mem[];
+    T *win = reinterpret_cast<T *>(win_mem);         // [kWinCols]
+    constexpr uint32_t NW = kWinNT / 64, PC = 64 * U;  // PC: entries per piece
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r0 = blockIdx.x * per_wg, nr = min(per_wg, rows - r0);
     const uint32_t mine = wv + NW * lane;  // lane k of wave w: row r0 + w + NW * k
@@ -514,13 +525,13 @@ __global__ __launch_bounds__(kWinNT) void scatter_window_kernel(const uint64_t *
             w0 = w1;
             continue;
         }
-        for (uint32_t i = tid; i < wn; i += kWinNT) win[i] = 0.0f;
+        for (uint32_t i = tid; i < wn; i += kWinNT) win[i] = T(0);
         __syncthreads();
         uint64_t todo = __ballot(NC < w1);
         if (todo) {
-            uint64_t p[kWinSlots], left[kWinSlots];  // next entry, entries from it on (0: no row)
-            uint32_t row[kWinSlots], c[kWinSlots], nopen = 0;
-            float a[kWinSlots], v[kWinSlots];
+            uint64_t p[S], left[S];  // next entry, entries from it on (0: no row)
+            uint32_t row[S], c[S][U], nopen = 0;
+            float a[S], v[S][U];
             auto take = [&](int j) {
                 p[j] = base;
                 left[j] = 0;
@@ -539,34 +550,52 @@ __global__ __launch_bounds__(kWinNT) void scatter_window_kernel(const uint64_t *
             // Lanes past the row's end re-read its entry p (a slot without a
             // row: the workgroup's first entry), so the loads are unconditional.
             auto fetch = [&](int j) {
-                const uint32_t l = lane < left[j] ? lane : 0u;
-                c[j] = ldnt(col + p[j] + l);
-                v[j] = ldnt(val + p[j] + l);
+#pragma unroll
+                for (uint32_t u = 0; u < (uint32_t)U; ++u) {
+                    const uint32_t l = lane + 64 * u < left[j] ? lane + 64 * u : 0u;
+                    c[j][u] = ldnt(col + p[j] + l);
+                    v[j][u] = ldnt(val + p[j] + l);
+                }
             };
 #pragma unroll
-            for (int j = 0; j < kWinSlots; ++j) {
+            for (int j = 0; j < S; ++j) {
                 take(j);
                 fetch(j);
             }
             while (nopen) {
 #pragma unroll
-                for (int j = 0; j < kWinSlots; ++j) {
-                    const uint32_t cc = c[j], rj = row[j];
+                for (int j = 0; j < S; ++j) {
+                    const uint32_t rj = row[j];
                     const uint64_t pj = p[j], lj = left[j];
-                    const float t = v[j] * a[j];
-                    const uint64_t m = __ballot(cc >= w0 && cc < w1 && lane < lj);
-                    const uint32_t n = m == ~0ull ? 64u : (uint32_t)__builtin_ctzll(~m);  // entries in the window
-                    if (n == 64u && lj > 64u) {
-                        p[j] += 64;
-                        left[j] -= 64;
+                    uint32_t cc[U], n = 0;  // n: entries in the window
+                    float t[U];
+#pragma unroll
+                    for (uint32_t u = 0; u < (uint32_t)U; ++u) {
+                        cc[u] = c[j][u];
+                        t[u] = v[j][u] * a[j];
+                        const uint64_t m = ~__ballot(cc[u] >= w0 && cc[u] < w1 && lane + 64 * u < lj);
+                        if (n == 64 * u) n += m ? (uint32_t)__builtin_ctzll(m) : 64u;
+                    }
+                    const bool more = n == PC && lj > PC;
+                    if (more) {
+                        p[j] += PC;
+                        left[j] -= PC;
                     } else {
                         nopen -= lj ? 1u : 0u;
                         take(j);
                     }
                     fetch(j);
-                    if (lane < n) unsafeAtomicAdd(win + (cc - w0), t);
-                    if (lj && !(n == 64u && lj > 64u)) {
-                        const uint32_t nc = n < lj ? (uint32_t)__builtin_amdgcn_readlane((int)cc, n) : 0xffffffffu;
+#pragma unroll
+                    for (uint32_t u = 0; u < (uint32_t)U; ++u)
+                        if (lane + 64 * u < n) unsafeAtomicAdd(win + (cc[u] - w0), (T)t[u]);
+                    if (lj && !more) {
+                        uint32_t nc = 0xffffffffu;
+                        if (n < lj) {
+                            nc = (uint32_t)__builtin_amdgcn_readlane((int)cc[0], n & 63u);
+#pragma unroll
+                            for (uint32_t u = 1; u < (uint32_t)U; ++u)
+                                if (n >= 64 * u) nc = (uint32_t)__builtin_amdgcn_readlane((int)cc[u], n & 63u);
+                        }
                         if (lane == rj) {
                             P = pj + n;
                             NC = nc;
@@ -577,7 +606,7 @@ __global__ __launch_bounds__(kWinNT) void scatter_window_kernel(const uint64_t *
         }
         __syncthreads();
         for (uint32_t i = tid; i < wn; i += kWinNT)
-            if (win[i] != 0.0f) unsafeAtomicAdd(out + w0 + i, win[i]);
+            if (win[i] != T(0)) unsafeAtomicAdd(out + w0 + i, (float)win[i]);
         __syncthreads();
         w0 = w1;
     }
@@ -782,6 +811,14 @@ hipError_t launch_csr_vector_g(const uint64_t *rowptr, const uint32_t *col, cons
     return hipGetLastError();
 }
 
+template <typename T, uint32_t COLS, int U, int S>
+hipError_t launch_window(const uint64_t *rowptr, const uint32_t *col, const float *val, const float *xrow, float *out,
+                         uint32_t rows, uint32_t cols, uint32_t per, hipStream_t s) {
+    hipLaunchKernelGGL((scatter_window_kernel<T, COLS, U, S>), dim3(blocks_for(rows, per)), dim3(kWinNT),
+                       COLS * sizeof(T), s, rowptr, col, val, xrow, out, rows, cols, per);
+    return hipGetLastError();
+}
+
 template <int G>
 hipError_t launch_scatter_g(const uint64_t *rowptr, const uint32_t *col, const float *val, const float *xrow,
                             float *out, uint32_t rows, hipStream_t s) {
@@ -927,14 +964,14 @@ hipError_t launch_scatter(uint32_t lanes, const uint64_t *rowptr, const uint32_t
         const uint32_t per = scatter_window_rows(rows);
         const uint64_t nwg = blocks_for(rows, per);
         // Each workgroup clears and sends out its columns once, so the windows
-        // pay from about one nonzero per 30 columns and workgroup on; with one
-        // per 10 (2e7 nonzeros in 1e6 x 200,000) 0.55 against 0.97 ms, with
-        // one per 25 even or up to 2.7 times slower (500 rows x 100,000, 71
-        // against 26 us).
+        // pay from about one nonzero per 16 columns and workgroup on; windows /
+        // scattered atomics, us: with one per 10 (1e6 x 200,000) 938 / 974,
+        // per 6 (500 x 100,000) 108 / 142, per 25 (1e6 x 200,000) 754 / 394.
         if (16 * nnz >= nwg * cols) {
-            hipLaunchKernelGGL(scatter_window_kernel, dim3((uint32_t)nwg), dim3(kWinNT), kWinLds, s, rowptr, col, val,
-                               xrow, out, rows, cols, per);
-            return hipGetLastError();
+            const uint64_t wins = (uint64_t)rows * blocks_for(cols, kWinColsF32);  // nnz / wins: e above
+            if (nnz < 25 * wins) return launch_window<float, kWinColsF32, 1, 4>(rowptr, col, val, xrow, out, rows, cols, per, s);
+            if (nnz < 100 * wins) return launch_window<double, kWinColsF64, 1, 4>(rowptr, col, val, xrow, out, rows, cols, per, s);
+            return launch_window<double, kWinColsF64, 2, 3>(rowptr, col, val, xrow, out, rows, cols, per, s);
         }
         lanes = auto_lanes(rows, nnz);
     }

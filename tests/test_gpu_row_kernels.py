@@ -118,3 +118,27 @@ def test_scatter_windows_over_several_rounds_of_rows():
         dr, out = M.DeviceArray.from_numpy(r), M.DeviceArray(A.cols, np.float32)
         M.bp_scatter(rp, ci, va, dr, out, A.rows, A.cols, A.nnz)
         assert np.all(np.abs(out.numpy() - y) <= (n + 64) * EPS * y)
+
+
+@pytest.mark.parametrize("lens,edge", [([127, 128, 129, 255, 256, 257, 383, 384] * 200, 20224), ([40, 64, 65, 90] * 1500, 20224),
+                                       ([20000, 4096, 1000] * 3, 20224), ([20000, 4096, 1000] * 3, 40448),
+                                       ([3, 9, 24, 1] * 15000, 32768)])
+def test_scatter_windows_of_each_kind(lens, edge):
+    """Rows of consecutive columns across a window's edge, with few, some and many entries per row and window (FP32
+    sums, FP64 sums 64 and 128 entries at a time), and rows that end with a piece."""
+    cols = edge + max(lens)
+    assert 16 * sum(lens) >= min(len(lens), 256) * cols  # windows
+    rng = np.random.default_rng(11)
+    start = [max(0, min(cols - n, edge - rng.integers(0, n + 1))) for n in lens]
+    start[0], start[1] = 0, edge  # from the first column; from the edge on
+    rowptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    col = np.concatenate([np.arange(s, s + n) for s, n in zip(start, lens)]).astype(np.uint32)
+    A = M.Csr(len(lens), cols, rowptr, col, (rng.random(col.size) + 0.01).astype(np.float32))
+    r = rng.random(A.rows).astype(np.float32) + 0.1
+    y = A.to_scipy().astype(np.float64).T @ r.astype(np.float64)
+    n = np.bincount(A.col, minlength=cols)
+    with M.ResidentMatrix(A) as mm:
+        rp, ci, va = mm.device_arrays()[:3]
+        dr, out = M.DeviceArray.from_numpy(r), M.DeviceArray.from_numpy(np.full(cols, 7.0, np.float32))
+        M.bp_scatter(rp, ci, va, dr, out, A.rows, cols, A.nnz)
+        assert np.all(np.abs(out.numpy() - y) <= (n + 64) * EPS * y)

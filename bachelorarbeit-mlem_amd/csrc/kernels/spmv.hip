@@ -481,7 +481,11 @@ __global__ __launch_bounds__(kWG) void scatter_kernel(const uint64_t *__restrict
 // whatever the addresses, measured), FP64 values in 20 to 60.  Half as many
 // columns fit, so rows open twice as often, which is what short rows cost.
 // Bound by the loads then (without the adds 0.50 ms, without what goes out
-// 0.51 of the 0.55).  us, every row's factor nonzero; FP32 sums / FP64 with
+// 0.51 of the 0.55; loads that stay in the caches for the next window's
+// pieces bring it to 0.51).  Rows dealt to the workgroups in turn, which
+// balances them better, lose: neighbours share columns, so fewer sums go out
+// (0.52, and 113 against 91 us with 4.4e7 nonzeros).  us with non-temporal
+// loads, every row's factor nonzero; FP32 sums / FP64 with
 // U = 1, S = 4 / FP64 with U = 2, S = 3, by the mean entries e of a row in
 // 32,768 columns:
 //   1e6 rows x 200,000, e = 3          938 / 1300 / 1581
@@ -549,12 +553,14 @@ __global__ __launch_bounds__(kWinNT) void scatter_window_kernel(const uint64_t *
             };
             // Lanes past the row's end re-read its entry p (a slot without a
             // row: the workgroup's first entry), so the loads are unconditional.
+            // Not non-temporal: a row's piece that ends in the next window is
+            // read again there, from the MALL.
             auto fetch = [&](int j) {
 #pragma unroll
                 for (uint32_t u = 0; u < (uint32_t)U; ++u) {
                     const uint32_t l = lane + 64 * u < left[j] ? lane + 64 * u : 0u;
-                    c[j][u] = ldnt(col + p[j] + l);
-                    v[j][u] = ldnt(val + p[j] + l);
+                    c[j][u] = col[p[j] + l];
+                    v[j][u] = val[p[j] + l];
                 }
             };
 #pragma unroll

@@ -173,12 +173,16 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
         shapes = {{1024, 1024}, {1024, 2048}, {1024, 4096}, {2048, 1024}, {2048, 2048}};
         groups = {16, 24, 32};
     } else if (BC == 4) {
-        shapes = {{512, 1024}, {512, 2048}, {1024, 1024}};
-        groups = {8, 16};
+        shapes = {{512, 1024}, {1024, 1024}, {1024, 2048}};
+        groups = {4, 8};
     } else {
         shapes = {{512, 512}, {512, 1024}};
-        groups = {8, 16};
+        groups = {4, 8};
     }
+    // Batches of several passes share their launches, and taller tiles pay
+    // then (683 M entries, one pass of 4 equal at 1024 and 2048 rows, four
+    // 4110 against 3600 us): they are timed four passes at a time.
+    const uint32_t passes = BC == 1 ? 1u : 4u;
     std::set<mlem_matrix::TileKey> before;
     {
         std::lock_guard<std::mutex> lk(m->mu);
@@ -189,8 +193,8 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
     DevBuf xf, xb, yf, yb;
     HIPCHK(xf.alloc(sizeof(float) * cols_x * BC));
     HIPCHK(xb.alloc(sizeof(float) * rows_x * BC));
-    HIPCHK(yf.alloc(sizeof(float) * rows_x * BC));
-    HIPCHK(yb.alloc(sizeof(float) * cols_x * BC));
+    HIPCHK(yf.alloc(sizeof(float) * rows_x * BC * passes));
+    HIPCHK(yb.alloc(sizeof(float) * cols_x * BC * passes));
     hipStream_t s = nullptr;
     HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -215,12 +219,17 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
     // One side's time per launch (partials + reduce), mean of three after a warm-up.
     auto time_side = [&](const Tiled *t, const TileWorkDev *w, DevBuf &part, const float *x, float *y, uint32_t nt,
                          double *ms) {
-        EpiArgs ea{};
-        ea.out = y;
+        PassX px{};
+        PassEpi pe{};
+        for (uint32_t k = 0; k < passes; ++k) {
+            px.x[k] = x;
+            pe.ea[k].out = y + k * (size_t)t->plan.rows * BC;
+        }
+        px.n = pe.n = passes;
         for (int rep = 0; rep < 4; ++rep) {
             if (rep == 1 && hipEventRecord(e0, s) != hipSuccess) return hipErrorUnknown;
-            const hipError_t e = launch_tiled_spmv(t->plan, t->view, w->view, one_pass(x), part.as<float>(), BC, nt,
-                                                   EPI_PLAIN, one_pass(ea), s);
+            const hipError_t e = launch_tiled_spmv(t->plan, t->view, w->view, px, part.as<float>(), BC, nt, EPI_PLAIN,
+                                                   pe, s);
             if (e != hipSuccess) return e;
         }
         hipError_t e = hipEventRecord(e1, s);
@@ -234,9 +243,18 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
         for (uint32_t g : groups) {
             const Tiled *tf = nullptr, *tb = nullptr;
             const TileWorkDev *wf = nullptr, *wb = nullptr;
-            DevBuf pf, pb;
-            int st = setup_tiled(m, 0, sh.first, sh.second, values, BC, g * (uint32_t)cus, &tf, &wf, &pf);
-            if (st == MLEM_OK) st = setup_tiled(m, 1, sh.first, sh.second, values, BC, g * (uint32_t)cus, &tb, &wb, &pb);
+            DevBuf part;  // FP and BP in turn
+            int st = setup_tiled(m, 0, sh.first, sh.second, values, BC, g * (uint32_t)cus, &tf, &wf, nullptr);
+            if (st == MLEM_OK)
+                st = setup_tiled(m, 1, sh.first, sh.second, values, BC, g * (uint32_t)cus, &tb, &wb, nullptr);
+            if (st == MLEM_OK) {
+                const hipError_t e = part.alloc(passes * std::max(tiled_part_bytes(tf->plan, wf->view.nwg, BC),
+                                                                  tiled_part_bytes(tb->plan, wb->view.nwg, BC)));
+                if (e == hipErrorOutOfMemory)
+                    st = MLEM_ERR_OUT_OF_MEMORY;
+                else
+                    HIPCHK(e);
+            }
             if (st == MLEM_ERR_UNSUPPORTED || st == MLEM_ERR_OUT_OF_MEMORY) {
                 (void)hipGetLastError();
                 continue;  // this shape does not suit or fit the matrix
@@ -246,9 +264,10 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
                 return st;
             }
             for (uint32_t nt : threads) {
+                if (tf->plan.slices && tb->plan.slices && nt != threads.back()) continue;  // without effect
                 double fp = 0, bp = 0;
-                hipError_t e = time_side(tf, wf, pf, xf.as<float>(), yf.as<float>(), nt, &fp);
-                if (e == hipSuccess) e = time_side(tb, wb, pb, xb.as<float>(), yb.as<float>(), nt, &bp);
+                hipError_t e = time_side(tf, wf, part, xf.as<float>(), yf.as<float>(), nt, &fp);
+                if (e == hipSuccess) e = time_side(tb, wb, part, xb.as<float>(), yb.as<float>(), nt, &bp);
                 if (e != hipSuccess) {
                     cleanup();
                     return hip_err(e, "mlem_autotune: timing", __FILE_NAME__, __LINE__);

@@ -432,7 +432,8 @@ typedef struct mlem_tune_result {
     uint32_t tile_width, tile_rows, tile_groups;
     uint32_t tile_threads; /* for mlem_batch_opts (0 for 1 per pass)       */
     uint32_t candidates;  /* shape x workgroup-count pairs timed            */
-    double fp_ms, bp_ms;  /* per launch of the chosen one, partials + reduce */
+    double fp_ms, bp_ms;  /* per launch of the chosen one, partials + reduce
+                             (4 or 8 per pass: of four passes)             */
 } mlem_tune_result;
 int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values,
                   mlem_tune_result *out);

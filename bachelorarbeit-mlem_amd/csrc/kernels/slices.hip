@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32
     const uint4 w = wl[run];
     const uint32_t nt = w.z;
     // Lane i: the segment of tile i of the run.
-    const uint32_t seg = tiles[w.y + min(lane, nt - 1)].x;
+    const uint32_t seg = tiles[w.y + min(lane, max(nt, 1u) - 1)].x;
     for (uint32_t i = tid; i < (R + 1) * BC; i += kSliceNT) acc[i] = 0.0f;
     if (tid < BC) {
         xs[W * BC + tid] = 0.0f;
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kSliceNT) void slice_spmv_kernel(uint32_t R, uint32
         const uint64_t wb = ((uint64_t)w.x * kStreams + wv) * nseg + seg;
         const uint32_t s0 = wbase[wb], s1 = wbase[wb + 1], cnt = s1 - s0;
         const uint32_t first = __builtin_amdgcn_readfirstlane(s0);
-        const uint32_t total = __builtin_amdgcn_readlane(s1, nt - 1) - first;
+        const uint32_t total = nt ? __builtin_amdgcn_readlane(s1, nt - 1) - first : 0u;
         // The wave's steps, kDepth in flight (past its last step: whatever follows).
         const uint8_t *src = tdata + (uint64_t)first * SB;
         uint32_t rw[kDepth];  // 16-bit values: the words; f32: the metas
@@ -550,13 +550,13 @@ bool slices_suit(const TilePlan &quads, uint64_t steps, uint32_t most) {
 // as many entries per block as there are other blocks to run beside it.
 // 4 right-hand sides per pass, 16 bits, us per iteration (FP and BP, FP's
 // blocks of 512 rows as one run or not), one pass / four / eight:
-//   64 x 64, 81 blocks of 24 Ki entries      32.7 -> 33.2 / 43.4 -> 39.7 / 55.8 -> 53.4
-//   40 x 40, 22 blocks of 15 Ki              24.2 -> 21.3 / 25.1 -> 22.1 / 26.7 -> 23.1
-//   96 x 96, 156 blocks of 36 Ki             47.0 -> 47.4 / 79.5 -> 73.9 /  129 ->  117
-//   128 x 128, 324 blocks of 48 Ki           75.5 -> 74.5 /  156 ->  146 /  310 ->  285
-//   128 x 128, 88 blocks of 48 Ki            43.0 -> 51.4 /  73  ->   69 /  119 ->  107
-// With 8 right-hand sides 24 Ki entries lose (one pass 40.4 -> 44.3, four
-// 70.8 -> 61.0) and 10 Ki win (977 blocks: 113 -> 94).
+//   64 x 64, 81 blocks of 24 Ki entries      32.7 -> 30.4 / 43.4 -> 37.1 / 55.8 -> 49.5
+//   40 x 40, 22 blocks of 15 Ki              24.2 -> 21.3 / 25.1 -> 22.2 / 26.7 -> 23.2
+//   96 x 96, 156 blocks of 36 Ki             47.0 -> 45.6 / 79.5 -> 70.1 /  129 ->  108
+//   128 x 128, 324 blocks of 48 Ki           75.5 -> 72.3 /  156 ->  140 /  310 ->  272
+//   128 x 128, 88 blocks of 48 Ki            43.0 -> 48.3 /   73 ->   65 /  119 ->  101
+// With 8 right-hand sides 24 Ki entries gain only in several passes (one
+// 40.1 -> 41.4, four 70.3 -> 57.7) and 10 Ki in one (977 blocks: 113 -> 94).
 bool slices_direct(uint32_t cols, uint32_t W, uint32_t R, uint64_t rows, uint64_t nnz, uint32_t BC) {
     const uint64_t blocks = (rows + R - 1) / R;
     const uint64_t most = BC == 8 ? 12288 : std::min<uint64_t>(65536, std::max<uint64_t>(16384, 400 * blocks));
@@ -625,6 +625,10 @@ TileWorkList slice_work_list(const TilePlan &p, const uint32_t *wbase, uint32_t 
             n.push_back(st);
             left += st;
         }
+        if (n.empty() && target_wgs == 1) {  // one run per block: an empty one too (launch_tiled_spmv)
+            L.wl.insert(L.wl.end(), {b, 0u, 0u, 0u});
+            ++L.nwg;
+        }
         // Runs of nearly equal steps over the block's tiles.
         uint64_t runs = (left + per_run - 1) / per_run;
         for (size_t i = 0; i < n.size();) {
@@ -637,6 +641,11 @@ TileWorkList slice_work_list(const TilePlan &p, const uint32_t *wbase, uint32_t 
             left -= got;
             runs = runs > 1 ? runs - 1 : 1;
         }
+    }
+    if (L.ntl == 0) {  // no entries at all: no runs
+        L.wl.clear();
+        L.nwg = 0;
+        std::fill(L.wl_first.begin(), L.wl_first.end(), 0u);
     }
     L.wl_first[p.nblk] = L.nwg;
     // Launch order: by the column segment each run starts in, as for the

@@ -79,7 +79,7 @@ def test_edges_of_slices_and_runs(name, values, per_pass, width, rows, groups):
 def test_row_blocks_as_one_run(rows, cols, gap, per_pass, values):
     """Default tiles of small matrices, whose row blocks are one run each (no partial sums): a last block of one
     row or one short of a block, as many column segments as such a run takes and one more, and a block without any
-    entries (rows 512 .. 512 + gap empty), which takes the reduction."""
+    entries (rows 512 .. 512 + gap empty), whose run has no tiles."""
     rng = np.random.default_rng(rows + cols)
     lens = rng.integers(0, 1 + min(cols, 24), rows)
     lens[0] = 3

@@ -348,11 +348,22 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
         std::vector<uint32_t> wb(ns + 1);
         HIPCHK(hipMemcpy(wb.data(), wsteps.p, 4 * ns, hipMemcpyDeviceToHost));
         uint64_t steps = 0;
+        const uint64_t quad_cap = t->plan.cap;
         if (!fh[0] && slice_prefix(W, &wb, &steps, &t->plan.group) && slices_suit(t->plan, steps, fh[1])) {
             t->plan.slices = true;
             t->plan.steps = steps;
             t->plan.cap = steps * 64 + 8;
-            HIPCHK(t->mem.alloc(tiled_matrix_bytes(t->plan)));
+            const hipError_t e = t->mem.alloc(tiled_matrix_bytes(t->plan));
+            if (e == hipErrorOutOfMemory) {  // the quads, which may be smaller
+                (void)hipGetLastError();
+                t->plan.slices = false;
+                t->plan.steps = 0;
+                t->plan.cap = quad_cap;
+            } else {
+                HIPCHK(e);
+            }
+        }
+        if (t->plan.slices) {
             t->view = tiled_matrix_view(t->plan, t->mem.p);
             HIPCHK(hipMemcpy(t->view.wbase, wb.data(), 4 * wb.size(), hipMemcpyHostToDevice));
             DevBuf q;

@@ -91,8 +91,16 @@ struct ChunkedTiles {
             P.steps = steps;
             P.cap = steps * 64 + 8;
         }
+        hipError_t e = t->mem.alloc(tiled_matrix_bytes(P));
+        if (e == hipErrorOutOfMemory && slices) {  // the quads, which may be smaller
+            (void)hipGetLastError();
+            slices = P.slices = false;
+            P.steps = 0;
+            P.cap = run + 8;
+            e = t->mem.alloc(tiled_matrix_bytes(P));
+        }
+        HIPCHK(e);
         t->plan = P;
-        HIPCHK(t->mem.alloc(tiled_matrix_bytes(P)));
         t->view = tiled_matrix_view(P, t->mem.p);
         if (slices) {
             HIPCHK(hipMemcpy(t->view.wbase, wbase.data(), 4 * wbase.size(), hipMemcpyHostToDevice));

@@ -29,6 +29,7 @@ int set_err(int st, const char *fmt, ...) {
 }
 
 int hip_err(hipError_t e, const char *what, const char *file, int line) {
+    (void)hipGetLastError();  // reported here: the launch checks of later calls are not to find it again
     int st = (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation) ? MLEM_ERR_OUT_OF_MEMORY
              : (e == hipErrorNoDevice || e == hipErrorInvalidDevice) ? MLEM_ERR_NO_DEVICE
                                                                        : MLEM_ERR_HIP;

@@ -39,16 +39,8 @@ int hip_err(hipError_t e, const char *what, const char *file, int line) {
 hipError_t DevBuf::alloc(size_t n) {
     reset();
     if (n == 0) return hipSuccess;
-    hipError_t e = hipMalloc(&p, n);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        scratch_trim();
-        e = hipMalloc(&p, n);
-    }
-    if (e == hipSuccess)
-        bytes = n;
-    else
-        p = nullptr;
+    const hipError_t e = device_malloc(&p, n);
+    if (e == hipSuccess) bytes = n;
     return e;
 }
 
@@ -74,24 +66,38 @@ static Kept *kept_scratch() {
     return &(*all)[dev];
 }
 
-hipError_t Scratch::get(size_t n) {
-    Kept *k = n <= kKept ? kept_scratch() : nullptr;
-    if (k && !k->busy.exchange(true)) {
-        if (k->bytes < n) {
-            k->free();
-            const hipError_t e = hipMalloc(&k->p, n);
-            if (e != hipSuccess) {
-                k->p = nullptr;
-                k->busy = false;
-                return e;
-            }
-            k->bytes = n;
-        }
-        held = k;
-        p = k->p;
-        bytes = k->bytes;
-        return hipSuccess;
+// Half of the device's memory is free beside `kept` bytes.
+static bool memory_is_plenty(size_t kept) {
+    size_t free_b = 0, total_b = 0;
+    return hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b + kept >= total_b / 2;
+}
+
+bool Scratch::take_kept(const mlem_matrix *m, size_t n) {
+    if (m->serial < kFirst || n > kKept) return false;
+    Kept *k = kept_scratch();
+    if (!k || k->busy.exchange(true)) return false;
+    if (!memory_is_plenty(k->bytes)) {
+        k->free();
+        k->busy = false;
+        return false;
     }
+    if (k->bytes < n) {
+        k->free();
+        if (hipMalloc(&k->p, n) != hipSuccess) {
+            (void)hipGetLastError();
+            k->p = nullptr;
+            k->busy = false;
+            return false;
+        }
+        k->bytes = n;
+    }
+    held = k;
+    p = k->p;
+    bytes = k->bytes;
+    return true;
+}
+
+hipError_t Scratch::alloc(size_t n) {
     const hipError_t e = own.alloc(n);
     p = own.p;
     bytes = own.bytes;
@@ -101,18 +107,21 @@ hipError_t Scratch::get(size_t n) {
 Scratch::~Scratch() {
     if (!held) return;
     (void)hipStreamSynchronize(nullptr);  // also where the call failed half way
+    if (!memory_is_plenty(held->bytes)) held->free();
     held->busy = false;
 }
 
-void scratch_trim() {
+bool scratch_trim() {
     Kept *k = kept_scratch();
-    if (!k || k->busy.exchange(true)) return;
+    if (!k || k->busy.exchange(true)) return false;
+    const bool any = k->p != nullptr;
     k->free();
     k->busy = false;
+    return any;
 }
 
 hipError_t free_device_bytes(size_t *free_b) {
-    scratch_trim();
+    (void)scratch_trim();
     size_t total = 0;
     *free_b = 0;
     return hipMemGetInfo(free_b, &total);
@@ -196,6 +205,14 @@ int Upload::wait() {
 
 }  // namespace abi
 }  // namespace mlem
+
+hipError_t mlem::device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && abi::scratch_trim()) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) *p = nullptr;
+    (void)hipGetLastError();  // the caller has the error: the next launch is not to report it
+    return e;
+}
 
 // The message mlem_last_error() returns, for the other translation units of
 // the library (server.hip).
@@ -327,9 +344,8 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     // The fill's scratch behind the count's where the kept scratch holds
     // both (its size is known after the count; the guess covers padding).
     const size_t count_b = (tile_count_scratch_bytes(t->plan) + 255) & ~size_t(255);
-    const size_t both = count_b + m->nnz * (vt == VAL_F32 ? 5 : 7) + 4096;
     Scratch scratch;
-    HIPCHK(scratch.get(both <= Scratch::kKept ? both : count_b));
+    if (!scratch.take_kept(m, count_b + m->nnz * (vt == VAL_F32 ? 5 : 7) + 4096)) HIPCHK(scratch.alloc(count_b));
     uint32_t fl = 0;
     HIPCHK(launch_tile_count(t->plan, rp, ci, scratch.p, &fl, nullptr));
     if (fl) {
@@ -747,12 +763,21 @@ int mlem_device_alloc(void **ptr, size_t bytes) {
     ARGCHK(ptr, "mlem_device_alloc: null ptr");
     *ptr = nullptr;
     if (bytes == 0) return MLEM_OK;
-    HIPCHK(hipMalloc(ptr, bytes));
+    HIPCHK(device_malloc(ptr, bytes));
     return MLEM_OK;
 }
 
 int mlem_device_free(void *ptr) {
     if (ptr) HIPCHK(hipFree(ptr));
+    return MLEM_OK;
+}
+
+int mlem_release_scratch(int device) {
+    int cur = 0;
+    HIPCHK(hipGetDevice(&cur));
+    HIPCHK(hipSetDevice(device));
+    (void)scratch_trim();
+    HIPCHK(hipSetDevice(cur));
     return MLEM_OK;
 }
 
@@ -1185,21 +1210,17 @@ int mlem_matrix_build_transpose_limited(mlem_matrix *m, uint64_t scratch_bytes, 
     HIPCHK(va.alloc(sizeof(float) * m->nnz));
     const size_t whole = transpose_scratch_bytes(m->rows, m->cols, m->nnz);
     size_t budget = scratch_bytes;
-    // Automatic: one sort when its scratch fits beside a margin (or is small
-    // enough to be kept and can be had), else ranges in what is free.
+    // Automatic: one sort where its scratch fits beside a margin, else ranges
+    // in what is free.
     Scratch scratch;
-    bool have = false;
-    if (budget == 0) {
+    const bool kept = budget == 0 && scratch.take_kept(m, whole);
+    if (budget == 0 && !kept) {
+        HIPCHK(free_device_bytes(&budget));
         const size_t margin = (size_t)1 << 30;
-        have = whole <= Scratch::kKept && scratch.get(whole) == hipSuccess;
-        if (!have) {
-            (void)hipGetLastError();
-            HIPCHK(free_device_bytes(&budget));
-            budget = budget > margin ? budget - margin : 0;
-        }
+        budget = budget > margin ? budget - margin : 0;
     }
-    if (have || whole <= budget) {
-        if (!have) HIPCHK(scratch.get(whole));
+    if (kept || whole <= budget) {
+        if (!kept) HIPCHK(scratch.alloc(whole));
         HIPCHK(launch_transpose(m->rows, m->cols, m->nnz, m->rowptr.as<uint64_t>(), m->col.as<uint32_t>(),
                                 m->val.as<float>(), rp.as<uint64_t>(), ci.as<uint32_t>(), va.as<float>(), scratch.p,
                                 nullptr));

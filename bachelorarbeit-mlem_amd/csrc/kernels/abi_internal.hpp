@@ -70,7 +70,7 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
     }
-    hipError_t alloc(size_t n);  // when memory is short, kept scratch (below) is freed first
+    hipError_t alloc(size_t n);
     template <typename T>
     T *as() const {
         return static_cast<T *>(p);
@@ -78,30 +78,39 @@ struct DevBuf {
 };
 
 // Device scratch of a set-up call (the transpose's sort, the tile builder)
-// on the null stream, which has passed its last use when the call returns.
-// One buffer per device of up to kKept bytes is kept from call to call;
-// larger requests, and those that find it in use by another thread, get
-// memory of their own.  It is freed when an allocation fails or the free
-// memory is asked for (free_device_bytes).  Without it a one-shot
-// reconstruction on 1.8e8 nonzeros allocates and frees 13 GB, faster than
-// freed device memory comes back cleared: after a dozen of them calls of 56
-// ms took 0.3 to 3 s.
+// on the null stream, which has passed its last use when the call returns:
+// memory of its own, or the device's kept buffer.
+//   A program that sets up one matrix after another (reconstructions once
+// through, 1.8e8 nonzeros each) allocates and frees 11 GB per matrix, faster
+// than freed device memory comes back cleared: after some twenty of them
+// calls of 56 ms take 203 in the median and up to 3 s.  So from the third
+// matrix of a process on one buffer per device of up to kKept bytes is kept
+// from call to call, while half of the device's memory is free; a call that
+// finds it in use by another thread, too small a device or less free memory
+// takes memory of its own.  The buffer is given back when an allocation of
+// the library fails or it asks for the free memory, when a batch or
+// a tiles-only matrix has been created or the autotuner has run (programs
+// that then keep the card to themselves for long), and by
+// mlem_release_scratch.  The first two matrices leave nothing behind.
 struct Scratch {
     static constexpr size_t kKept = size_t(8) << 30;
+    static constexpr uint64_t kFirst = 3;  // the first matrix of the process that uses the kept buffer
     void *p = nullptr;
     size_t bytes = 0;  // at least what was asked for
     Scratch() = default;
     Scratch(const Scratch &) = delete;
     Scratch &operator=(const Scratch &) = delete;
     ~Scratch();
-    hipError_t get(size_t n);
+    bool take_kept(const mlem_matrix *m, size_t n);  // n bytes of the kept buffer, if it may be used
+    hipError_t alloc(size_t n);                      // memory of its own
 
 private:
     struct Kept *held = nullptr;
     DevBuf own;
 };
-// Frees the kept scratch of the current device unless it is in use.
-void scratch_trim();
+// Frees the kept scratch of the current device unless it is in use (or none
+// is kept: false).
+bool scratch_trim();
 // Free device memory with no scratch kept.
 hipError_t free_device_bytes(size_t *free_b);
 
@@ -175,6 +184,11 @@ struct Tiled {
 };
 
 struct mlem_matrix {
+    mlem_matrix() {
+        static std::atomic<uint64_t> made{0};
+        serial = ++made;
+    }
+    uint64_t serial;  // the how-manieth matrix of the process (Scratch)
     int device = 0;
     uint32_t rows = 0, cols = 0;
     uint64_t nnz = 0;

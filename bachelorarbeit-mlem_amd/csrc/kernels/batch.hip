@@ -295,6 +295,7 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
             it = (!before.count(k) && !chosen) ? m->tiles.erase(it) : std::next(it);
         }
     }
+    (void)scratch_trim();
     if (!tried) return set_err(MLEM_ERR_UNSUPPORTED, "mlem_autotune: no tile shape suits or fits this matrix");
     out->tile_width = bestW;
     out->tile_rows = bestR;
@@ -378,6 +379,7 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     else if (int st = sens_on_device(m, b->sens.as<float>(), nullptr, b->stream))
         return st;
     HIPCHK(hipStreamSynchronize(b->stream));
+    (void)scratch_trim();
     m->users.fetch_add(1);
     *out = b.release();
     return MLEM_OK;

@@ -12,6 +12,14 @@
 
 namespace mlem {
 
+// hipMalloc, tried again without the device's kept scratch (Scratch,
+// abi_internal.hpp) where memory is short; *p null on failure.
+hipError_t device_malloc(void **p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T **p, size_t bytes) {
+    return device_malloc(reinterpret_cast<void **>(p), bytes);
+}
+
 constexpr int kWG = 256;              // work-items per workgroup (4 wave64)
 constexpr uint32_t kMaxSecsize = 32;  // merge-path items per work-item
 

@@ -67,8 +67,8 @@ hipError_t reorder_rows(uint32_t rows, uint64_t nnz, const uint64_t *rowptr, con
     uint64_t *len = nullptr;
     void *tmp = nullptr;
     size_t tmp_bytes = 0;
-    if ((e = hipMalloc(&inv, sizeof(uint32_t) * std::max<uint32_t>(1, rows))) != hipSuccess) return e;
-    if ((e = hipMalloc(&len, sizeof(uint64_t) * ((size_t)rows + 1))) != hipSuccess) goto done;
+    if ((e = device_malloc(&inv, sizeof(uint32_t) * std::max<uint32_t>(1, rows))) != hipSuccess) return e;
+    if ((e = device_malloc(&len, sizeof(uint64_t) * ((size_t)rows + 1))) != hipSuccess) goto done;
     hipLaunchKernelGGL(invert_order_kernel, dim3(grid_for(rows)), dim3(kWG), 0, s, order, rows, inv);
     hipLaunchKernelGGL(placed_lengths_kernel, dim3(grid_for((uint64_t)rows + 1)), dim3(kWG), 0, s, rowptr, inv, rows,
                        len);
@@ -76,7 +76,7 @@ hipError_t reorder_rows(uint32_t rows, uint64_t nnz, const uint64_t *rowptr, con
     if ((e = rocprim::exclusive_scan(nullptr, tmp_bytes, len, rowptr_out, uint64_t(0), (size_t)rows + 1,
                                      rocprim::plus<uint64_t>(), s)) != hipSuccess)
         goto done;
-    if ((e = hipMalloc(&tmp, std::max<size_t>(tmp_bytes, 4))) != hipSuccess) goto done;
+    if ((e = device_malloc(&tmp, std::max<size_t>(tmp_bytes, 4))) != hipSuccess) goto done;
     if ((e = rocprim::exclusive_scan(tmp, tmp_bytes, len, rowptr_out, uint64_t(0), (size_t)rows + 1,
                                      rocprim::plus<uint64_t>(), s)) != hipSuccess)
         goto done;

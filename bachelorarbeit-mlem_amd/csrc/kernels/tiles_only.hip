@@ -341,6 +341,7 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     }
     m->tiles.emplace(std::make_tuple(0, W, R, values, quad, false), std::move(tA));
     m->tiles.emplace(std::make_tuple(1, W, RT, values, quad, false), std::move(tT));
+    (void)scratch_trim();
     *out = m.release();
     return MLEM_OK;
 }

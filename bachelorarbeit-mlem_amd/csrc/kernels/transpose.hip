@@ -190,7 +190,7 @@ hipError_t transpose_in_ranges(uint32_t rows, uint32_t cols, uint64_t nnz, const
     // take 20.3 ms this way and 33.5 as one range.
     const size_t whole = transpose_scratch_bytes(rows, cols, nnz);
     void *mem = nullptr;
-    if (whole <= budget && hipMalloc(&mem, whole) == hipSuccess) {
+    if (whole <= budget && device_malloc(&mem, whole) == hipSuccess) {
         *ranges_out = 0;
         hipError_t e = launch_transpose(rows, cols, nnz, rowptr, col, val, colptrT, rowT, valT, mem, s);
         const hipError_t e2 = hipStreamSynchronize(s);
@@ -230,7 +230,7 @@ hipError_t transpose_ranges_to(uint32_t rows, uint32_t cols, uint64_t nnz, const
     }
     const uint64_t max_n = lo;
     void *mem = nullptr;
-    if ((e = hipMalloc(&mem, fixed + range_scratch_bytes(cols, max_n))) != hipSuccess) return e;
+    if ((e = device_malloc(&mem, fixed + range_scratch_bytes(cols, max_n))) != hipSuccess) return e;
     char *p = static_cast<char *>(mem);
     uint32_t *ccnt = reinterpret_cast<uint32_t *>(p);
     p += align256(4 * ((size_t)cols + 1));

@@ -19,7 +19,7 @@ __all__ = ["hip_lib", "device_count", "device_info", "DeviceArray", "Stream", "E
            "fp_csr_vector",
            "bp_csr_vector", "bp_scatter", "fp_ratio_merge", "fp_ratio_csr_vector", "bp_update_merge",
            "bp_update_csr_vector", "ratio", "update", "colsum_f64", "colsum_scatter_f64", "fill_f32", "copy_f32",
-           "device_sync",
+           "device_sync", "release_scratch",
            "version"]
 
 _hip = None
@@ -40,6 +40,7 @@ def hip_lib() -> C.CDLL:
             "mlem_device_info": (cint, [cint, C.c_char_p, sz, P(u64), P(cint)]),
             "mlem_device_alloc": (cint, [P(vp), sz]),
             "mlem_device_free": (cint, [vp]),
+            "mlem_release_scratch": (cint, [cint]),
             "mlem_memcpy_h2d": (cint, [vp, vp, sz, vp]),
             "mlem_memcpy_d2h": (cint, [vp, vp, sz, vp]),
             "mlem_memcpy_d2d": (cint, [vp, vp, sz, vp]),
@@ -140,6 +141,11 @@ def device_info(dev: int = 0):
     mem, cus = u64(), cint()
     _check(hip_lib().mlem_device_info(dev, name, 256, C.byref(mem), C.byref(cus)))
     return name.value.decode(), mem.value, cus.value
+
+
+def release_scratch(dev: int = 0):
+    """Gives back the device memory that set-up calls keep for the next matrix (mlem_release_scratch)."""
+    _check(hip_lib().mlem_release_scratch(dev))
 
 
 def device_sync():

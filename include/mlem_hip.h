@@ -58,6 +58,16 @@ int mlem_device_info(int device, char *name, size_t name_len,
                      uint64_t *total_mem, int *cu_count);
 int mlem_device_alloc(void **ptr, size_t bytes);
 int mlem_device_free(void *ptr);
+/* A program that sets up one matrix after another (from its third on) keeps
+ * the scratch of a set-up call (mlem_matrix_build_transpose, the tiles of
+ * mlem_recon_create) for the next one: one buffer per device of at most
+ * 8 GiB, and only while half of the device's memory is free.  No other
+ * figure of this library counts it.  It is given back when an allocation of
+ * the library finds the memory short, when a batch, a server's matrix or
+ * a tiles-only matrix has been created or mlem_autotune has run, and here:
+ * call it before another allocator of the process, or another process, needs
+ * the whole device. */
+int mlem_release_scratch(int device);
 int mlem_memcpy_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int mlem_memcpy_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int mlem_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);

@@ -241,17 +241,54 @@ int get_partition(mlem_matrix *m, int which, uint32_t secsize, const Partition *
     return MLEM_OK;
 }
 
+// Row slices for a plan that has been counted into `scratch` (quad tiles),
+// where they suit the matrix: *taken, t's memory and first steps then set up.
+// *unsuited: the matrix's layout is why not.  The quads' positions in
+// `scratch` are gone either way.
+static int take_slices(Tiled *t, void *scratch, DevBuf *wsteps, bool *taken, bool *unsuited) {
+    TilePlan &p = t->plan;
+    const size_t ns = slice_stream_count(p);
+    HIPCHK(wsteps->alloc(4 * (ns + 3)));
+    uint32_t fh[2] = {};
+    HIPCHK(launch_slice_count(p, tile_count_entries(p, scratch), tile_count_rowpos(p, scratch),
+                              wsteps->as<uint32_t>(), wsteps->as<uint32_t>() + ns, fh, nullptr));
+    std::vector<uint32_t> wb(ns + 1);
+    HIPCHK(hipMemcpy(wb.data(), wsteps->p, 4 * ns, hipMemcpyDeviceToHost));
+    uint64_t steps = 0;
+    *unsuited = fh[0] || !slice_prefix(p.W, &wb, &steps, &p.group) || !slices_suit(p, steps, fh[1]);
+    if (*unsuited) return MLEM_OK;
+    TilePlan q = p;
+    q.slices = true;
+    q.steps = steps;
+    q.most = fh[1];
+    q.cap = steps * 64 + 8;
+    const hipError_t e = t->mem.alloc(tiled_matrix_bytes(q));
+    if (e == hipErrorOutOfMemory) {  // the quads, which may be smaller
+        (void)hipGetLastError();
+        return MLEM_OK;
+    }
+    HIPCHK(e);
+    p = q;
+    t->view = tiled_matrix_view(p, t->mem.p);
+    HIPCHK(hipMemcpy(t->view.wbase, wb.data(), 4 * wb.size(), hipMemcpyHostToDevice));
+    *taken = true;
+    return MLEM_OK;
+}
+
 // Tiles of A (which 0) or A^T (which 1) with segment width W and R rows per
-// block, built on first use.  MLEM_ERR_UNSUPPORTED (and *flags) when the
-// matrix does not allow them (a row not sorted by column).  Quad tiles (the
-// batched layouts) of a matrix with a row order are built from A with its
-// rows in that order, and from that matrix's transpose for A^T.
-int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bool quad, const Tiled **out,
-              uint32_t *flags) {
+// block, built on first use; where row slices do not suit the matrix, Rq
+// rows (R, or the block streams' own default).  MLEM_ERR_UNSUPPORTED (and
+// *flags) when the matrix does not allow them (a row not sorted by column).
+// Quad tiles (the batched layouts) of a matrix with a row order are built
+// from A with its rows in that order, and from that matrix's transpose for
+// A^T.
+int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, uint32_t vt, bool quad,
+              const Tiled **out, uint32_t *flags) {
     std::lock_guard<std::mutex> lk(m->mu);
     const bool ordered = quad && m->has_order;
     auto key = std::make_tuple(which, W, R, vt, quad, ordered);
     *flags = 0;
+    if (R != Rq && m->unsliced.count(key)) std::get<2>(key) = R = Rq;
     auto it = m->tiles.find(key);
     if (it != m->tiles.end()) {
         *out = it->second.get();
@@ -343,7 +380,10 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
     }
     // The fill's scratch behind the count's where the kept scratch holds
     // both (its size is known after the count; the guess covers padding).
-    const size_t count_b = (tile_count_scratch_bytes(t->plan) + 255) & ~size_t(255);
+    TilePlan plan_q = tile_plan(nrow, ncol, m->nnz, W, Rq, vt, quad);
+    plan_q.unit_scale = t->plan.unit_scale;
+    const size_t count_b =
+        (std::max(tile_count_scratch_bytes(t->plan), tile_count_scratch_bytes(plan_q)) + 255) & ~size_t(255);
     Scratch scratch;
     if (!scratch.take_kept(m, count_b + m->nnz * (vt == VAL_F32 ? 5 : 7) + 4096)) HIPCHK(scratch.alloc(count_b));
     uint32_t fl = 0;
@@ -355,47 +395,37 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bo
                        R);
     }
     // Several right-hand sides: row slices where they suit the matrix.
-    if (slices_possible(t->plan)) {
-        const size_t ns = slice_stream_count(t->plan);
-        DevBuf wsteps;
-        HIPCHK(wsteps.alloc(4 * (ns + 3)));
-        uint32_t *flags = wsteps.as<uint32_t>() + ns, fh[2] = {};
-        HIPCHK(launch_slice_count(t->plan, tile_count_entries(t->plan, scratch.p), tile_count_rowpos(t->plan, scratch.p),
-                                  wsteps.as<uint32_t>(), flags, fh, nullptr));
-        std::vector<uint32_t> wb(ns + 1);
-        HIPCHK(hipMemcpy(wb.data(), wsteps.p, 4 * ns, hipMemcpyDeviceToHost));
-        uint64_t steps = 0;
-        const uint64_t quad_cap = t->plan.cap;
-        if (!fh[0] && slice_prefix(W, &wb, &steps, &t->plan.group) && slices_suit(t->plan, steps, fh[1])) {
-            t->plan.slices = true;
-            t->plan.steps = steps;
-            t->plan.cap = steps * 64 + 8;
-            const hipError_t e = t->mem.alloc(tiled_matrix_bytes(t->plan));
-            if (e == hipErrorOutOfMemory) {  // the quads, which may be smaller
-                (void)hipGetLastError();
-                t->plan.slices = false;
-                t->plan.steps = 0;
-                t->plan.cap = quad_cap;
-            } else {
-                HIPCHK(e);
-            }
+    DevBuf wsteps;
+    bool counted = true;  // the quads' positions are in place
+    for (bool unsuited = false; slices_possible(t->plan) && !t->plan.slices;) {
+        bool taken = false;
+        counted = false;
+        if (int st = take_slices(t.get(), scratch.p, &wsteps, &taken, &unsuited)) return st;
+        if (taken || R == Rq) break;
+        if (unsuited) m->unsliced.insert(key);
+        std::get<2>(key) = R = Rq;
+        if ((it = m->tiles.find(key)) != m->tiles.end()) {
+            *out = it->second.get();
+            return MLEM_OK;
         }
-        if (t->plan.slices) {
-            t->view = tiled_matrix_view(t->plan, t->mem.p);
-            HIPCHK(hipMemcpy(t->view.wbase, wb.data(), 4 * wb.size(), hipMemcpyHostToDevice));
-            DevBuf q;
-            HIPCHK(launch_fill_u32(flags, 0u, 1, nullptr));
-            if (vt != VAL_F32) {
-                HIPCHK(q.alloc(sizeof(uint16_t) * std::max<uint64_t>(1, m->nnz)));
-                HIPCHK(launch_row_codes(t->plan, rp, va, t->view.scale, q.as<uint16_t>(), flags, nullptr));
-            }
-            HIPCHK(launch_slice_clear(t->plan, t->view, nullptr));
-            HIPCHK(launch_slice_scatter(t->plan, rp, ci, va, q.as<uint16_t>(),
-                                        tile_count_rowpos(t->plan, scratch.p), t->view.wbase, t->view.tdata, nullptr));
-            HIPCHK(hipMemcpy(&fl, flags, 4, hipMemcpyDeviceToHost));
-        } else {  // the quads' positions again
-            HIPCHK(launch_tile_count(t->plan, rp, ci, scratch.p, &fl, nullptr));
+        t->plan = plan_q;
+        HIPCHK(launch_tile_count(t->plan, rp, ci, scratch.p, &fl, nullptr));
+        counted = true;
+    }
+    if (t->plan.slices) {
+        uint32_t *bad = wsteps.as<uint32_t>() + slice_stream_count(t->plan);
+        DevBuf q;
+        HIPCHK(launch_fill_u32(bad, 0u, 1, nullptr));
+        if (vt != VAL_F32) {
+            HIPCHK(q.alloc(sizeof(uint16_t) * std::max<uint64_t>(1, m->nnz)));
+            HIPCHK(launch_row_codes(t->plan, rp, va, t->view.scale, q.as<uint16_t>(), bad, nullptr));
         }
+        HIPCHK(launch_slice_clear(t->plan, t->view, nullptr));
+        HIPCHK(launch_slice_scatter(t->plan, rp, ci, va, q.as<uint16_t>(), tile_count_rowpos(t->plan, scratch.p),
+                                    t->view.wbase, t->view.tdata, nullptr));
+        HIPCHK(hipMemcpy(&fl, bad, 4, hipMemcpyDeviceToHost));
+    } else if (!counted) {
+        HIPCHK(launch_tile_count(t->plan, rp, ci, scratch.p, &fl, nullptr));
     }
     if (!t->plan.slices) {
         HIPCHK(t->mem.alloc(tiled_matrix_bytes(t->plan)));
@@ -493,7 +523,7 @@ int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev *
 // a work list of about `groups` runs (0: the default, one run per row block
 // where slices_direct says so) and the partial-sum
 // buffer for BC right-hand sides.  MLEM_ERR_UNSUPPORTED when the matrix or
-// the LDS does not allow the shape.
+// the LDS does not allow the shape.  R 0: the default rows.
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
                 const Tiled **tiled, const TileWorkDev **work, DevBuf *part) {
     *tiled = nullptr;
@@ -502,7 +532,14 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
         return set_err(MLEM_ERR_UNSUPPORTED, "no blocked kernel for width %u with %u right-hand sides", W, BC);
     uint32_t flags = 0;
     const Tiled *t = nullptr;
-    if (int st = get_tiled(m, which, W, R, vt, BC > 1, &t, &flags)) return st;
+    uint32_t Rq = R;
+    if (R == 0) {
+        const uint32_t rows = which ? m->cols : m->rows, cols = which ? m->rows : m->cols;
+        R = default_tile_rows(rows, cols, m->nnz, groups, vt, BC, true);
+        Rq = default_tile_rows(rows, cols, m->nnz, groups, vt, BC, false);
+    }
+    if (int st = get_tiled(m, which, W, R, Rq, vt, BC > 1, &t, &flags)) return st;
+    R = t->plan.R;
     int dev = 0, lds_max = 65536;
     if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
@@ -554,6 +591,16 @@ static uint32_t device_cus() {
 // block is then one run and needs no partial sums (slices_direct).  Eight
 // right-hand sides of 2048 rows leave one workgroup per CU (u = 163 at 8
 // runs per CU: 2798 / 4153).
+//   Block streams (matrices that row slices do not suit) keep three workgroups
+// per CU at 1024 rows and lose the third at 2048.  us per iteration, 1024 rows
+// x 8 per CU / 1024 x 4 / 2048 x 4, four right-hand sides, one pass and four:
+//   1.0e7 nonzeros (u = 2, A^T only)   f32    69 /   64 /   70    182 /  148 /  169
+//   1.35e8 (u = 32)                    f32   429 /  434 /  432   1631 / 1547 / 1601
+//                                   16-bit   344 /  373 /  399   1232 / 1192 / 1296
+//   6.8e8 (u = 162)                    f32  1983 / 1976 / 1972   7196 / 7254 / 7428
+//                                   16-bit  1552 / 1528 / 1663   5995 / 5945 / 6226
+// (The number of runs sets the order of the sums, so it does not follow the
+// number of passes: a slot's image is the same in any batch.)
 uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
     const uint32_t cus = device_cus();
     if (BC != 1) return (BC == 4 ? 4u : 8u) * cus;
@@ -561,11 +608,13 @@ uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC) {
     return (u >= 2 && u < (vt == VAL_F32 ? 40u : 24u) ? 12u : 24u) * cus;
 }
 
-uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC) {
-    const uint64_t target = groups ? groups : (BC == 1 ? 24u : BC == 4 ? 4u : 8u) * (uint64_t)device_cus();
+uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC,
+                           bool slices) {
+    const bool four = BC == 4 && slices;
+    const uint64_t target = groups ? groups : (BC == 1 ? 24u : four ? 4u : 8u) * (uint64_t)device_cus();
     const uint32_t W = BC == 8 ? 512u : 1024u;
-    if (BC != 1 && !groups && slices_direct(cols, W, 512, rows, nnz, BC)) return 512u;
-    if (BC == 4) return nnz < target * 48 * kTileUnit ? 1024u : 2048u;
+    if (BC != 1 && slices && !groups && slices_direct(cols, W, 512, rows, nnz, BC)) return 512u;
+    if (four) return nnz < target * 48 * kTileUnit ? 1024u : 2048u;
     if (nnz < target * 2 * kTileUnit) return 512u;
     if (BC != 1) return 1024u;
     return !groups && nnz < target * (vt == VAL_F32 ? 40u : 8u) * kTileUnit ? 1024u : 2048u;
@@ -581,8 +630,7 @@ int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t sec
     *work = nullptr;
     if (o.tile_width != 1) {
         const uint32_t W = o.tile_width == 0 ? 1024u : o.tile_width;
-        const uint32_t R = o.tile_rows == 0 ? default_tile_rows(m->rows, m->cols, m->nnz, o.tile_groups, o.values, 1) : o.tile_rows;
-        const int st = setup_tiled(m, which, W, R, o.values, 1, o.tile_groups, tiled, work, part);
+        const int st = setup_tiled(m, which, W, o.tile_rows, o.values, 1, o.tile_groups, tiled, work, part);
         if (st == MLEM_OK || m->tiles_only) return st;
         // Automatic width with f32 values: a matrix the tiles do not suit, or
         // whose tiles do not fit beside the resident copies (the 100 GB
@@ -1248,6 +1296,7 @@ int mlem_matrix_build_transpose_limited(mlem_matrix *m, uint64_t scratch_bytes, 
         it = it->first.first == 1 ? m->parts.erase(it) : std::next(it);
     for (auto it = m->tiles.begin(); it != m->tiles.end();)
         it = std::get<0>(it->first) == 1 ? m->tiles.erase(it) : std::next(it);
+    m->unsliced.clear();
     for (auto it = m->tile_refused.begin(); it != m->tile_refused.end();)
         it = std::get<0>(it->first) == 1 ? m->tile_refused.erase(it) : std::next(it);
     return MLEM_OK;
@@ -1274,6 +1323,7 @@ int mlem_matrix_set_row_order(mlem_matrix *m, const uint32_t *order) {
     std::lock_guard<std::mutex> lk(m->mu);
     for (auto it = m->tiles.begin(); it != m->tiles.end();)  // tiles built in the previous order
         it = std::get<5>(it->first) ? m->tiles.erase(it) : std::next(it);
+    m->unsliced.clear();
     for (auto it = m->tile_refused.begin(); it != m->tile_refused.end();)
         it = std::get<5>(it->first) ? m->tile_refused.erase(it) : std::next(it);
     std::swap(m->row_order.p, buf.p);

@@ -212,6 +212,7 @@ struct mlem_matrix {
     using TileKey = std::tuple<int, uint32_t, uint32_t, uint32_t, bool, bool>;
     std::map<TileKey, std::unique_ptr<Tiled>> tiles;
     std::map<TileKey, uint32_t> tile_refused;  // build flags of refused tilings
+    std::set<TileKey> unsliced;                // shapes that row slices were found not to suit
     // Reconstructions and batches alive on this matrix: they hold its arrays,
     // tiles and work lists by address, so the transpose is not rebuilt and
     // the matrix is not destroyed while any exists.
@@ -303,12 +304,12 @@ namespace abi {
 int get_partition(mlem_matrix *m, int which, uint32_t secsize, const Partition **out);
 // Tiles of A or A^T, built on first use from the resident CSR (a
 // tiles-only matrix has only the ones it was built with).
-int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, bool quad, const Tiled **out,
-              uint32_t *flags);
+int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, uint32_t vt, bool quad,
+              const Tiled **out, uint32_t *flags);
 // Work list of t for about `target` workgroups, built on first use.
 int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev **out);
 // Tiles, work list and partial-sum buffer (part null: none) of one side for
-// BC right-hand sides.
+// BC right-hand sides (R 0: default_tile_rows).
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
                 const Tiled **tiled, const TileWorkDev **work, DevBuf *part);
 // The blocked or the plain merge path for one side of a reconstruction.
@@ -318,9 +319,10 @@ int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t sec
 int sens_on_device(const mlem_matrix *m, float *s32, double *s64_or_null, hipStream_t s);
 // Runs (workgroups) per blocked SpMV and rows per tile block for BC
 // right-hand sides and `vt` values when none are asked for, on the current
-// device (groups 0: the default runs).
+// device (groups 0: the default runs; slices: for tiles that are row slices).
 uint32_t default_tile_groups(uint64_t nnz, uint32_t vt, uint32_t BC);
-uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC);
+uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t groups, uint32_t vt, uint32_t BC,
+                           bool slices);
 // Batch slots without waiting on the host (the serving loop): the set
 // copies g (rows) and f0 (cols) in and marks the slot active, allocating its
 // pass if that is the first slot set in it (*allocated = bytes allocated,

@@ -337,19 +337,14 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
         o.values = m->tile_vt;
     }
     // Widths: 1024, 512 for 8 per pass (whose x of 1024 columns would leave
-    // one workgroup per CU); rows: default_tile_rows, for FP and BP by itself.
+    // one workgroup per CU); default rows: setup_tiled, for FP and BP by itself.
     const uint32_t W = o.tile_width ? o.tile_width : (BC == 8 ? 512u : 1024u);
     ARGCHK(valid_tile_config(W, BC), "mlem_batch_create: no blocked kernel for width %u with %u per pass", W, BC);
     ARGCHK(o.tile_rows == 0 || valid_tile_rows(o.tile_rows),
            "mlem_batch_create: tile_rows must be 512 ... 16384 (a power of two)");
     ARGCHK(valid_stream_threads(o.tile_threads), "mlem_batch_create: tile_threads must be 0, 128, 256 or 512");
     HIPCHK(hipSetDevice(m->device));
-    auto side_rows = [&](int which) {
-        if (m->tiles_only) return m->tile_R[which];
-        if (o.tile_rows) return o.tile_rows;
-        return which ? default_tile_rows(m->cols, m->rows, m->nnz, o.tile_groups, o.values, BC)
-                     : default_tile_rows(m->rows, m->cols, m->nnz, o.tile_groups, o.values, BC);
-    };
+    auto side_rows = [&](int which) { return m->tiles_only ? m->tile_R[which] : o.tile_rows; };
     auto b = std::make_unique<mlem_batch>();
     b->m = m;
     b->slots = slots;
@@ -453,6 +448,21 @@ int mlem_batch_info(const mlem_batch *b, uint32_t *slots, uint32_t *per_pass, ui
     if (per_pass) *per_pass = b->BC;
     if (passes) *passes = b->passes;
     if (device_bytes) *device_bytes = b->device_bytes();
+    return MLEM_OK;
+}
+
+int mlem_batch_layout(const mlem_batch *b, int side, mlem_tile_layout *out) {
+    ARGCHK(b && out && (side == 0 || side == 1), "mlem_batch_layout: null argument or a side that is not 0 or 1");
+    const Tiled *t = side ? b->tbp : b->tfp;
+    const TileWorkDev *w = side ? b->wbp : b->wfp;
+    const TilePlan &p = t->plan;
+    out->kind = !p.quad ? 0u : !p.slices ? 1u : w->view.direct ? 3u : 2u;
+    out->tile_width = p.W;
+    out->tile_rows = p.R;
+    out->runs = w->view.nwg;
+    out->max_steps = p.slices ? p.most : 0u;
+    out->entries = p.cap - 8;
+    out->bytes = t->mem.bytes;
     return MLEM_OK;
 }
 

@@ -154,6 +154,7 @@ struct TilePlan {
     bool slices = false;
     uint64_t steps = 0;
     uint32_t group = 1;  // steps taken together
+    uint32_t most = 0;   // steps of the longest stream of a tile (before whole groups)
     uint32_t vb() const { return vt == VAL_F32 ? 4u : 2u; }  // bytes per stored value
 };
 struct TiledMatrix {

@@ -18,11 +18,12 @@ namespace {
 // the choice of row slices is made from the whole matrix's counts).
 struct ChunkedTiles {
     TilePlan P;
-    std::vector<uint64_t> size;   // padded entries per tile, then (allocate) offsets
+    std::vector<uint64_t> size;   // padded entries per tile, then (lay_out) offsets
     std::vector<uint32_t> nz;     // entries per tile
-    std::vector<uint32_t> wbase;  // row slices: steps per (row block, stream, segment), then (allocate) first steps
+    std::vector<uint32_t> wbase;  // row slices: steps per (row block, stream, segment), then (lay_out) first steps
     uint32_t most = 0;            // the most steps of a stream in a tile
-    bool slices;                  // still possible; from allocate() on: taken
+    bool slices;                  // still possible; from lay_out() on: suit; from allocate() on: taken
+    uint64_t quad_cap = 0;        // entries of the quads, whatever the layout
     Tiled *t = nullptr;
 
     ChunkedTiles(const TilePlan &p, Tiled *tiled)
@@ -76,27 +77,32 @@ struct ChunkedTiles {
         return MLEM_OK;
     }
 
-    int allocate() {
+    // After the counts: the offsets, and whether row slices suit the matrix.
+    void lay_out() {
         uint64_t run = 0;
         for (uint64_t i = 0; i <= P.ntiles; ++i) {
             const uint64_t n = i < P.ntiles ? size[i] : 0;
             size[i] = run;
             run += n;
         }
-        P.cap = run + 8;  // as one build: a multiple of 8, at least one group
+        quad_cap = P.cap = run + 8;  // as one build: a multiple of 8, at least one group
         uint64_t steps = 0;
         slices = slices && slice_prefix(P.W, &wbase, &steps, &P.group) && slices_suit(P, steps, most);
         if (slices) {
             P.slices = true;
             P.steps = steps;
+            P.most = most;
             P.cap = steps * 64 + 8;
         }
+    }
+
+    int allocate() {
         hipError_t e = t->mem.alloc(tiled_matrix_bytes(P));
         if (e == hipErrorOutOfMemory && slices) {  // the quads, which may be smaller
             (void)hipGetLastError();
             slices = P.slices = false;
             P.steps = 0;
-            P.cap = run + 8;
+            P.cap = quad_cap;
             e = t->mem.alloc(tiled_matrix_bytes(P));
         }
         HIPCHK(e);
@@ -173,8 +179,11 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     ARGCHK(values <= VAL_UF16, "mlem_matrix_create_tiled: values must be 0 (f32), 1 (bf16), 2 (fp16) or 3 (uf16)");
     HIPCHK(hipSetDevice(device));
     // as a reconstruction over the resident CSR would choose
-    const uint32_t R = tile_rows ? tile_rows : default_tile_rows(rows, cols, nnz, 0, values, BC),
-                   RT = tile_rows ? tile_rows : default_tile_rows(cols, rows, nnz, 0, values, BC);
+    auto rows_for = [&](uint32_t nrow, uint32_t ncol, bool slices) {
+        return tile_rows ? tile_rows : default_tile_rows(nrow, ncol, nnz, 0, values, BC, slices);
+    };
+    uint32_t R = rows_for(rows, cols, true), RT = rows_for(cols, rows, true);
+    const uint32_t Rq = rows_for(rows, cols, false), RTq = rows_for(cols, rows, false);  // without row slices
     auto m = std::make_unique<mlem_matrix>();
     m->device = device;
     m->rows = rows;
@@ -182,8 +191,6 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     m->nnz = nnz;
     m->tiles_only = true;
     m->tile_W = W;
-    m->tile_R[0] = R;
-    m->tile_R[1] = RT;
     m->tile_vt = values;
     m->tile_bc = BC;
     const size_t margin = (size_t)1 << 30;
@@ -233,6 +240,15 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             if (fl & 8u)
                 return set_err(MLEM_ERR_INVALID_ARGUMENT, "uf16 values need a matrix without negative values");
         }
+        // The block streams' rows, counted again: where row slices turn out
+        // not to suit.
+        auto other_rows = [&]() {
+            RT = RTq;
+            pT = tile_plan(cols, rows, nnz, W, RT, values, quad);
+            pT.unit_scale = values != VAL_F32;
+            bT = ChunkedTiles(pT, tT.get());
+            return -1;  // the pass before the first
+        };
         for (int pass = 0; pass < 2; ++pass) {
             if (pass == 1)
                 if (int st = bT.allocate()) return st;
@@ -270,12 +286,21 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             HIPCHK(e);
             progress("A^T tiles %s over %u column ranges (%.1f GB of range scratch)", pass ? "filled" : "counted", nr,
                      budget / 2 / 1e9);
+            if (pass == 0) {
+                bT.lay_out();
+                if (!bT.slices && RT != RTq) pass = other_rows();
+            }
         }
         HIPCHK(hipDeviceSynchronize());
     }
     // A's tiles from row chunks of the host CSR (A's device copy is gone),
     // whole row blocks whose CSR and tiling scratch fit.
     const uint64_t nseg = bA.P.nseg;
+    auto other_rows = [&]() {  // as for A^T
+        R = Rq;
+        bA = ChunkedTiles(tile_plan(rows, cols, nnz, W, R, values, quad), tA.get());
+        return -1;
+    };
     progress("A^T tiles %.1f GB; A's device copy freed", tT->mem.bytes / 1e9);
     for (int pass = 0; pass < 2; ++pass) {
         if (pass == 1)
@@ -332,6 +357,10 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
         }
         progress("A tiles %s over %u row chunks (%u smaller after a failed allocation; %.1f GB of chunk scratch)",
                  pass ? "filled" : "counted", chunks, retries, budget / 1e9);
+        if (pass == 0) {
+            bA.lay_out();
+            if (!bA.slices && R != Rq) pass = other_rows();
+        }
     }
     HIPCHK(hipDeviceSynchronize());
     progress("A tiles %.1f GB", tA->mem.bytes / 1e9);
@@ -342,6 +371,8 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     m->tiles.emplace(std::make_tuple(0, W, R, values, quad, false), std::move(tA));
     m->tiles.emplace(std::make_tuple(1, W, RT, values, quad, false), std::move(tT));
     (void)scratch_trim();
+    m->tile_R[0] = R;
+    m->tile_R[1] = RT;
     *out = m.release();
     return MLEM_OK;
 }

@@ -85,6 +85,7 @@ def hip_lib() -> C.CDLL:
             "mlem_batch_sync": (cint, [vp]),
             "mlem_batch_get_image": (cint, [vp, u32, vp]),
             "mlem_batch_info": (cint, [vp, P(u32), P(u32), P(u32), P(u64)]),
+            "mlem_batch_layout": (cint, [vp, cint, vp]),
             "mlem_batch_stream": (vp, [vp]),
             "mlem_batch_destroy": (cint, [vp]),
             "mlem_server_create": (cint, [u64, vp, P(vp)]),
@@ -366,6 +367,11 @@ class BatchOpts(C.Structure):
                 ("tile_threads", u32), ("use_graph", u32)]
 
 
+class TileLayout(C.Structure):
+    _fields_ = [("kind", u32), ("tile_width", u32), ("tile_rows", u32), ("runs", u32), ("max_steps", u32),
+                ("entries", u64), ("bytes", u64)]
+
+
 class Batch:
     """Many reconstructions over one resident matrix (A and A^T), iterated together (mlem_batch_*)."""
 
@@ -402,6 +408,14 @@ class Batch:
         a, b, c, d = u32(), u32(), u32(), u64()
         _check(hip_lib().mlem_batch_info(self.h, C.byref(a), C.byref(b), C.byref(c), C.byref(d)))
         return dict(slots=a.value, per_pass=b.value, passes=c.value, device_bytes=d.value)
+
+    LAYOUTS = ("row steps", "block streams", "row slices", "row slices, one run per row block")
+
+    def layout(self, side: int) -> dict:
+        """How A (side 0) or A^T (side 1) is kept (mlem_batch_layout)."""
+        t = TileLayout()
+        _check(hip_lib().mlem_batch_layout(self.h, side, C.byref(t)))
+        return dict(kind=self.LAYOUTS[t.kind], **{k: getattr(t, k) for k, _ in TileLayout._fields_[1:]})
 
     def close(self):
         if self.h:

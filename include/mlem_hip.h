@@ -425,6 +425,20 @@ int mlem_batch_sync(mlem_batch *b);
 int mlem_batch_get_image(mlem_batch *b, uint32_t slot, float *f_out);
 int mlem_batch_info(const mlem_batch *b, uint32_t *slots, uint32_t *per_pass,
                     uint32_t *passes, uint64_t *device_bytes);
+/* How the batch keeps A (side 0, forward projection) or A^T (side 1, back
+ * projection): what the automatic shape and the matrix led to. */
+typedef struct mlem_tile_layout {
+    uint32_t kind;       /* 0 = row steps (1 per pass), 1 = block streams,
+                            2 = row slices, 3 = row slices, each row block
+                            one run (no partial sums)                      */
+    uint32_t tile_width, tile_rows;
+    uint32_t runs;       /* workgroups per pass                            */
+    uint32_t max_steps;  /* row slices: 64-entry steps of the longest
+                            stream in a tile, else 0                       */
+    uint64_t entries;    /* stored, padding included                       */
+    uint64_t bytes;      /* of the tiles                                   */
+} mlem_tile_layout;
+int mlem_batch_layout(const mlem_batch *b, int side, mlem_tile_layout *out);
 void *mlem_batch_stream(mlem_batch *b);
 int mlem_batch_destroy(mlem_batch *b);
 

@@ -241,9 +241,10 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
                 return set_err(MLEM_ERR_INVALID_ARGUMENT, "uf16 values need a matrix without negative values");
         }
         // The block streams' rows, counted again: where row slices turn out
-        // not to suit.
+        // not to suit, or the scratch holds no block of the slices' rows.
         auto other_rows = [&]() {
             RT = RTq;
+            tT->mem.reset();
             pT = tile_plan(cols, rows, nnz, W, RT, values, quad);
             pT.unit_scale = values != VAL_F32;
             bT = ChunkedTiles(pT, tT.get());
@@ -280,6 +281,11 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             const hipError_t e = transpose_ranges_to(rows, cols, nnz, rp.as<uint64_t>(), ci.as<uint32_t>(),
                                                      va.as<float>(), colptrT.as<uint64_t>(), nullptr, nullptr,
                                                      budget / 2, RT, sink, &nr, nullptr);
+            if ((e == hipErrorOutOfMemory || st_sink == MLEM_ERR_OUT_OF_MEMORY) && RT > RTq) {
+                (void)hipGetLastError();
+                pass = other_rows();
+                continue;
+            }
             if (st_sink != MLEM_OK) return st_sink;
             if (e == hipErrorOutOfMemory)
                 return set_err(MLEM_ERR_OUT_OF_MEMORY, "mlem_matrix_create_tiled: %u rows of A^T do not fit", RT);
@@ -298,6 +304,7 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     const uint64_t nseg = bA.P.nseg;
     auto other_rows = [&]() {  // as for A^T
         R = Rq;
+        tA->mem.reset();
         bA = ChunkedTiles(tile_plan(rows, cols, nnz, W, R, values, quad), tA.get());
         return -1;
     };
@@ -335,7 +342,8 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             if (pass == 0) return bA.count(r0, rc, n, rp.as<uint64_t>(), ci.as<uint32_t>());
             return bA.fill(r0, rc, n, rp.as<uint64_t>(), ci.as<uint32_t>(), va.as<float>());
         };
-        for (uint32_t r0 = 0; r0 < rows; ++chunks) {
+        bool again = false;
+        for (uint32_t r0 = 0; r0 < rows && !again; ++chunks) {
             uint32_t r1 = std::min<uint64_t>((uint64_t)r0 + R, rows);
             while (r1 < rows) {
                 const uint32_t nx = (uint32_t)std::min<uint64_t>((uint64_t)r1 + R, rows);
@@ -348,12 +356,18 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
                 const int st = chunk(r0, r1);
                 if (st == MLEM_OK) break;
                 const uint32_t blocks = (r1 - r0 + R - 1) / R;
+                again = st == MLEM_ERR_OUT_OF_MEMORY && blocks < 2 && R > Rq;
+                if (again) break;
                 if (st != MLEM_ERR_OUT_OF_MEMORY || blocks < 2) return st;
                 (void)hipGetLastError();
                 r1 = r0 + (blocks / 2) * R;
                 ++retries;
             }
             r0 = r1;
+        }
+        if (again) {
+            pass = other_rows();
+            continue;
         }
         progress("A tiles %s over %u row chunks (%u smaller after a failed allocation; %.1f GB of chunk scratch)",
                  pass ? "filled" : "counted", chunks, retries, budget / 1e9);

@@ -620,6 +620,11 @@ uint32_t default_tile_rows(uint32_t rows, uint32_t cols, uint64_t nnz, uint32_t 
     return !groups && nnz < target * (vt == VAL_F32 ? 40u : 8u) * kTileUnit ? 1024u : 2048u;
 }
 
+uint32_t automatic_rows_name(uint64_t nnz, uint32_t BC) {
+    if (nnz < (BC == 1 ? 24u : 8u) * (uint64_t)device_cus() * 2 * kTileUnit) return 512u;
+    return BC == 1 ? 2048u : 1024u;
+}
+
 // Chooses the blocked (LDS-tiled) or the plain merge path for one side of
 // the iteration.  The blocked path (default_tile_rows x 1024 columns) runs
 // about tile_groups workgroups (0: default_tile_groups); secsize applies to
@@ -1412,7 +1417,7 @@ int mlem_recon_create(const mlem_matrix *mc, const int32_t *g, const float *sens
         ARGCHK(o.spmv == 0 && o.using_trans == 0 && o.bp_spmv <= 1,
                "mlem_recon_create: a tiles-only matrix takes merge-based FP and BP on A^T");
         ARGCHK(m->tile_bc == 1, "mlem_recon_create: the matrix holds the tiles of batches of %u per pass", m->tile_bc);
-        ARGCHK((o.tile_width == 0 || o.tile_width == m->tile_W) && (o.tile_rows == 0 || o.tile_rows == m->tile_R[0]) &&
+        ARGCHK((o.tile_width == 0 || o.tile_width == m->tile_W) && m->takes_rows(o.tile_rows) &&
                    (o.values == 0 || o.values == m->tile_vt),
                "mlem_recon_create: the matrix holds tiles of width %u and %u rows with values %u", m->tile_W,
                m->tile_R[0], m->tile_vt);

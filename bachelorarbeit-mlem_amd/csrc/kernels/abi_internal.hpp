@@ -200,6 +200,11 @@ struct mlem_matrix {
     // sensitivity taken while they were built.
     bool tiles_only = false;
     uint32_t tile_W = 0, tile_R[2] = {}, tile_vt = 0, tile_bc = 1;  // tile_bc: right-hand sides per pass
+    uint32_t tile_auto = 0;  // rows chosen automatically: the rows that stand for them (0: they were asked for)
+    // Whether a reconstruction or batch may ask for these rows.
+    bool takes_rows(uint32_t rows) const {
+        return rows == 0 || (rows == tile_R[0] && rows == tile_R[1]) || (tile_auto && rows == tile_auto);
+    }
     mlem::abi::DevBuf sens32, sens64;
     // Row order for the batched (quad) tiles: row_order[i] = place of row i
     // of A (mlem_matrix_set_row_order); has_order false: A's own order.
@@ -315,6 +320,9 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
 // The blocked or the plain merge path for one side of a reconstruction.
 int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t secsize, const Tiled **tiled,
                      const TileWorkDev **work, DevBuf *part, const Partition **partn, DevBuf *scratch);
+// The rows that name the automatic shape of a tiles-only matrix, whatever it
+// is (mlem_matrix_create_tiled).
+uint32_t automatic_rows_name(uint64_t nnz, uint32_t BC);
 // FP64 column sums of A (s32 and s64 may be null).
 int sens_on_device(const mlem_matrix *m, float *s32, double *s64_or_null, hipStream_t s);
 // Runs (workgroups) per blocked SpMV and rows per tile block for BC

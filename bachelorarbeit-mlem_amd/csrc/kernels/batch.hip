@@ -329,10 +329,11 @@ int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opt
     ARGCHK(m->has_T || m->tiles_only, "mlem_batch_create: the transpose must be resident (upload it or build it)");
     if (m->tiles_only) {
         ARGCHK(BC == m->tile_bc && (o.tile_width == 0 || o.tile_width == m->tile_W) &&
-                   (o.tile_rows == 0 || o.tile_rows == m->tile_R[0] || o.tile_rows == m->tile_R[1]) &&
+                   m->takes_rows(o.tile_rows) &&
                    (o.values == 0 || o.values == m->tile_vt),
-               "mlem_batch_create: the matrix holds tiles of width %u and %u rows with values %u for %u per pass",
-               m->tile_W, m->tile_R[0], m->tile_vt, m->tile_bc);
+               "mlem_batch_create: the matrix holds tiles of width %u and %u (A) and %u (A^T) rows with values %u for "
+               "%u per pass",
+               m->tile_W, m->tile_R[0], m->tile_R[1], m->tile_vt, m->tile_bc);
         o.tile_width = m->tile_W;
         o.values = m->tile_vt;
     }

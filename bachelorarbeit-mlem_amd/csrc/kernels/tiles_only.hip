@@ -387,6 +387,7 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     (void)scratch_trim();
     m->tile_R[0] = R;
     m->tile_R[1] = RT;
+    m->tile_auto = tile_rows ? 0 : automatic_rows_name(nnz, BC);
     *out = m.release();
     return MLEM_OK;
 }

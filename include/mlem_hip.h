@@ -298,7 +298,10 @@ int mlem_matrix_set_row_order(mlem_matrix *m, const uint32_t *order);
  * resident path.  chunk_bytes bounds the scratch of each range / chunk
  * (0 = what is free).  A reconstruction on it (per_pass 1) takes merge-based
  * FP and BP on A^T (spmv 0, using_trans 0) with the matrix's tile shape and
- * values, a batch (per_pass 4 or 8) the matrix's per_pass, shape and values;
+ * values, a batch (per_pass 4 or 8) the matrix's per_pass, shape and values
+ * (tile_rows 0, or the rows given here; where they were 0, and the sides may
+ * differ, 512 for nnz < 2 x 2048 x 24 per CU (batches: 8 per CU), else 2048
+ * (batches: 1024) stand for the automatic rows);
  * the plain kernels, batches, the autotuner and the transpose calls refuse
  * it.  MLEM_ERR_OUT_OF_MEMORY when the tiles or one row block's scratch do
  * not fit. */

@@ -242,10 +242,10 @@ int get_partition(mlem_matrix *m, int which, uint32_t secsize, const Partition *
 }
 
 // Row slices for a plan that has been counted into `scratch` (quad tiles),
-// where they suit the matrix: *taken, t's memory and first steps then set up.
-// *unsuited: the matrix's layout is why not.  The quads' positions in
-// `scratch` are gone either way.
-static int take_slices(Tiled *t, void *scratch, DevBuf *wsteps, bool *taken, bool *unsuited) {
+// where they suit the matrix and `use` allows it: *taken, t's memory and first
+// steps then set up.  *unsuited: the matrix's layout is why not.  The quads'
+// positions in `scratch` are gone either way.
+static int take_slices(Tiled *t, void *scratch, SliceUse use, DevBuf *wsteps, bool *taken, bool *unsuited) {
     TilePlan &p = t->plan;
     const size_t ns = slice_stream_count(p);
     HIPCHK(wsteps->alloc(4 * (ns + 3)));
@@ -262,13 +262,11 @@ static int take_slices(Tiled *t, void *scratch, DevBuf *wsteps, bool *taken, boo
     q.steps = steps;
     q.most = fh[1];
     q.cap = steps * 64 + 8;
-    const hipError_t e = t->mem.alloc(tiled_matrix_bytes(q));
-    if (e == hipErrorOutOfMemory) {  // the quads, which may be smaller
-        (void)hipGetLastError();
-        return MLEM_OK;
-    }
-    HIPCHK(e);
+    const bool larger = tiled_matrix_bytes(q) > tiled_matrix_bytes(p);
+    if (larger && use == SliceUse::kNotLarger) return MLEM_OK;
+    HIPCHK(t->mem.alloc(tiled_matrix_bytes(q)));
     p = q;
+    t->larger = larger;
     t->view = tiled_matrix_view(p, t->mem.p);
     HIPCHK(hipMemcpy(t->view.wbase, wb.data(), 4 * wb.size(), hipMemcpyHostToDevice));
     *taken = true;
@@ -282,7 +280,7 @@ static int take_slices(Tiled *t, void *scratch, DevBuf *wsteps, bool *taken, boo
 // Quad tiles (the batched layouts) of a matrix with a row order are built
 // from A with its rows in that order, and from that matrix's transpose for
 // A^T.
-int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, uint32_t vt, bool quad,
+int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, uint32_t vt, bool quad, SliceUse use,
               const Tiled **out, uint32_t *flags) {
     std::lock_guard<std::mutex> lk(m->mu);
     const bool ordered = quad && m->has_order;
@@ -400,7 +398,7 @@ int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, ui
     for (bool unsuited = false; slices_possible(t->plan) && !t->plan.slices;) {
         bool taken = false;
         counted = false;
-        if (int st = take_slices(t.get(), scratch.p, &wsteps, &taken, &unsuited)) return st;
+        if (int st = take_slices(t.get(), scratch.p, use, &wsteps, &taken, &unsuited)) return st;
         if (taken || R == Rq) break;
         if (unsuited) m->unsliced.insert(key);
         std::get<2>(key) = R = Rq;
@@ -525,7 +523,7 @@ int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev *
 // buffer for BC right-hand sides.  MLEM_ERR_UNSUPPORTED when the matrix or
 // the LDS does not allow the shape.  R 0: the default rows.
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
-                const Tiled **tiled, const TileWorkDev **work, DevBuf *part) {
+                SliceUse use, const Tiled **tiled, const TileWorkDev **work, DevBuf *part) {
     *tiled = nullptr;
     *work = nullptr;
     if (!valid_tile_config(W, BC))
@@ -538,7 +536,7 @@ int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, 
         R = default_tile_rows(rows, cols, m->nnz, groups, vt, BC, true);
         Rq = default_tile_rows(rows, cols, m->nnz, groups, vt, BC, false);
     }
-    if (int st = get_tiled(m, which, W, R, Rq, vt, BC > 1, &t, &flags)) return st;
+    if (int st = get_tiled(m, which, W, R, Rq, vt, BC > 1, use, &t, &flags)) return st;
     R = t->plan.R;
     int dev = 0, lds_max = 65536;
     if (hipGetDevice(&dev) == hipSuccess)
@@ -635,7 +633,8 @@ int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t sec
     *work = nullptr;
     if (o.tile_width != 1) {
         const uint32_t W = o.tile_width == 0 ? 1024u : o.tile_width;
-        const int st = setup_tiled(m, which, W, o.tile_rows, o.values, 1, o.tile_groups, tiled, work, part);
+        const int st = setup_tiled(m, which, W, o.tile_rows, o.values, 1, o.tile_groups, SliceUse::kAny, tiled, work,
+                                   part);
         if (st == MLEM_OK || m->tiles_only) return st;
         // Automatic width with f32 values: a matrix the tiles do not suit, or
         // whose tiles do not fit beside the resident copies (the 100 GB

@@ -180,6 +180,7 @@ struct Tiled {
     mlem::TiledMatrix view;
     mlem::abi::DevBuf sens;  // A^T tiles of 16-bit values: the quantized matrix's column sums (f32)
     bool ordered = false;    // built with A's rows in the matrix's row order (mlem_matrix_set_row_order)
+    bool larger = false;     // row slices that take more memory than the quads
     std::map<uint32_t, std::unique_ptr<TileWorkDev>> works;  // by target workgroup count
 };
 
@@ -198,6 +199,7 @@ struct mlem_matrix {
     // Tiles only (mlem_matrix_create_tiled): no CSR copies on the device, the
     // tiles of A and A^T (width tile_W, tile_R[0] and [1] rows) and the
     // sensitivity taken while they were built.
+    std::mutex build_mu;  // held while a batch takes its tiles, or the autotuner its candidates
     bool tiles_only = false;
     uint32_t tile_W = 0, tile_R[2] = {}, tile_vt = 0, tile_bc = 1;  // tile_bc: right-hand sides per pass
     uint32_t tile_auto = 0;  // rows chosen automatically: the rows that stand for them (0: they were asked for)
@@ -307,16 +309,19 @@ namespace abi {
 
 // Merge-path partition of A (which 0) or A^T (1) for secsize, built on first use.
 int get_partition(mlem_matrix *m, int which, uint32_t secsize, const Partition **out);
+// Row slices where they suit the matrix, or only where they take no more
+// memory than the quads (they may take a quarter more).
+enum class SliceUse { kAny, kNotLarger };
 // Tiles of A or A^T, built on first use from the resident CSR (a
 // tiles-only matrix has only the ones it was built with).
-int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, uint32_t vt, bool quad,
+int get_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t Rq, uint32_t vt, bool quad, SliceUse use,
               const Tiled **out, uint32_t *flags);
 // Work list of t for about `target` workgroups, built on first use.
 int get_tile_work(mlem_matrix *m, Tiled *t, uint32_t target, const TileWorkDev **out);
 // Tiles, work list and partial-sum buffer (part null: none) of one side for
 // BC right-hand sides (R 0: default_tile_rows).
 int setup_tiled(mlem_matrix *m, int which, uint32_t W, uint32_t R, uint32_t vt, uint32_t BC, uint32_t groups,
-                const Tiled **tiled, const TileWorkDev **work, DevBuf *part);
+                SliceUse use, const Tiled **tiled, const TileWorkDev **work, DevBuf *part);
 // The blocked or the plain merge path for one side of a reconstruction.
 int setup_merge_side(mlem_matrix *m, int which, const mlem_opts &o, uint32_t secsize, const Tiled **tiled,
                      const TileWorkDev **work, DevBuf *part, const Partition **partn, DevBuf *scratch);
@@ -345,6 +350,9 @@ int batch_deactivate_async(mlem_batch *b, uint32_t slot);
 // stream, the flags swapped.  A slot's arithmetic does not depend on its
 // place, so the images are bitwise those it would have had in `from`.
 int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to);
+// mlem_batch_create under a server's budget (0: none): the bytes left of it
+// for the matrix, the batch and its passes.
+int batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opts, uint64_t budget, mlem_batch **out);
 // The partial-sum buffer for up to `passes` passes per launch (at most
 // kMaxPasses), fewer where the memory for them is not free.
 int batch_alloc_part(mlem_batch *b, uint32_t passes);

@@ -132,6 +132,121 @@ int batch_alloc_part(mlem_batch *b, uint32_t passes) {
     }
 }
 
+// The batch's tiles, work lists and partial sums.  Row slices may take more
+// memory than the quads: where the batch would then find no room (in the
+// budget, or on the device for all its passes) for what it holds with the
+// quads, the larger ones built here are dropped and quads built instead.
+static int batch_take_tiles(mlem_batch *b, uint32_t W, const uint32_t rows[2], const mlem_batch_opts &o,
+                            uint64_t budget) {
+    mlem_matrix *m = b->m;
+    std::lock_guard<std::mutex> building(m->build_mu);
+    std::set<mlem_matrix::TileKey> before;
+    {
+        std::lock_guard<std::mutex> lk(m->mu);
+        for (const auto &t : m->tiles) before.insert(t.first);
+    }
+    auto build = [&](SliceUse use) -> int {
+        if (int st = setup_tiled(m, 0, W, rows[0], o.values, b->BC, o.tile_groups, use, &b->tfp, &b->wfp, nullptr))
+            return st;
+        if (int st = setup_tiled(m, 1, W, rows[1], o.values, b->BC, o.tile_groups, use, &b->tbp, &b->wbp, nullptr))
+            return st;
+        return batch_alloc_part(b, b->passes);
+    };
+    auto room = [&]() -> bool {
+        const uint64_t more = (uint64_t)b->passes * b->pass_bytes() + sizeof(float) * m->cols +
+                              sizeof(uint32_t) * (uint64_t)b->passes * b->BC +
+                              sizeof(float) * std::max<uint64_t>(m->rows, m->cols);
+        if (!budget) {
+            size_t free_b = 0;
+            return free_device_bytes(&free_b) != hipSuccess || more <= free_b;
+        }
+        uint64_t held = 0;
+        (void)mlem_matrix_info(m, nullptr, nullptr, nullptr, nullptr, &held);
+        return held + b->part.bytes + more <= budget;
+    };
+    const int st = build(SliceUse::kAny);
+    if (b->BC == 1 || m->tiles_only || (st != MLEM_OK && st != MLEM_ERR_OUT_OF_MEMORY)) return st;
+    if (st == MLEM_OK) {
+        bool larger = false;
+        {
+            std::lock_guard<std::mutex> lk(m->mu);
+            for (const auto &t : m->tiles) larger = larger || (t.second->larger && !before.count(t.first));
+        }
+        if (!larger || room()) return MLEM_OK;
+    }
+    b->part.reset();
+    {
+        std::lock_guard<std::mutex> lk(m->mu);
+        for (auto it = m->tiles.begin(); it != m->tiles.end();)
+            it = it->second->larger && !before.count(it->first) ? m->tiles.erase(it) : std::next(it);
+    }
+    return build(SliceUse::kNotLarger);
+}
+
+int batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opts, uint64_t budget, mlem_batch **out) {
+    ARGCHK(out, "mlem_batch_create: null out");
+    *out = nullptr;
+    ARGCHK(m && slots > 0, "mlem_batch_create: null matrix or no slots");
+    mlem_batch_opts o;
+    if (opts)
+        o = *opts;
+    else
+        mlem_batch_opts_default(&o);
+    const uint32_t BC = o.per_pass ? o.per_pass : 4u;
+    ARGCHK(BC == 1 || BC == 4 || BC == 8, "mlem_batch_create: per_pass must be 1, 4 or 8");
+    ARGCHK(o.values <= VAL_UF16, "mlem_batch_create: values must be 0 (f32), 1 (bf16), 2 (fp16) or 3 (uf16)");
+    ARGCHK(m->has_T || m->tiles_only, "mlem_batch_create: the transpose must be resident (upload it or build it)");
+    if (m->tiles_only) {
+        ARGCHK(BC == m->tile_bc && (o.tile_width == 0 || o.tile_width == m->tile_W) &&
+                   m->takes_rows(o.tile_rows) && (o.values == 0 || o.values == m->tile_vt),
+               "mlem_batch_create: the matrix holds tiles of width %u and %u (A) and %u (A^T) rows with values %u for "
+               "%u per pass",
+               m->tile_W, m->tile_R[0], m->tile_R[1], m->tile_vt, m->tile_bc);
+        o.tile_width = m->tile_W;
+        o.values = m->tile_vt;
+    }
+    // Widths: 1024, 512 for 8 per pass (whose x of 1024 columns would leave
+    // one workgroup per CU); default rows: setup_tiled, for FP and BP by itself.
+    const uint32_t W = o.tile_width ? o.tile_width : (BC == 8 ? 512u : 1024u);
+    ARGCHK(valid_tile_config(W, BC), "mlem_batch_create: no blocked kernel for width %u with %u per pass", W, BC);
+    ARGCHK(o.tile_rows == 0 || valid_tile_rows(o.tile_rows),
+           "mlem_batch_create: tile_rows must be 512 ... 16384 (a power of two)");
+    ARGCHK(valid_stream_threads(o.tile_threads), "mlem_batch_create: tile_threads must be 0, 128, 256 or 512");
+    HIPCHK(hipSetDevice(m->device));
+    const uint32_t side_rows[2] = {o.tile_rows, o.tile_rows};
+    auto b = std::make_unique<mlem_batch>();
+    b->m = m;
+    b->slots = slots;
+    b->BC = BC;
+    b->nt = o.tile_threads;
+    b->use_graph = o.use_graph != 0;
+    b->passes = (slots + BC - 1) / BC;
+    b->rows_x = (m->rows + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
+    b->cols_x = (m->cols + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
+    HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
+    if (int st = batch_take_tiles(b.get(), W, m->tiles_only ? m->tile_R : side_rows, o, budget)) return st;
+    if (b->tfp->ordered != b->tbp->ordered)  // a row order set from another thread between the two builds
+        return set_err(MLEM_ERR_INVALID_ARGUMENT, "mlem_batch_create: the row order changed while the tiles were built");
+    if (b->tfp->ordered) b->row_order = m->row_order.as<uint32_t>();
+    const size_t per = (size_t)BC * b->passes;
+    b->pass.resize(b->passes);  // passes are allocated when first used (batch_set_async)
+    HIPCHK(b->sens.alloc(sizeof(float) * m->cols));
+    HIPCHK(b->active.alloc(sizeof(uint32_t) * per));
+    HIPCHK(b->stage.alloc(sizeof(float) * std::max<size_t>(1, std::max(m->rows, m->cols))));
+    HIPCHK(launch_fill_u32(b->active.as<uint32_t>(), 0u, per, b->stream));
+    b->active_host.assign(per, 0);
+    if (o.values != VAL_F32)  // the quantized matrix's own sensitivity
+        HIPCHK(hipMemcpyAsync(b->sens.p, b->tbp->sens.p, sizeof(float) * m->cols, hipMemcpyDeviceToDevice,
+                              b->stream));
+    else if (int st = sens_on_device(m, b->sens.as<float>(), nullptr, b->stream))
+        return st;
+    HIPCHK(hipStreamSynchronize(b->stream));
+    (void)scratch_trim();
+    m->users.fetch_add(1);
+    *out = b.release();
+    return MLEM_OK;
+}
+
 uint64_t batch_release_pass(mlem_batch *b, uint32_t p) {
     if (!b || p >= b->passes || !b->pass[p]) return 0;
     for (uint32_t q = 0; q < b->BC; ++q)
@@ -163,6 +278,7 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
     ARGCHK(values <= VAL_UF16, "mlem_autotune: values must be 0 (f32), 1 (bf16), 2 (fp16) or 3 (uf16)");
     ARGCHK(m->has_T, "mlem_autotune: the transpose must be resident");
     HIPCHK(hipSetDevice(m->device));
+    std::lock_guard<std::mutex> building(m->build_mu);
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     std::vector<std::pair<uint32_t, uint32_t>> shapes;  // (W, R)
@@ -244,9 +360,11 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
             const Tiled *tf = nullptr, *tb = nullptr;
             const TileWorkDev *wf = nullptr, *wb = nullptr;
             DevBuf part;  // FP and BP in turn
-            int st = setup_tiled(m, 0, sh.first, sh.second, values, BC, g * (uint32_t)cus, &tf, &wf, nullptr);
+            int st = setup_tiled(m, 0, sh.first, sh.second, values, BC, g * (uint32_t)cus, SliceUse::kAny, &tf, &wf,
+                                 nullptr);
             if (st == MLEM_OK)
-                st = setup_tiled(m, 1, sh.first, sh.second, values, BC, g * (uint32_t)cus, &tb, &wb, nullptr);
+                st = setup_tiled(m, 1, sh.first, sh.second, values, BC, g * (uint32_t)cus, SliceUse::kAny, &tb, &wb,
+                                 nullptr);
             if (st == MLEM_OK) {
                 const hipError_t e = part.alloc(passes * std::max(tiled_part_bytes(tf->plan, wf->view.nwg, BC),
                                                                   tiled_part_bytes(tb->plan, wb->view.nwg, BC)));
@@ -315,70 +433,7 @@ void mlem_batch_opts_default(mlem_batch_opts *o) {
 }
 
 int mlem_batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opts, mlem_batch **out) {
-    ARGCHK(out, "mlem_batch_create: null out");
-    *out = nullptr;
-    ARGCHK(m && slots > 0, "mlem_batch_create: null matrix or no slots");
-    mlem_batch_opts o;
-    if (opts)
-        o = *opts;
-    else
-        mlem_batch_opts_default(&o);
-    const uint32_t BC = o.per_pass ? o.per_pass : 4u;
-    ARGCHK(BC == 1 || BC == 4 || BC == 8, "mlem_batch_create: per_pass must be 1, 4 or 8");
-    ARGCHK(o.values <= VAL_UF16, "mlem_batch_create: values must be 0 (f32), 1 (bf16), 2 (fp16) or 3 (uf16)");
-    ARGCHK(m->has_T || m->tiles_only, "mlem_batch_create: the transpose must be resident (upload it or build it)");
-    if (m->tiles_only) {
-        ARGCHK(BC == m->tile_bc && (o.tile_width == 0 || o.tile_width == m->tile_W) &&
-                   m->takes_rows(o.tile_rows) &&
-                   (o.values == 0 || o.values == m->tile_vt),
-               "mlem_batch_create: the matrix holds tiles of width %u and %u (A) and %u (A^T) rows with values %u for "
-               "%u per pass",
-               m->tile_W, m->tile_R[0], m->tile_R[1], m->tile_vt, m->tile_bc);
-        o.tile_width = m->tile_W;
-        o.values = m->tile_vt;
-    }
-    // Widths: 1024, 512 for 8 per pass (whose x of 1024 columns would leave
-    // one workgroup per CU); default rows: setup_tiled, for FP and BP by itself.
-    const uint32_t W = o.tile_width ? o.tile_width : (BC == 8 ? 512u : 1024u);
-    ARGCHK(valid_tile_config(W, BC), "mlem_batch_create: no blocked kernel for width %u with %u per pass", W, BC);
-    ARGCHK(o.tile_rows == 0 || valid_tile_rows(o.tile_rows),
-           "mlem_batch_create: tile_rows must be 512 ... 16384 (a power of two)");
-    ARGCHK(valid_stream_threads(o.tile_threads), "mlem_batch_create: tile_threads must be 0, 128, 256 or 512");
-    HIPCHK(hipSetDevice(m->device));
-    auto side_rows = [&](int which) { return m->tiles_only ? m->tile_R[which] : o.tile_rows; };
-    auto b = std::make_unique<mlem_batch>();
-    b->m = m;
-    b->slots = slots;
-    b->BC = BC;
-    b->nt = o.tile_threads;
-    b->use_graph = o.use_graph != 0;
-    b->passes = (slots + BC - 1) / BC;
-    b->rows_x = (m->rows + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
-    b->cols_x = (m->cols + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
-    HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-    if (int st = setup_tiled(m, 0, W, side_rows(0), o.values, BC, o.tile_groups, &b->tfp, &b->wfp, nullptr)) return st;
-    if (int st = setup_tiled(m, 1, W, side_rows(1), o.values, BC, o.tile_groups, &b->tbp, &b->wbp, nullptr)) return st;
-    if (int st = batch_alloc_part(b.get(), b->passes)) return st;
-    if (b->tfp->ordered != b->tbp->ordered)  // a row order set from another thread between the two builds
-        return set_err(MLEM_ERR_INVALID_ARGUMENT, "mlem_batch_create: the row order changed while the tiles were built");
-    if (b->tfp->ordered) b->row_order = m->row_order.as<uint32_t>();
-    const size_t per = (size_t)BC * b->passes;
-    b->pass.resize(b->passes);  // passes are allocated when first used (batch_set_async)
-    HIPCHK(b->sens.alloc(sizeof(float) * m->cols));
-    HIPCHK(b->active.alloc(sizeof(uint32_t) * per));
-    HIPCHK(b->stage.alloc(sizeof(float) * std::max<size_t>(1, std::max(m->rows, m->cols))));
-    HIPCHK(launch_fill_u32(b->active.as<uint32_t>(), 0u, per, b->stream));
-    b->active_host.assign(per, 0);
-    if (o.values != VAL_F32)  // the quantized matrix's own sensitivity
-        HIPCHK(hipMemcpyAsync(b->sens.p, b->tbp->sens.p, sizeof(float) * m->cols, hipMemcpyDeviceToDevice,
-                              b->stream));
-    else if (int st = sens_on_device(m, b->sens.as<float>(), nullptr, b->stream))
-        return st;
-    HIPCHK(hipStreamSynchronize(b->stream));
-    (void)scratch_trim();
-    m->users.fetch_add(1);
-    *out = b.release();
-    return MLEM_OK;
+    return batch_create(m, slots, opts, 0, out);
 }
 
 int mlem_batch_set(mlem_batch *b, uint32_t slot, const int32_t *g, const float *f0) {

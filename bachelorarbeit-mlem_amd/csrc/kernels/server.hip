@@ -112,7 +112,8 @@ int mlem_server_add_matrix(mlem_server *s, mlem_matrix *m, uint32_t max_slots, u
     // the matrix, the batch's fixed buffers and one pass fit in what is left
     // of the budget.
     mlem_batch *b = nullptr;
-    if (int st = mlem_batch_create(m, max_slots, &s->bopts, &b))
+    const uint64_t left = s->budget ? std::max<uint64_t>(1, s->budget - std::min(s->budget, s->used)) : 0;
+    if (int st = mlem::abi::batch_create(m, max_slots, &s->bopts, left, &b))
         return fail(st, "mlem_server_add_matrix: %s", std::string(mlem_last_error()).c_str());
     // Under a budget the partial sums are those of one pass: what several
     // passes per launch would add goes to requests.

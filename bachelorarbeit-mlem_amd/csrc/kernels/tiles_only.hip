@@ -22,8 +22,8 @@ struct ChunkedTiles {
     std::vector<uint32_t> nz;     // entries per tile
     std::vector<uint32_t> wbase;  // row slices: steps per (row block, stream, segment), then (lay_out) first steps
     uint32_t most = 0;            // the most steps of a stream in a tile
-    bool slices;                  // still possible; from lay_out() on: suit; from allocate() on: taken
-    uint64_t quad_cap = 0;        // entries of the quads, whatever the layout
+    bool slices;                  // still possible; from lay_out() on: taken
+    bool larger = false;          // taken, and larger than the quads
     Tiled *t = nullptr;
 
     ChunkedTiles(const TilePlan &p, Tiled *tiled)
@@ -78,35 +78,42 @@ struct ChunkedTiles {
     }
 
     // After the counts: the offsets, and whether row slices suit the matrix.
-    void lay_out() {
+    // Such a matrix shares the device with nothing but the vectors of batches
+    // to come: slices that are larger than the quads are taken only where
+    // they leave a quarter of the device (freed_later: what the build itself
+    // gives back afterwards).
+    int lay_out(SliceUse use, size_t freed_later) {
         uint64_t run = 0;
         for (uint64_t i = 0; i <= P.ntiles; ++i) {
             const uint64_t n = i < P.ntiles ? size[i] : 0;
             size[i] = run;
             run += n;
         }
-        quad_cap = P.cap = run + 8;  // as one build: a multiple of 8, at least one group
+        P.cap = run + 8;  // as one build: a multiple of 8, at least one group
         uint64_t steps = 0;
         slices = slices && slice_prefix(P.W, &wbase, &steps, &P.group) && slices_suit(P, steps, most);
-        if (slices) {
-            P.slices = true;
-            P.steps = steps;
-            P.most = most;
-            P.cap = steps * 64 + 8;
-        }
+        if (!slices) return MLEM_OK;
+        TilePlan S = P;
+        S.slices = true;
+        S.steps = steps;
+        S.most = most;
+        S.cap = steps * 64 + 8;
+        const size_t bytes = tiled_matrix_bytes(S);
+        larger = bytes > tiled_matrix_bytes(P);
+        size_t free_b = 0, total_b = 0;
+        (void)scratch_trim();
+        HIPCHK(hipMemGetInfo(&free_b, &total_b));
+        if (larger && (use == SliceUse::kNotLarger || free_b + freed_later < bytes + total_b / 4))
+            slices = larger = false;
+        else
+            P = S;
+        return MLEM_OK;
     }
 
     int allocate() {
-        hipError_t e = t->mem.alloc(tiled_matrix_bytes(P));
-        if (e == hipErrorOutOfMemory && slices) {  // the quads, which may be smaller
-            (void)hipGetLastError();
-            slices = P.slices = false;
-            P.steps = 0;
-            P.cap = quad_cap;
-            e = t->mem.alloc(tiled_matrix_bytes(P));
-        }
-        HIPCHK(e);
+        HIPCHK(t->mem.alloc(tiled_matrix_bytes(P)));
         t->plan = P;
+        t->larger = larger;
         t->view = tiled_matrix_view(P, t->mem.p);
         if (slices) {
             HIPCHK(hipMemcpy(t->view.wbase, wbase.data(), 4 * wbase.size(), hipMemcpyHostToDevice));
@@ -157,13 +164,10 @@ struct ChunkedTiles {
     }
 };
 
-}  // namespace
-
-extern "C" {
-
-int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t nnz, const uint64_t *rowptr,
-                             const uint32_t *col, const float *val, uint32_t tile_width, uint32_t tile_rows,
-                             uint32_t values, uint32_t per_pass, uint64_t chunk_bytes, mlem_matrix **out) {
+// *larger: row slices larger than the quads were taken on the way.
+int create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t nnz, const uint64_t *rowptr, const uint32_t *col,
+                 const float *val, uint32_t tile_width, uint32_t tile_rows, uint32_t values, uint32_t per_pass,
+                 uint64_t chunk_bytes, SliceUse use, bool *larger, mlem_matrix **out) {
     ARGCHK(out, "mlem_matrix_create_tiled: null out");
     *out = nullptr;
     ARGCHK(rowptr && (nnz == 0 || (col && val)), "mlem_matrix_create_tiled: null matrix array");
@@ -293,8 +297,9 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
             progress("A^T tiles %s over %u column ranges (%.1f GB of range scratch)", pass ? "filled" : "counted", nr,
                      budget / 2 / 1e9);
             if (pass == 0) {
-                bT.lay_out();
+                if (int st = bT.lay_out(use, ci.bytes + va.bytes)) return st;
                 if (!bT.slices && RT != RTq) pass = other_rows();
+                *larger = *larger || bT.larger;
             }
         }
         HIPCHK(hipDeviceSynchronize());
@@ -372,8 +377,9 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
         progress("A tiles %s over %u row chunks (%u smaller after a failed allocation; %.1f GB of chunk scratch)",
                  pass ? "filled" : "counted", chunks, retries, budget / 1e9);
         if (pass == 0) {
-            bA.lay_out();
+            if (int st = bA.lay_out(use, 0)) return st;
             if (!bA.slices && R != Rq) pass = other_rows();
+            *larger = *larger || bA.larger;
         }
     }
     HIPCHK(hipDeviceSynchronize());
@@ -390,6 +396,22 @@ int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t 
     m->tile_auto = tile_rows ? 0 : automatic_rows_name(nnz, BC);
     *out = m.release();
     return MLEM_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int mlem_matrix_create_tiled(int device, uint32_t rows, uint32_t cols, uint64_t nnz, const uint64_t *rowptr,
+                             const uint32_t *col, const float *val, uint32_t tile_width, uint32_t tile_rows,
+                             uint32_t values, uint32_t per_pass, uint64_t chunk_bytes, mlem_matrix **out) {
+    bool larger = false;
+    auto build = [&](SliceUse use) {
+        return create_tiled(device, rows, cols, nnz, rowptr, col, val, tile_width, tile_rows, values, per_pass,
+                            chunk_bytes, use, &larger, out);
+    };
+    const int st = build(SliceUse::kAny);
+    return st == MLEM_ERR_OUT_OF_MEMORY && larger ? build(SliceUse::kNotLarger) : st;
 }
 
 }  // extern "C"

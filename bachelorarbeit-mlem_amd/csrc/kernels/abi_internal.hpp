@@ -354,8 +354,9 @@ int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to);
 // for the matrix, the batch and its passes.
 int batch_create(mlem_matrix *m, uint32_t slots, const mlem_batch_opts *opts, uint64_t budget, mlem_batch **out);
 // The partial-sum buffer for up to `passes` passes per launch (at most
-// kMaxPasses), fewer where the memory for them is not free.
-int batch_alloc_part(mlem_batch *b, uint32_t passes);
+// kMaxPasses), fewer where the memory for them is not free beside `keep`
+// bytes that the batch will need.
+int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t keep);
 // Frees pass p when none of its slots is active (returns the bytes freed).
 uint64_t batch_release_pass(mlem_batch *b, uint32_t p);
 // Progress of long builds on stderr when MLEM_VERBOSE is set.

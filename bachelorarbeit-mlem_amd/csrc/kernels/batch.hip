@@ -36,6 +36,12 @@ int enqueue_batch_iteration(mlem_batch *b, const std::vector<uint8_t> &passes) {
     return MLEM_OK;
 }
 
+// A captured iteration holds the addresses of the passes and of the partial sums.
+void drop_graph(mlem_batch *b) {
+    if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
+    b->gexec = nullptr;
+}
+
 }  // namespace
 
 namespace mlem {
@@ -51,9 +57,20 @@ int batch_set_async(mlem_batch *b, uint32_t slot, const int32_t *g, const float 
     hipStream_t s = b->stream;
     if (!b->pass[p]) {  // first slot of this pass: its vectors, zero-filled (padding included)
         auto np = std::make_unique<BatchPass>();
-        HIPCHK(np->g.alloc(sizeof(int32_t) * b->rows_x * b->BC));
-        HIPCHK(np->ratio.alloc(sizeof(float) * b->rows_x * b->BC));
-        HIPCHK(np->f.alloc(sizeof(float) * b->cols_x * b->BC));
+        auto vectors = [&]() {
+            hipError_t e = np->g.alloc(sizeof(int32_t) * b->rows_x * b->BC);
+            if (e == hipSuccess) e = np->ratio.alloc(sizeof(float) * b->rows_x * b->BC);
+            if (e == hipSuccess) e = np->f.alloc(sizeof(float) * b->cols_x * b->BC);
+            return e;
+        };
+        hipError_t e = vectors();
+        if (e == hipErrorOutOfMemory && b->group > 1) {  // the partial sums of one pass will do
+            HIPCHK(hipStreamSynchronize(s));
+            drop_graph(b);
+            if (int st = batch_alloc_part(b, 1, 0)) return st;
+            e = vectors();
+        }
+        HIPCHK(e);
         HIPCHK(launch_fill_u32(np->g.as<uint32_t>(), 0u, b->rows_x * b->BC, s));
         HIPCHK(launch_fill(np->ratio.as<float>(), 0.0f, b->rows_x * b->BC, s));
         HIPCHK(launch_fill(np->f.as<float>(), 0.0f, b->cols_x * b->BC, s));
@@ -116,13 +133,17 @@ int batch_move_slot_async(mlem_batch *b, uint32_t from, uint32_t to) {
     return MLEM_OK;
 }
 
-int batch_alloc_part(mlem_batch *b, uint32_t passes) {
+int batch_alloc_part(mlem_batch *b, uint32_t passes, uint64_t keep) {
     auto bytes = [&](const Tiled *t, const TileWorkDev *w) {
         return w->view.direct ? 0 : tiled_part_bytes(t->plan, w->view.nwg, b->BC);
     };
     const uint64_t one = std::max<uint64_t>(4, std::max(bytes(b->tfp, b->wfp), bytes(b->tbp, b->wbp)));
     // One right-hand side per pass: the blocked kernel takes one pass per launch.
     uint32_t n = b->BC == 1 ? 1u : std::max(1u, std::min(passes, kMaxPasses));
+    b->part.reset();
+    size_t free_b = 0;
+    if (n > 1) HIPCHK(free_device_bytes(&free_b));
+    while (n > 1 && n * one + keep > free_b) n = (n + 1) / 2;
     for (;; n = (n + 1) / 2) {
         const hipError_t e = b->part.alloc(n * one);
         b->group = n;
@@ -145,17 +166,19 @@ static int batch_take_tiles(mlem_batch *b, uint32_t W, const uint32_t rows[2], c
         std::lock_guard<std::mutex> lk(m->mu);
         for (const auto &t : m->tiles) before.insert(t.first);
     }
+    // What the batch is still to hold: its passes, sensitivity, flags and staging vector.
+    const uint64_t more = (uint64_t)b->passes * b->pass_bytes() + sizeof(float) * m->cols +
+                          sizeof(uint32_t) * (uint64_t)b->passes * b->BC +
+                          sizeof(float) * std::max<uint64_t>(m->rows, m->cols);
     auto build = [&](SliceUse use) -> int {
         if (int st = setup_tiled(m, 0, W, rows[0], o.values, b->BC, o.tile_groups, use, &b->tfp, &b->wfp, nullptr))
             return st;
         if (int st = setup_tiled(m, 1, W, rows[1], o.values, b->BC, o.tile_groups, use, &b->tbp, &b->wbp, nullptr))
             return st;
-        return batch_alloc_part(b, b->passes);
+        // Under a budget one pass per launch: what several would add goes to requests.
+        return batch_alloc_part(b, budget ? 1 : b->passes, more);
     };
     auto room = [&]() -> bool {
-        const uint64_t more = (uint64_t)b->passes * b->pass_bytes() + sizeof(float) * m->cols +
-                              sizeof(uint32_t) * (uint64_t)b->passes * b->BC +
-                              sizeof(float) * std::max<uint64_t>(m->rows, m->cols);
         if (!budget) {
             size_t free_b = 0;
             return free_device_bytes(&free_b) != hipSuccess || more <= free_b;
@@ -253,10 +276,7 @@ uint64_t batch_release_pass(mlem_batch *b, uint32_t p) {
         if (b->active_host[(size_t)p * b->BC + q]) return 0;
     if (hipSetDevice(b->m->device) != hipSuccess || hipStreamSynchronize(b->stream) != hipSuccess) return 0;
     const uint64_t bytes = b->pass[p]->g.bytes + b->pass[p]->ratio.bytes + b->pass[p]->f.bytes;
-    if (b->gexec) {  // a captured iteration may hold the pass's addresses
-        (void)hipGraphExecDestroy(b->gexec);
-        b->gexec = nullptr;
-    }
+    drop_graph(b);
     b->pass[p].reset();
     return bytes;
 }
@@ -446,6 +466,7 @@ int mlem_batch_deactivate(mlem_batch *b, uint32_t slot) { return batch_deactivat
 
 int mlem_batch_iterate(mlem_batch *b, uint32_t iters) {
     ARGCHK(b, "mlem_batch_iterate: null handle");
+    if (!b->part.p) return set_err(MLEM_ERR_OUT_OF_MEMORY, "mlem_batch_iterate: the batch has lost its partial sums");
     HIPCHK(hipSetDevice(b->m->device));
     const uint32_t BC = b->BC;
     std::vector<uint8_t> passes(b->passes, 0);

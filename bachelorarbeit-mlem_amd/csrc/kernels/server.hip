@@ -115,14 +115,6 @@ int mlem_server_add_matrix(mlem_server *s, mlem_matrix *m, uint32_t max_slots, u
     const uint64_t left = s->budget ? std::max<uint64_t>(1, s->budget - std::min(s->budget, s->used)) : 0;
     if (int st = mlem::abi::batch_create(m, max_slots, &s->bopts, left, &b))
         return fail(st, "mlem_server_add_matrix: %s", std::string(mlem_last_error()).c_str());
-    // Under a budget the partial sums are those of one pass: what several
-    // passes per launch would add goes to requests.
-    if (s->budget)
-        if (int st = mlem::abi::batch_alloc_part(b, 1)) {
-            const std::string msg = mlem_last_error();
-            mlem_batch_destroy(b);
-            return fail(st, "mlem_server_add_matrix: %s", msg.c_str());
-        }
     const uint64_t bbytes = b->fixed_bytes(), pbytes = b->pass_bytes();
     mlem_matrix_info(m, nullptr, nullptr, nullptr, nullptr, &mbytes);  // with the tiles the batch built
     if (s->budget && s->used + mbytes + bbytes + pbytes > s->budget) {

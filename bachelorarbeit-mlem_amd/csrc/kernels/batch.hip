@@ -284,9 +284,145 @@ uint64_t batch_release_pass(mlem_batch *b, uint32_t p) {
 }  // namespace abi
 }  // namespace mlem
 
+// -------------------------------------------------------------- autotuner
+namespace {
+
+// The stream and events that candidates are timed with.
+struct TuneClock {
+    hipStream_t s = nullptr;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    ~TuneClock() {
+        if (s) (void)hipStreamSynchronize(s);
+        if (e0) (void)hipEventDestroy(e0);
+        if (e1) (void)hipEventDestroy(e1);
+        if (s) (void)hipStreamDestroy(s);
+    }
+};
+
+// Times the candidates `passes` passes at a time; *short_of_memory: one of
+// them, or the vectors, did not fit (with several passes nothing further is
+// timed then).
+int tune(mlem_matrix *m, uint32_t BC, uint32_t values, uint32_t passes, SliceUse use, mlem_tune_result *out,
+         bool *short_of_memory) {
+    int dev = 0, cus_i = 256;
+    if (hipGetDevice(&dev) == hipSuccess)
+        (void)hipDeviceGetAttribute(&cus_i, hipDeviceAttributeMultiprocessorCount, dev);
+    const uint32_t cus = (uint32_t)std::max(1, cus_i);
+    std::vector<std::pair<uint32_t, uint32_t>> shapes;  // (W, R)
+    if (BC == 1)
+        shapes = {{1024, 1024}, {1024, 2048}, {1024, 4096}, {2048, 1024}, {2048, 2048}};
+    else if (BC == 4)
+        shapes = {{512, 1024}, {1024, 512}, {1024, 1024}, {1024, 2048}, {512, 2048}};
+    else
+        shapes = {{512, 512}, {512, 1024}};
+    const size_t rows_x = ((size_t)m->rows + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
+    const size_t cols_x = ((size_t)m->cols + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
+    DevBuf xf, xb, yf, yb;
+    for (auto v : {std::make_pair(&xf, cols_x), std::make_pair(&xb, rows_x), std::make_pair(&yf, rows_x),
+                   std::make_pair(&yb, cols_x)}) {
+        const hipError_t e = v.first->alloc(sizeof(float) * v.second * BC * passes);
+        *short_of_memory = *short_of_memory || e == hipErrorOutOfMemory;
+        HIPCHK(e);
+    }
+    TuneClock c;
+    HIPCHK(hipStreamCreateWithFlags(&c.s, hipStreamNonBlocking));
+    HIPCHK(hipEventCreate(&c.e0));
+    HIPCHK(hipEventCreate(&c.e1));
+    HIPCHK(launch_fill(xf.as<float>(), 1.0f, cols_x * BC * passes, c.s));
+    HIPCHK(launch_fill(xb.as<float>(), 1.0f, rows_x * BC * passes, c.s));
+    // One side's time per launch (partials + reduce), mean of three after a warm-up.
+    auto time_side = [&](const Tiled *t, const TileWorkDev *w, const DevBuf &part, const float *x, size_t x_pass,
+                         float *y, uint32_t nt, double *ms) -> int {
+        PassX px{};
+        PassEpi pe{};
+        for (uint32_t k = 0; k < passes; ++k) {
+            px.x[k] = x + k * x_pass * BC;
+            pe.ea[k].out = y + k * (size_t)t->plan.rows * BC;
+        }
+        px.n = pe.n = passes;
+        for (int rep = 0; rep < 4; ++rep) {
+            if (rep == 1) HIPCHK(hipEventRecord(c.e0, c.s));
+            HIPCHK(launch_tiled_spmv(t->plan, t->view, w->view, px, part.as<float>(), BC, nt, EPI_PLAIN, pe, c.s));
+        }
+        HIPCHK(hipEventRecord(c.e1, c.s));
+        HIPCHK(hipEventSynchronize(c.e1));
+        float f = 0.0f;
+        HIPCHK(hipEventElapsedTime(&f, c.e0, c.e1));
+        *ms = f / 3.0;
+        return MLEM_OK;
+    };
+    double best = 1e300;
+    bool sliced = false;  // a shape kept both sides as row slices
+    for (const auto &sh : shapes) {
+        const uint32_t W = sh.first, R = sh.second;
+        if (W == 512 && R == 2048 && sliced) continue;  // too tall for slices
+        // The automatic runs where they are one per row block for a side.
+        const bool direct = BC != 1 && (slices_direct(m->cols, W, R, m->rows, m->nnz, BC) ||
+                                        slices_direct(m->rows, W, R, m->cols, m->nnz, BC));
+        std::vector<uint32_t> groups;  // per CU, 0: automatic
+        if (BC == 1) {
+            groups = {16, 24, 32};
+            if (default_tile_groups(m->nnz, values, 1) == 12 * cus) groups.push_back(12);
+        } else if (W == 1024 && R == 512) {
+            if (!direct) continue;  // small tiles pay where whole blocks are runs
+            groups = {0};
+        } else {
+            groups = {4, 8, 16};
+            if (direct) groups.push_back(0);
+        }
+        for (uint32_t g : groups) {
+            const Tiled *t[2] = {};
+            const TileWorkDev *w[2] = {};
+            DevBuf part;  // FP and BP in turn
+            int st = MLEM_OK;
+            for (int side = 0; side < 2 && st == MLEM_OK; ++side)
+                st = setup_tiled(m, side, W, R, values, BC, g * cus, use, &t[side], &w[side], nullptr);
+            const bool slices = st == MLEM_OK && t[0]->plan.slices && t[1]->plan.slices;
+            sliced = sliced || slices;
+            if (slices && g == 16) continue;  // more runs than pay: 4 per CU beat 8 (default_tile_groups)
+            if (st == MLEM_OK) {
+                const hipError_t e = part.alloc(passes * std::max(tiled_part_bytes(t[0]->plan, w[0]->view.nwg, BC),
+                                                                  tiled_part_bytes(t[1]->plan, w[1]->view.nwg, BC)));
+                if (e == hipErrorOutOfMemory)
+                    st = MLEM_ERR_OUT_OF_MEMORY;
+                else
+                    HIPCHK(e);
+            }
+            if (st == MLEM_ERR_OUT_OF_MEMORY) {
+                *short_of_memory = true;
+                if (passes > 1) return st;
+            }
+            if (st == MLEM_ERR_UNSUPPORTED || st == MLEM_ERR_OUT_OF_MEMORY) continue;  // does not suit or fit the matrix
+            if (st != MLEM_OK) return st;
+            // Work-items per workgroup of the block streams (128 was slower at
+            // every shape timed on the 3D scanner matrix).
+            for (uint32_t nt : {256u, 512u}) {
+                if ((BC == 1 || slices) && nt != 512) continue;  // without effect
+                double fp = 0, bp = 0;
+                st = time_side(t[0], w[0], part, xf.as<float>(), cols_x, yf.as<float>(), BC == 1 ? 0 : nt, &fp);
+                if (st == MLEM_OK)
+                    st = time_side(t[1], w[1], part, xb.as<float>(), rows_x, yb.as<float>(), BC == 1 ? 0 : nt, &bp);
+                if (st != MLEM_OK) return st;
+                ++out->candidates;
+                if (fp + bp < best) {
+                    best = fp + bp;
+                    out->tile_width = W;
+                    out->tile_rows = R;
+                    out->tile_groups = g * cus;
+                    out->tile_threads = BC == 1 ? 0 : nt;
+                    out->fp_ms = fp;
+                    out->bp_ms = bp;
+                }
+            }
+        }
+    }
+    return MLEM_OK;
+}
+
+}  // namespace
+
 extern "C" {
 
-// -------------------------------------------------------------- autotuner
 // Times the blocked kernels of both sides over a few tile shapes and
 // workgroup counts and reports the fastest.  Candidate tiles that did not
 // exist before and were not chosen are freed again.
@@ -299,149 +435,36 @@ int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values, mlem_tune_
     ARGCHK(m->has_T, "mlem_autotune: the transpose must be resident");
     HIPCHK(hipSetDevice(m->device));
     std::lock_guard<std::mutex> building(m->build_mu);
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    std::vector<std::pair<uint32_t, uint32_t>> shapes;  // (W, R)
-    std::vector<uint32_t> groups;                       // per CU
-    std::vector<uint32_t> threads = {0};                // work-items per workgroup (several right-hand sides)
-    if (BC > 1) threads = {256, 512};  // 128 was slower at every shape timed on the 3D scanner matrix
-    if (BC == 1) {
-        shapes = {{1024, 1024}, {1024, 2048}, {1024, 4096}, {2048, 1024}, {2048, 2048}};
-        groups = {16, 24, 32};
-    } else if (BC == 4) {
-        shapes = {{512, 1024}, {1024, 1024}, {1024, 2048}};
-        groups = {4, 8};
-    } else {
-        shapes = {{512, 512}, {512, 1024}};
-        groups = {4, 8};
-    }
-    // Batches of several passes share their launches, and taller tiles pay
-    // then (683 M entries, one pass of 4 equal at 1024 and 2048 rows, four
-    // 4110 against 3600 us): they are timed four passes at a time.
-    const uint32_t passes = BC == 1 ? 1u : 4u;
     std::set<mlem_matrix::TileKey> before;
     {
         std::lock_guard<std::mutex> lk(m->mu);
         for (const auto &t : m->tiles) before.insert(t.first);
     }
-    const size_t rows_x = ((size_t)m->rows + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
-    const size_t cols_x = ((size_t)m->cols + kTileXPad - 1) / kTileXPad * kTileXPad + kTileXPad;
-    DevBuf xf, xb, yf, yb;
-    HIPCHK(xf.alloc(sizeof(float) * cols_x * BC));
-    HIPCHK(xb.alloc(sizeof(float) * rows_x * BC));
-    HIPCHK(yf.alloc(sizeof(float) * rows_x * BC * passes));
-    HIPCHK(yb.alloc(sizeof(float) * cols_x * BC * passes));
-    hipStream_t s = nullptr;
-    HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    auto cleanup = [&]() {
-        if (e0) (void)hipEventDestroy(e0);
-        if (e1) (void)hipEventDestroy(e1);
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
-    };
-    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
-        cleanup();
-        return set_err(MLEM_ERR_HIP, "mlem_autotune: event creation failed");
-    }
-    if (launch_fill(xf.as<float>(), 1.0f, cols_x * BC, s) != hipSuccess ||
-        launch_fill(xb.as<float>(), 1.0f, rows_x * BC, s) != hipSuccess) {
-        cleanup();
-        return set_err(MLEM_ERR_HIP, "mlem_autotune: fill failed");
-    }
-    double best = 1e300;
-    uint32_t bestW = 0, bestR = 0, bestG = 0, bestT = 0, tried = 0;
-    double best_fp = 0, best_bp = 0;
-    // One side's time per launch (partials + reduce), mean of three after a warm-up.
-    auto time_side = [&](const Tiled *t, const TileWorkDev *w, DevBuf &part, const float *x, float *y, uint32_t nt,
-                         double *ms) {
-        PassX px{};
-        PassEpi pe{};
-        for (uint32_t k = 0; k < passes; ++k) {
-            px.x[k] = x;
-            pe.ea[k].out = y + k * (size_t)t->plan.rows * BC;
-        }
-        px.n = pe.n = passes;
-        for (int rep = 0; rep < 4; ++rep) {
-            if (rep == 1 && hipEventRecord(e0, s) != hipSuccess) return hipErrorUnknown;
-            const hipError_t e = launch_tiled_spmv(t->plan, t->view, w->view, px, part.as<float>(), BC, nt, EPI_PLAIN,
-                                                   pe, s);
-            if (e != hipSuccess) return e;
-        }
-        hipError_t e = hipEventRecord(e1, s);
-        if (e == hipSuccess) e = hipEventSynchronize(e1);
-        float f = 0.0f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&f, e0, e1);
-        *ms = f / 3.0;
-        return e;
-    };
-    for (const auto &sh : shapes) {
-        for (uint32_t g : groups) {
-            const Tiled *tf = nullptr, *tb = nullptr;
-            const TileWorkDev *wf = nullptr, *wb = nullptr;
-            DevBuf part;  // FP and BP in turn
-            int st = setup_tiled(m, 0, sh.first, sh.second, values, BC, g * (uint32_t)cus, SliceUse::kAny, &tf, &wf,
-                                 nullptr);
-            if (st == MLEM_OK)
-                st = setup_tiled(m, 1, sh.first, sh.second, values, BC, g * (uint32_t)cus, SliceUse::kAny, &tb, &wb,
-                                 nullptr);
-            if (st == MLEM_OK) {
-                const hipError_t e = part.alloc(passes * std::max(tiled_part_bytes(tf->plan, wf->view.nwg, BC),
-                                                                  tiled_part_bytes(tb->plan, wb->view.nwg, BC)));
-                if (e == hipErrorOutOfMemory)
-                    st = MLEM_ERR_OUT_OF_MEMORY;
-                else
-                    HIPCHK(e);
-            }
-            if (st == MLEM_ERR_UNSUPPORTED || st == MLEM_ERR_OUT_OF_MEMORY) {
-                (void)hipGetLastError();
-                continue;  // this shape does not suit or fit the matrix
-            }
-            if (st != MLEM_OK) {
-                cleanup();
-                return st;
-            }
-            for (uint32_t nt : threads) {
-                if (tf->plan.slices && tb->plan.slices && nt != threads.back()) continue;  // without effect
-                double fp = 0, bp = 0;
-                hipError_t e = time_side(tf, wf, part, xf.as<float>(), yf.as<float>(), nt, &fp);
-                if (e == hipSuccess) e = time_side(tb, wb, part, xb.as<float>(), yb.as<float>(), nt, &bp);
-                if (e != hipSuccess) {
-                    cleanup();
-                    return hip_err(e, "mlem_autotune: timing", __FILE_NAME__, __LINE__);
-                }
-                ++tried;
-                if (fp + bp < best) {
-                    best = fp + bp;
-                    bestW = sh.first;
-                    bestR = sh.second;
-                    bestG = g;
-                    bestT = nt;
-                    best_fp = fp;
-                    best_bp = bp;
-                }
-            }
-        }
-    }
-    cleanup();
-    {  // free the candidate tiles that were built here and not chosen
+    auto drop_others = [&]() {
         std::lock_guard<std::mutex> lk(m->mu);
         for (auto it = m->tiles.begin(); it != m->tiles.end();) {
             const auto &k = it->first;
-            const bool chosen = std::get<1>(k) == bestW && std::get<2>(k) == bestR && std::get<3>(k) == values &&
+            const bool chosen = out->candidates && std::get<1>(k) == out->tile_width &&
+                                std::get<2>(k) == out->tile_rows && std::get<3>(k) == values &&
                                 std::get<4>(k) == (BC > 1);
             it = (!before.count(k) && !chosen) ? m->tiles.erase(it) : std::next(it);
         }
+    };
+    // Batches of several passes share their launches, and taller tiles pay
+    // then (683 M entries, one pass of 4 equal at 1024 and 2048 rows, four
+    // 4110 against 3600 us): they are timed four passes at a time, each with
+    // its own vectors, or one where that does not fit.
+    bool short_of_memory = false;
+    int st = tune(m, BC, values, BC == 1 ? 1u : 4u, SliceUse::kAny, out, &short_of_memory);
+    if (short_of_memory && BC != 1) {
+        std::memset(out, 0, sizeof(*out));
+        drop_others();
+        st = tune(m, BC, values, 1, SliceUse::kNotLarger, out, &short_of_memory);
     }
+    drop_others();
     (void)scratch_trim();
-    if (!tried) return set_err(MLEM_ERR_UNSUPPORTED, "mlem_autotune: no tile shape suits or fits this matrix");
-    out->tile_width = bestW;
-    out->tile_rows = bestR;
-    out->tile_groups = bestG * (uint32_t)cus;
-    out->tile_threads = bestT;
-    out->candidates = tried;
-    out->fp_ms = best_fp;
-    out->bp_ms = best_bp;
+    if (st != MLEM_OK) return st;
+    if (!out->candidates) return set_err(MLEM_ERR_UNSUPPORTED, "mlem_autotune: no tile shape suits or fits this matrix");
     return MLEM_OK;
 }
 

@@ -452,7 +452,10 @@ int mlem_batch_destroy(mlem_batch *b);
 /* Times the blocked FP and BP kernels of the matrix over a few tile shapes
  * (width x rows) and workgroup counts for `per_pass` right-hand sides (1, 4
  * or 8) and `values` (0 f32, 1 bf16, 2 fp16, 3 uf16), and reports the fastest for
- * mlem_opts / mlem_batch_opts (tile_width, tile_rows, tile_groups).  Tiles
+ * mlem_opts / mlem_batch_opts (tile_width, tile_rows, tile_groups; 0 groups:
+ * the automatic number, which for these rows is one run per row block on
+ * a side).  With 4 or 8 per pass four passes are timed together, or one where
+ * the memory does not hold their vectors and partial sums.  Tiles
  * built for candidates that were not chosen are freed again.  No counterpart
  * in the reference (its section sizes come from argv[5]/[6]). */
 typedef struct mlem_tune_result {
@@ -460,7 +463,7 @@ typedef struct mlem_tune_result {
     uint32_t tile_threads; /* for mlem_batch_opts (0 for 1 per pass)       */
     uint32_t candidates;  /* shape x workgroup-count pairs timed            */
     double fp_ms, bp_ms;  /* per launch of the chosen one, partials + reduce
-                             (4 or 8 per pass: of four passes)             */
+                             (4 or 8 per pass: of the passes together)     */
 } mlem_tune_result;
 int mlem_autotune(mlem_matrix *m, uint32_t per_pass, uint32_t values,
                   mlem_tune_result *out);

@@ -42,8 +42,8 @@ def test_block_stream_candidates():
 
 
 def test_memory_for_one_pass_only():
-    """8e6 rows of one entry: vectors and partial sums of four passes need over 2.2 GB beside the tiles, those of one
-    about 0.6; 1.7 GB are free."""
+    """8e6 rows of one entry: vectors and partial sums of four passes need 1.15 GB beside 0.3 of tiles and their scratch,
+    those of one 0.3; 1.3 GiB are free."""
     rows = 8_000_000
     rowptr = np.arange(rows + 1, dtype=np.uint64)
     col = (np.arange(rows, dtype=np.uint64) * 2654435761 % 1000).astype(np.uint32)
@@ -53,11 +53,11 @@ def test_memory_for_one_pass_only():
         m.build_transpose()
         M.release_scratch()
         before = m.info()["device_bytes"]
-        assert M.hip_lib().mlem_device_alloc(C.byref(p), torch.cuda.mem_get_info(0)[0] - (1700 << 20)) == 0
+        assert M.hip_lib().mlem_device_alloc(C.byref(p), torch.cuda.mem_get_info(0)[0] - (1300 << 20)) == 0
         try:
             t = m.autotune(per_pass=4)
         finally:
             M.hip_lib().mlem_device_free(p)
         print(t, flush=True)
-        assert t["candidates"] >= 1
+        assert t["candidates"] >= 12  # four passes at a time left 4
         assert m.info()["device_bytes"] < before + 2 * 6 * 4 * rows + (256 << 20)  # the chosen tiles at most

@@ -76,7 +76,7 @@ bool Scratch::take_kept(const mlem_matrix *m, size_t n) {
     if (m->serial < kFirst || n > kKept) return false;
     Kept *k = kept_scratch();
     if (!k || k->busy.exchange(true)) return false;
-    if (!memory_is_plenty(k->bytes)) {
+    if (std::max(n, k->bytes) > kSmall && !memory_is_plenty(k->bytes)) {
         k->free();
         k->busy = false;
         return false;
@@ -107,7 +107,7 @@ hipError_t Scratch::alloc(size_t n) {
 Scratch::~Scratch() {
     if (!held) return;
     (void)hipStreamSynchronize(nullptr);  // also where the call failed half way
-    if (!memory_is_plenty(held->bytes)) held->free();
+    if (held->bytes > kSmall && !memory_is_plenty(held->bytes)) held->free();
     held->busy = false;
 }
 

@@ -85,7 +85,8 @@ struct DevBuf {
 // than freed device memory comes back cleared: after some twenty of them
 // calls of 56 ms take 203 in the median and up to 3 s.  So from the third
 // matrix of a process on one buffer per device of up to kKept bytes is kept
-// from call to call, while half of the device's memory is free; a call that
+// from call to call, over kSmall bytes while half of the device's memory is
+// free (asking costs 5 us, a small one-shot reconstruction 60); a call that
 // finds it in use by another thread, too small a device or less free memory
 // takes memory of its own.  The buffer is given back when an allocation of
 // the library fails or it asks for the free memory, when a batch or
@@ -93,7 +94,7 @@ struct DevBuf {
 // that then keep the card to themselves for long), and by
 // mlem_release_scratch.  The first two matrices leave nothing behind.
 struct Scratch {
-    static constexpr size_t kKept = size_t(8) << 30;
+    static constexpr size_t kKept = size_t(8) << 30, kSmall = size_t(64) << 20;
     static constexpr uint64_t kFirst = 3;  // the first matrix of the process that uses the kept buffer
     void *p = nullptr;
     size_t bytes = 0;  // at least what was asked for

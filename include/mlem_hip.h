@@ -61,7 +61,7 @@ int mlem_device_free(void *ptr);
 /* A program that sets up one matrix after another (from its third on) keeps
  * the scratch of a set-up call (mlem_matrix_build_transpose, the tiles of
  * mlem_recon_create) for the next one: one buffer per device of at most
- * 8 GiB, and only while half of the device's memory is free.  No other
+ * 8 GiB, and over 64 MiB only while half of the device's memory is free.  No other
  * figure of this library counts it.  It is given back when an allocation of
  * the library finds the memory short, when a batch, a server's matrix or
  * a tiles-only matrix has been created or mlem_autotune has run, and here:

@@ -751,9 +751,15 @@ __global__ __launch_bounds__(NT) void stream_spmv_kernel(uint32_t R, uint32_t ns
 // y += the partials of row i (of R = 2^rshift) in workgroups w0, w0 + S,
 // ... below we, in that order.  The partials of U workgroups are loaded
 // together, then added in order: one memory latency per U workgroups
-// instead of one each.
+// instead of one each.  The sums are FP64: a run's own sums are chains of FP32
+// additions, and with fewer, longer runs (default_tile_groups) a second chain
+// over the runs would round further than many short ones did.  30 iterations
+// on the mid-sized scanner against 64 bits: 7.7e-7, with FP32 sums here
+// 8.2e-7, with those and twice the runs 8.6e-7; 10 iterations 2.7e-7, 3.3e-7
+// and 3.2e-7.  The reduction waits for memory either way (2D ring, 16 slots
+// of 4 per pass: 2.78 ms, with FP32 2.77; 12 GB scanner 31.4 ms both).
 template <int BC, uint32_t S>
-__device__ __forceinline__ void sum_partials(float (&y)[BC], const float *__restrict__ part, uint32_t w0,
+__device__ __forceinline__ void sum_partials(double (&y)[BC], const float *__restrict__ part, uint32_t w0,
                                              uint32_t we, uint32_t rshift, uint32_t i) {
     constexpr uint32_t U = BC == 1 ? 16 : (BC == 4 ? 8 : 4);
     uint32_t w = w0;
@@ -791,11 +797,14 @@ __global__ void blocked_reduce_kernel(const float *__restrict__ part, uint64_t p
     part += blockIdx.y * pass_part;
     const uint32_t b = r >> rshift, i = r & ((1u << rshift) - 1u);
     const ReduceIn<BC> in = reduce_load<EPI, BC>(r, scale, ea);
-    float y[BC];
+    double y[BC];
 #pragma unroll
-    for (int q = 0; q < BC; ++q) y[q] = 0.0f;
+    for (int q = 0; q < BC; ++q) y[q] = 0.0;
     sum_partials<BC, 1>(y, part, wl_first[b], wl_first[b + 1], rshift, i);
-    reduce_epilogue<EPI, BC>(r, y, in, scale != nullptr, ea);
+    float yf[BC];
+#pragma unroll
+    for (int q = 0; q < BC; ++q) yf[q] = (float)y[q];
+    reduce_epilogue<EPI, BC>(r, yf, in, scale != nullptr, ea);
 }
 
 // The same for blocks with many workgroups (a small matrix spread over the
@@ -810,12 +819,12 @@ __global__ __launch_bounds__(64 * kSlices) void blocked_reduce_sliced_kernel(
     uint32_t rows, const float *__restrict__ scale, PassEpi pe) {
     const EpiArgs ea = pe.ea[blockIdx.y];
     part += blockIdx.y * pass_part;
-    __shared__ float s_y[kSlices][64][BC];
+    __shared__ double s_y[kSlices][64][BC];
     const uint32_t x = threadIdx.x, j = threadIdx.y;
     const uint32_t r = blockIdx.x * 64 + x;
-    float y[BC];
+    double y[BC];
 #pragma unroll
-    for (int q = 0; q < BC; ++q) y[q] = 0.0f;
+    for (int q = 0; q < BC; ++q) y[q] = 0.0;
     ReduceIn<BC> in{};
     if (r < rows) {
         if (j == 0) in = reduce_load<EPI, BC>(r, scale, ea);  // wave 0 applies the epilogue
@@ -830,7 +839,10 @@ __global__ __launch_bounds__(64 * kSlices) void blocked_reduce_sliced_kernel(
     for (uint32_t jj = 1; jj < kSlices; ++jj)
 #pragma unroll
         for (int q = 0; q < BC; ++q) y[q] += s_y[jj][x][q];
-    reduce_epilogue<EPI, BC>(r, y, in, scale != nullptr, ea);
+    float yf[BC];
+#pragma unroll
+    for (int q = 0; q < BC; ++q) yf[q] = (float)y[q];
+    reduce_epilogue<EPI, BC>(r, yf, in, scale != nullptr, ea);
 }
 
 // ----------------------------------------------------------------- builder

@@ -275,7 +275,7 @@ hipError_t launch_tiled_reduce(const TilePlan &p, const TiledMatrix &tm, const T
 // launch_tile_count with quads (its counts in `scratch`): the steps of every
 // (row block, stream, segment) into wsteps (slice_stream_count(p), device)
 // and the rows' places into rowloc (tile_count_rowpos: the quads' positions
-// are gone then); flags_host[0] bit 16: the layout cannot hold a row or a
+// are gone then); flags_host[0] bit 16: the layout cannot hold a row of a
 // tile, [1]: the most steps of a stream in a tile.  flags: 8 bytes on the
 // device.  The call waits.
 bool slices_possible(const TilePlan &p);

@@ -71,8 +71,11 @@ constexpr uint32_t kStagers = 4;                            // waves that stage 
 constexpr int kSliceNT = 64 * (int)(kStreams + kStagers);
 constexpr uint32_t kSliceRows = 16;
 constexpr uint32_t kRowSteps = 255;            // steps of a row in a tile at most
-constexpr uint32_t kStreamSteps = 1u << 14;    // steps of a stream in a tile below this
 constexpr uint32_t kSliceMaxR = 2048;          // rows per block at most
+constexpr uint32_t kStreamSteps = 1u << 14;    // steps of a stream in a tile are fewer
+static_assert(kSliceMaxR / kSliceRows * kRowSteps < kStreamSteps * kStreams &&
+                  (kSliceMaxR / kSliceRows / kStreams + 1) * kRowSteps < kStreamSteps,
+              "each slice goes to the shortest stream, so a stream exceeds the mean by one slice at most");
 constexpr uint32_t kRunTiles = 64;             // tiles per run at most (one per lane)
 // Steps in flight per wave, G taken together.  683 M entries in 16 bits, 4
 // right-hand sides, fours, us per iteration with 8 / 12 / 16 / 24 in flight:
@@ -302,8 +305,7 @@ __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOM
 // A wave per tile: a counting sort of its rows by steps (longest first,
 // stable), their slices and streams.  rowloc as above for rows with entries;
 // wsteps[(b * 8 + w) * nseg + s] = steps of stream w; *most = the most of
-// any; bit 16 of *bad: a row or a stream with more steps than the layout
-// holds.
+// any; bit 16 of *bad: a row with more steps than the layout holds.
 __global__ __launch_bounds__(kWG) void slice_rows_kernel(const uint32_t *__restrict__ cnt, uint32_t rows, uint32_t R,
                                                          uint32_t nseg, uint64_t ntiles,
                                                          uint32_t *__restrict__ rowloc,
@@ -375,8 +377,7 @@ __global__ __launch_bounds__(kWG) void slice_rows_kernel(const uint32_t *__restr
         for (uint32_t o = 1; o < kStreams; o <<= 1) key = min(key, __shfl_xor(key, o));
         if (key == key0) {
             const uint32_t st = sl[i];
-            over = over || n >= kStreamSteps;
-            if (lane < kStreams) sl[i] = st | ((n & (kStreamSteps - 1)) << 8) | (w8 << 22);
+            if (lane < kStreams) sl[i] = st | (n << 8) | (w8 << 22);
             n += st;
         }
     }

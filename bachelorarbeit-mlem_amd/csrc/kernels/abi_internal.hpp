@@ -190,7 +190,7 @@ struct mlem_matrix {
         static std::atomic<uint64_t> made{0};
         serial = ++made;
     }
-    uint64_t serial;  // the how-manieth matrix of the process (Scratch)
+    uint64_t serial;  // 1 for the first matrix of the process (Scratch)
     int device = 0;
     uint32_t rows = 0, cols = 0;
     uint64_t nnz = 0;

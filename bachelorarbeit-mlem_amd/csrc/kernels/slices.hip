@@ -40,9 +40,10 @@
 // number of passes.  Partial sums, their reduction and the epilogue are
 // those of tiled.hip.
 //
-// What bounds it: instructions (VALU two thirds of the time, 12 per step)
-// and the LDS gather (16 bytes per entry and 4 right-hand sides, 60%), then
-// the barriers (a tile waits for its longest stream).  us per launch, 4
+// What bounds it: instructions (VALU 75% busy, 12 per step) and the LDS
+// gather (16 bytes per entry and 4 right-hand sides; LDS 69% busy, half of
+// that bank conflicts), then the barriers (a tile waits for its longest
+// stream; with about 5 steps per stream and tile VALU 59%, LDS 64%).  us per launch, 4
 // passes of 4 right-hand sides over 683 M entries (16-bit) and 2 passes of 8
 // over 135 M (f32):
 //   block streams                                        2702 / 629

@@ -295,7 +295,9 @@ int mlem_matrix_set_row_order(mlem_matrix *m, const uint32_t *order);
  * column ranges of A (whole row blocks of A^T) and the sensitivity from their
  * row sums; A's copy is freed; A's tiles are built from row chunks of the
  * host CSR (read a second time).  The tiles are byte for byte those of the
- * resident path.  chunk_bytes bounds the scratch of each range / chunk
+ * resident path, except that automatic rows are fewer where the scratch holds
+ * no block of the resident path's, and row slices larger than the quads are
+ * taken only where a quarter of the device stays free.  chunk_bytes bounds the scratch of each range / chunk
  * (0 = what is free).  A reconstruction on it (per_pass 1) takes merge-based
  * FP and BP on A^T (spmv 0, using_trans 0) with the matrix's tile shape and
  * values, a batch (per_pass 4 or 8) the matrix's per_pass, shape and values
@@ -398,7 +400,7 @@ typedef struct mlem_batch_opts {
     uint32_t tile_rows;   /* 0 = automatic, for FP and BP by themselves (as
                              in mlem_opts for 1 per pass; 1024; 512 for
                              small matrices; with 4 per pass 2048 for
-                             large ones)                                   */
+                             large ones that row slices suit)              */
     uint32_t tile_groups; /* workgroups per blocked SpMV, 0 = automatic    */
     uint32_t tile_threads; /* work-items per workgroup of the block-stream
                               kernel for 4 or 8 per pass: 128, 256 or 512
